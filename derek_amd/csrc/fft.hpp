@@ -15,6 +15,8 @@
 // The transform length is a template constant for the hot sizes (the
 // compiler then folds all index arithmetic) and a runtime plan otherwise.
 #pragma once
+#include <type_traits>
+
 #include "common.hpp"
 
 namespace derek {
@@ -27,8 +29,8 @@ struct FftPlan {
   int r[kMaxStages];
 };
 
-// Radices with a register DFT; composite ones (6, 9, 12, 16) are built from
-// the prime-power kernels with internal twiddles.
+// Radices with a register DFT that the Stockham plans use; composite ones
+// (6, 9, 12, 16) are built from the prime-power kernels with internal twiddles.
 constexpr int kRadices[12] = {16, 12, 9, 8, 6, 5, 4, 3, 2, 7, 11, 13};
 
 // Depth-first search for the factorisation with the fewest stages, ties
@@ -80,6 +82,20 @@ constexpr FftPlan make_plan(int n) {
       }
   if (n == 1) p.ns = 0;
   return p;
+}
+
+// n = r1 * r2 with 1 <= r2 <= r1 <= 16 and r1 smallest, the split of the
+// two-stage register transforms (every radix from 1 to 16 has a register
+// DFT); r1 = 0 where there is none: lengths above 256 and 125, 147, 162, 175,
+// 189, 198, 200 among the smooth ones below 200.
+struct TwoStage {
+  int n, r1, r2;
+};
+constexpr int kMaxRadix = 16;
+constexpr TwoStage two_stage(int n) {
+  for (int r1 = 1; r1 <= kMaxRadix; ++r1)
+    if (n >= 1 && n % r1 == 0 && n / r1 <= r1) return TwoStage{n, r1, n / r1};
+  return TwoStage{n, 0, 0};
 }
 
 // ---------------------------------------------------------------- R-point DFTs
@@ -157,24 +173,69 @@ template <int S, typename C> __device__ __forceinline__ C twid(const C* tw, int 
   return S > 0 ? cconj(w) : w;
 }
 
-// Odd primes 7, 11, 13: direct O(R^2) sum with table roots of unity.
-template <int R, int S, typename C> __device__ __forceinline__ void dft_direct(C* v, const C* tw, int N) {
-  C out[R];
-  const int step = N / R;
-#pragma unroll
-  for (int k = 0; k < R; ++k) {
-    C acc = v[0];
-#pragma unroll
-    for (int j = 1; j < R; ++j) acc = cadd(acc, cmul(v[j], twid<S>(tw, ((j * k) % R) * step)));
-    out[k] = acc;
+// cos and sin of 2*pi*m/R, m = 0..(R-1)/2, of the odd primes 7, 11, 13.
+template <int R> __device__ __forceinline__ void prime_cs(int m, double& c, double& s) {
+  if constexpr (R == 7) {
+    constexpr double cc[4] = {1.0, 0.6234898018587335305250, -0.2225209339563144042889, -0.9009688679024191262361};
+    constexpr double ss[4] = {0.0, 0.7818314824680298087084, 0.9749279121818236070181, 0.4338837391175581204758};
+    c = cc[m];
+    s = ss[m];
+  } else if constexpr (R == 11) {
+    constexpr double cc[6] = {1.0, 0.8412535328311811688618, 0.4154150130018864255293, -0.1423148382732851404438,
+                              -0.6548607339452850640569, -0.9594929736144973898904};
+    constexpr double ss[6] = {0.0, 0.5406408174555975821076, 0.9096319953545183714117, 0.9898214418809327323761,
+                              0.7557495743542582837740, 0.2817325568414296977114};
+    c = cc[m];
+    s = ss[m];
+  } else {
+    static_assert(R == 13, "prime radix without a root table");
+    constexpr double cc[7] = {1.0, 0.8854560256532098959004, 0.5680647467311558025118, 0.1205366802553230533491,
+                              -0.3546048870425356259696, -0.7485107481711010986346, -0.9709418174260520271570};
+    constexpr double ss[7] = {0.0, 0.4647231720437685456560, 0.8229838658936563945796, 0.9927088740980539928008,
+                              0.9350162426854148234398, 0.6631226582407952023768, 0.2393156642875577671488};
+    c = cc[m];
+    s = ss[m];
   }
+}
+
+// Odd primes 7, 11, 13 from the sums p_j = v_j + v_{R-j} and differences
+// m_j = v_j - v_{R-j}: X_k, X_{R-k} = (v_0 + sum_j cos(2 pi j k/R) p_j)
+// +- S i (sum_j sin(2 pi j k/R) m_j).  The coefficients are real immediates,
+// so a 13-point transform takes 144 fused multiply-adds (144 complex products
+// with table roots otherwise).
+template <int R, int S, typename C> __device__ __forceinline__ void dft_prime(C* v) {
+  using Rl = decltype(C::x);
+  constexpr int H = (R - 1) / 2;
+  C p[H], m[H];
 #pragma unroll
-  for (int k = 0; k < R; ++k) v[k] = out[k];
+  for (int j = 0; j < H; ++j) {
+    p[j] = cadd(v[j + 1], v[R - 1 - j]);
+    m[j] = csub(v[j + 1], v[R - 1 - j]);
+  }
+  const C v0 = v[0];
+#pragma unroll
+  for (int j = 0; j < H; ++j) v[0] = cadd(v[0], p[j]);
+#pragma unroll
+  for (int k = 1; k <= H; ++k) {
+    C a = v0, b = cmk<C>(0, 0);
+#pragma unroll
+    for (int j = 1; j <= H; ++j) {
+      const int q = (j * k) % R;
+      double c, s;
+      prime_cs<R>(q <= H ? q : R - q, c, s);
+      const Rl cr = (Rl)c, sr = (Rl)(q <= H ? s : -s);
+      a = cmk<C>(a.x + cr * p[j - 1].x, a.y + cr * p[j - 1].y);
+      b = cmk<C>(b.x + sr * m[j - 1].x, b.y + sr * m[j - 1].y);
+    }
+    const C t = cmul_si<S>(b);
+    v[k] = cadd(a, t);
+    v[R - k] = csub(a, t);
+  }
 }
 
 template <int R, int S, typename C> __device__ __forceinline__ void dftR(C* v, const C* tw, int N);
 
-// cos and sin of 2*pi*m/R for the composite radices 6, 9, 12, 16 (m is a
+// cos and sin of 2*pi*m/R for the composite radices 6, 9, 10, 12, 14, 15, 16 (m is a
 // compile-time constant once the radix loops are unrolled, so these fold
 // into immediates instead of table loads held in registers).
 template <int R> __device__ __forceinline__ void root_cs(int m, double& c, double& s) {
@@ -198,6 +259,37 @@ template <int R> __device__ __forceinline__ void root_cs(int m, double& c, doubl
   } else if constexpr (R == 12) {
     constexpr double cc[12] = {1.0, h3, 0.5, 0.0, -0.5, -h3, -1.0, -h3, -0.5, 0.0, 0.5, h3};
     constexpr double ss[12] = {0.0, 0.5, h3, 1.0, h3, 0.5, 0.0, -0.5, -h3, -1.0, -h3, -0.5};
+    c = cc[q];
+    s = ss[q];
+  } else if constexpr (R == 10) {
+    constexpr double cc[10] = {1.0, 0.8090169943749474241023, 0.3090169943749474241023, -0.3090169943749474241023,
+                               -0.8090169943749474241023, -1.0, -0.8090169943749474241023, -0.3090169943749474241023,
+                               0.3090169943749474241023, 0.8090169943749474241023};
+    constexpr double ss[10] = {0.0, 0.5877852522924731291687, 0.9510565162951535721164, 0.9510565162951535721164,
+                               0.5877852522924731291687, 0.0, -0.5877852522924731291687, -0.9510565162951535721164,
+                               -0.9510565162951535721164, -0.5877852522924731291687};
+    c = cc[q];
+    s = ss[q];
+  } else if constexpr (R == 14) {
+    constexpr double cc[14] = {1.0, 0.9009688679024191262361, 0.6234898018587335305250, 0.2225209339563144042889,
+                               -0.2225209339563144042889, -0.6234898018587335305250, -0.9009688679024191262361, -1.0,
+                               -0.9009688679024191262361, -0.6234898018587335305250, -0.2225209339563144042889,
+                               0.2225209339563144042889, 0.6234898018587335305250, 0.9009688679024191262361};
+    constexpr double ss[14] = {0.0, 0.4338837391175581204758, 0.7818314824680298087084, 0.9749279121818236070181,
+                               0.9749279121818236070181, 0.7818314824680298087084, 0.4338837391175581204758, 0.0,
+                               -0.4338837391175581204758, -0.7818314824680298087084, -0.9749279121818236070181,
+                               -0.9749279121818236070181, -0.7818314824680298087084, -0.4338837391175581204758};
+    c = cc[q];
+    s = ss[q];
+  } else if constexpr (R == 15) {
+    constexpr double cc[15] = {1.0, 0.9135454576426008955021, 0.6691306063588582138263, 0.3090169943749474241023,
+                               -0.1045284632676534713998, -0.5, -0.8090169943749474241023, -0.9781476007338056379286,
+                               -0.9781476007338056379286, -0.8090169943749474241023, -0.5, -0.1045284632676534713998,
+                               0.3090169943749474241023, 0.6691306063588582138263, 0.9135454576426008955021};
+    constexpr double ss[15] = {0.0, 0.4067366430758002077540, 0.7431448254773942350147, 0.9510565162951535721164,
+                               0.9945218953682733369227, h3, 0.5877852522924731291687, 0.2079116908177593371017,
+                               -0.2079116908177593371017, -0.5877852522924731291687, -h3, -0.9945218953682733369227,
+                               -0.9510565162951535721164, -0.7431448254773942350147, -0.4067366430758002077540};
     c = cc[q];
     s = ss[q];
   } else {
@@ -255,7 +347,8 @@ template <int A, int B, int S, typename C> __device__ __forceinline__ void dft_c
 }
 
 template <int R, int S, typename C> __device__ __forceinline__ void dftR(C* v, const C* tw, int N) {
-  if constexpr (R == 2) dft2<S>(v);
+  if constexpr (R == 1) return;
+  else if constexpr (R == 2) dft2<S>(v);
   else if constexpr (R == 3) dft3<S>(v);
   else if constexpr (R == 4) dft4<S>(v);
   else if constexpr (R == 5) dft5<S>(v);
@@ -264,7 +357,33 @@ template <int R, int S, typename C> __device__ __forceinline__ void dftR(C* v, c
   else if constexpr (R == 9) dft_comp<3, 3, S>(v, tw, N);
   else if constexpr (R == 12) dft_comp<4, 3, S>(v, tw, N);
   else if constexpr (R == 16) dft_comp<4, 4, S>(v, tw, N);
-  else dft_direct<R, S>(v, tw, N);
+  else if constexpr (R == 10) dft_comp<5, 2, S>(v, tw, N);
+  else if constexpr (R == 14) dft_comp<7, 2, S>(v, tw, N);
+  else if constexpr (R == 15) dft_comp<5, 3, S>(v, tw, N);
+  else dft_prime<R, S>(v);
+}
+
+// f(std::integral_constant<int, r>) for a wave-uniform runtime radix r in
+// 1..kMaxRadix: one kernel holds every radix, the branch is scalar.
+template <typename F> __device__ __forceinline__ void with_radix(int r, F&& f) {
+  switch (r) {
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 3: f(std::integral_constant<int, 3>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    case 5: f(std::integral_constant<int, 5>{}); break;
+    case 6: f(std::integral_constant<int, 6>{}); break;
+    case 7: f(std::integral_constant<int, 7>{}); break;
+    case 8: f(std::integral_constant<int, 8>{}); break;
+    case 9: f(std::integral_constant<int, 9>{}); break;
+    case 10: f(std::integral_constant<int, 10>{}); break;
+    case 11: f(std::integral_constant<int, 11>{}); break;
+    case 12: f(std::integral_constant<int, 12>{}); break;
+    case 13: f(std::integral_constant<int, 13>{}); break;
+    case 14: f(std::integral_constant<int, 14>{}); break;
+    case 15: f(std::integral_constant<int, 15>{}); break;
+    default: f(std::integral_constant<int, 16>{}); break;
+  }
 }
 
 // ---------------------------------------------------------------- one stage

@@ -12,6 +12,7 @@
 //   S[item][stick][nz]           stick lines (nst_cap sticks per item)
 //   P[item][active x][ny][nz]    active planes (nax_cap planes per item)
 #include "launch.hpp"
+#include "pw_any.hpp"
 #include "pw_fft.hpp"
 
 namespace derek {
@@ -726,25 +727,6 @@ __device__ __forceinline__ void xcd_task(int& major, int& minor) {
   minor = t % (int)gridDim.y;
 }
 
-// Streaming (non-temporal) 16- or 8-byte access of one complex value, for the
-// stick rows that the inverse z pass writes and the forward z pass reads:
-// each is touched once.  (Measured at 108^3: the inverse z pass 87 -> 63 us
-// per 80-band launch; the same hint on the y/x pass's stick rows slowed the
-// complex64 forward z pass, whose input then no longer came from the cache.)
-template <typename C> __device__ __forceinline__ void nt_store(C* p, C v) {
-  using V = decltype(v.x) __attribute__((ext_vector_type(2)));
-  V t = {v.x, v.y};
-  __builtin_nontemporal_store(t, reinterpret_cast<V*>(p));
-}
-template <typename C> __device__ __forceinline__ C nt_load(const C* p) {
-  using V = decltype(p->x) __attribute__((ext_vector_type(2)));
-  const V t = __builtin_nontemporal_load(reinterpret_cast<const V*>(p));
-  C r;
-  r.x = t.x;
-  r.y = t.y;
-  return r;
-}
-
 // psi[b][perm[p]] -> S[item][s][:] for the block's sticks
 template <typename R, int N, bool ZM, int SL_>
 __global__ __launch_bounds__((StickSplit<N, SL_>::NT)) void k_sticks_z_inv2(PwBatch B, PwBlock<R> psi,
@@ -902,7 +884,11 @@ void sticks_z_inv(const PwBatch& B, PwBlock<R> psi, const Axis<R>* ax, int nz, c
     case 144: sticks_z_inv2<R, 144>(B, psi, ax, S, zmajor, s); DEREK_HIP(hipGetLastError()); return;
     default: break;
   }
-  DEREK_REQUIRE(!zmajor, "z-major sticks need a z length with a compiled kernel");
+  if (any_z_inv<R>(B, psi, ax[2], S, zmajor, s)) {
+    DEREK_HIP(hipGetLastError());
+    return;
+  }
+  DEREK_REQUIRE(!zmajor, "z-major sticks need a z length with a two-stage split");
   const int lpb = sticks_per_block(nz);
   const size_t lds = sizeof(cx_t<R>) * ((size_t)nz + 2 * (size_t)lpb * contig_stride(nz));
   check_lds_pw(lds, nz);
@@ -957,6 +943,7 @@ void planes_y(const PwBatch& B, cx_t<R>* S, cx_t<R>* P, const Axis<R>* ax, int n
     case 108: planes_y2_bpw<R, 108>(B, S, P, ax, nz, sign, bpw, s); break;
     case 144: planes_y2_bpw<R, 144>(B, S, P, ax, nz, sign, bpw, s); break;
     default: {
+      if (any_y<R>(B, S, P, ax[1], nz, sign, bpw, s)) break;
       const int ztiles = (int)ceil_div(nz, PL);
       const size_t lds = sizeof(cx_t<R>) * ((size_t)ny + 2 * (size_t)PL * ny);
       check_lds_pw(lds, ny);
@@ -986,7 +973,11 @@ void sticks_z_fwd(const PwBatch& B, const cx_t<R>* S, const Axis<R>* ax, int nz,
     case 144: sticks_z_fwd2<R, 144>(B, S, ax, psi, hpsi, zmajor, s); DEREK_HIP(hipGetLastError()); return;
     default: break;
   }
-  DEREK_REQUIRE(!zmajor, "z-major sticks need a z length with a compiled kernel");
+  if (any_z_fwd<R>(B, S, ax[2], psi, hpsi, zmajor, s)) {
+    DEREK_HIP(hipGetLastError());
+    return;
+  }
+  DEREK_REQUIRE(!zmajor, "z-major sticks need a z length with a two-stage split");
   const int lpb = sticks_per_block(nz);
   const size_t lds = sizeof(cx_t<R>) * ((size_t)nz + 2 * (size_t)lpb * contig_stride(nz));
   check_lds_pw(lds, nz);
@@ -1020,6 +1011,7 @@ static void planes_x_vmul_bpw(const PwBatch& B, cx_t<R>* P, const Axis<R>* ax, i
     case 108: C2_(108); break;
     case 144: C2_(144); break;
     default: {
+      if (any_x_vmul<R>(B, P, ax[0], nyz, vloc, vscale, BPW, s)) break;
       const size_t lds = sizeof(cx_t<R>) * ((size_t)nx + 2 * (size_t)PL * nx) + sizeof(R) * (size_t)PL * nx;
       check_lds_pw(lds, nx);
       auto kern = k_planes_x_vmul<R, 0, BPW>;
@@ -1065,6 +1057,7 @@ void planes_x_density(const PwBatch& B, const cx_t<R>* P, const Axis<R>* ax, int
     case 108: C2_(108); break;
     case 144: C2_(144); break;
     default: {
+      if (any_x_density<R>(B, P, ax[0], nyz, occ, occ_ks, rho, keep, s)) break;
       const size_t lds = sizeof(cx_t<R>) * ((size_t)nx + 2 * (size_t)PL * nx) + sizeof(double) * (size_t)PL * nx;
       check_lds_pw(lds, nx);
       auto kern = k_planes_x_density<R, 0>;

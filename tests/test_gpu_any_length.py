@@ -1,0 +1,61 @@
+"""H|psi> and the density at FFT lengths without kernels of their own, against
+the oracle: every radix from 1 to 16 in both stages of a length r1 * r2, axes
+of different lengths, column tiles and stick blocks with remainders, active
+rows in any order, and the lengths that have no such split (Stockham).
+
+An FFT of n points carries a relative rounding error of a few eps * log2(n)
+(eps = 1.1e-16 / 6e-8), at most 30 eps here for inverse, multiply and forward
+together; the bounds are the ones of the other pipeline tests, 1e-12 and 5e-5
+of the largest value.
+"""
+import numpy as np
+import pytest
+
+from derek_amd import lib
+from oracle import ks as oks
+from tests.conftest import assert_close
+
+pytestmark = pytest.mark.gpu
+
+DIMS = [(1, 2, 3), (5, 7, 4), (8, 6, 13), (22, 26, 10), (65, 33, 30), (16, 15, 210), (28, 98, 11), (99, 40, 24),
+        (50, 63, 64), (140, 21, 39), (12, 225, 18), (45, 14, 240), (256, 9, 91), (65, 65, 65), (54, 54, 36),
+        (125, 8, 162), (35, 147, 20)]
+
+
+def waves(dims, rng, share=0.3):
+    """A random set of FFT bins on a few columns, in shuffled order."""
+    nx, ny, nz = dims
+    xs = rng.permutation(nx)[:max(1, int(share * 1.5 * nx))]
+    idx = []
+    for x in xs:
+        for y in rng.permutation(ny)[:max(1, int(share * ny))]:
+            z = rng.permutation(nz)[:max(1, int(share * nz))]
+            idx.append((x * ny + y) * nz + z)
+    return rng.permutation(np.concatenate(idx)).astype(np.int32)
+
+
+@pytest.mark.parametrize("dims", DIMS)
+@pytest.mark.parametrize("precision", [lib.DEREK_FP64, lib.DEREK_MIXED])
+def test_any_length_apply_h_and_density(dims, precision):
+    rng = np.random.default_rng(sum(dims))
+    nb, volume, weight = 5, 37.0, 0.7
+    sets = [waves(dims, rng), waves(dims, rng, 0.2)]
+    kins = [rng.uniform(0.0, 3.0, len(s)) for s in sets]
+    v = rng.normal(size=int(np.prod(dims)))
+    tol = 1e-12 if precision == lib.DEREK_FP64 else 5e-5
+    ctx = lib.Context(list(dims), 2, nb, volume, max(len(s) for s in sets), precision)
+    for k in range(2):
+        ctx.set_basis(k, sets[k], kins[k], weight)
+    ctx.set_vloc(v)
+    for zs in (16, 32):
+        print("any length", dims, precision, "sticks", zs, flush=True)
+        ctx.set_tiles(zs, 2, 64)
+        ctx.set_launch(bands_per_wg=2, items_per_launch=3, fused=zs == 16)
+        for k in range(2):
+            psi = rng.normal(size=(nb, len(sets[k]))) + 1j * rng.normal(size=(nb, len(sets[k])))
+            assert_close(ctx.apply_h(k, psi), oks.apply_h(psi, sets[k], kins[k], v, dims), tol, f"H psi k={k}")
+            occ = np.array([2.0, 0.0, 1.3, 0.4, 2.0])
+            r0 = rng.uniform(size=v.size)
+            ref = r0 + oks.density([psi], [occ], [weight], [sets[k]], dims, volume)
+            assert_close(ctx.density(k, psi, occ, r0), ref, tol, f"density k={k}")
+    ctx.close()
