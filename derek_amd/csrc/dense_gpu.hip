@@ -16,9 +16,9 @@
 //      whose vectors are computed by one thread in order and re-orthogonalised
 //      (modified Gram-Schmidt) against the earlier members.
 //   5. Back-transformation by the reflectors, one wavefront per vector.
-// k_chol_drop: Cholesky of a unit-diagonal Hermitian overlap that skips every
-//   column whose remaining pivot is below tol (dependent on earlier columns).
-// k_trinv: inverse of a lower-triangular matrix, one wavefront per column.
+// k_chol_panel: inverse Cholesky factor of a unit-diagonal Hermitian overlap,
+//   skipping every column whose remaining pivot is below tol (dependent on
+//   earlier columns); many workgroups, one launch per panel of columns.
 #include <cfloat>
 
 #include "dense_gpu.hpp"
@@ -1209,217 +1209,205 @@ void heev_gpu(double2* A, int lda, int64_t strideA, int n, int nev, double* Wv, 
 // All matrices m x m, column-major, ld m; matrix kz of a batch at kz*m*m
 // (blockIdx.y or blockIdx.x selects it).
 
-// dsc = 1/sqrt(diag S) (0 for a zero column), S <- D S D
-__global__ void k_unit_diag(double2* __restrict__ Sall, int m, double* __restrict__ dscall) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  double* sd = reinterpret_cast<double*>(smem);
-  const int kz = blockIdx.y;
-  double2* S = Sall + (int64_t)kz * m * m;
-  double* dsc = dscall + (int64_t)kz * m;
-  for (int i = threadIdx.x; i < m; i += blockDim.x) {
-    const double d = S[i + (int64_t)i * m].x;
-    const double v = d > 0.0 ? 1.0 / sqrt(d) : 0.0;
-    sd[i] = v;
-    dsc[i] = v;
-  }
-  __syncthreads();
-  const int64_t mm = (int64_t)m * m;
-  for (int64_t q = threadIdx.x; q < mm; q += blockDim.x) {
-    const int r = (int)(q % m), c = (int)(q / m);
-    const double f = sd[r] * sd[c];
-    S[q] = make_double2(S[q].x * f, S[q].y * f);
-  }
+// 1/sqrt of the diagonal entry i of S (0 for a zero column)
+__device__ __forceinline__ double diag_scale(const double2* S, int m, int i) {
+  const double d = S[i + (int64_t)i * m].x;
+  return d > 0.0 ? 1.0 / sqrt(d) : 0.0;
 }
 
-// Blocked right-looking Cholesky of the unit-diagonal S with dropping, on a
-// work copy Wm (lower triangle used).  A panel of nb columns is staged in
-// LDS and factored there: column j is kept if its updated pivot exceeds
-// tol * S_jj; a kept column is L's column j and updates the rest of the
-// panel; a dropped column is zeroed and contributes nothing.  The panel then
-// updates the trailing lower triangle in one pass (one wavefront per column,
-// rows over the lanes).  Output: Lf (lower triangular) = L on the kept rows
-// and columns, the identity on the dropped ones, keep[j], na = #kept, ok =
-// (na >= nev).
-__global__ __launch_bounds__(DT) void k_chol_drop(const double2* __restrict__ Sall, int m, int nb, double tol,
-                                                  int nev, double2* __restrict__ Wall, double2* __restrict__ Lall,
-                                                  int* __restrict__ keepall, int* __restrict__ naall,
-                                                  int* __restrict__ okall) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  double2* P = reinterpret_cast<double2*>(smem);               // [nb][m]: P[jj*m + i]
-  double* sd = reinterpret_cast<double*>(P + (size_t)nb * m);  // [m] diagonal of S
-  int* kp = reinterpret_cast<int*>(sd + m);                    // [m] keep flags
-  const int kz = blockIdx.x;
-  const int64_t mm = (int64_t)m * m;
-  const double2* S = Sall + kz * mm;
-  double2* Wm = Wall + kz * mm;
-  double2* Lf = Lall + kz * mm;
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  for (int64_t q = tid; q < mm; q += DT) Wm[q] = S[q];
-  for (int i = tid; i < m; i += DT) sd[i] = S[i + (int64_t)i * m].x;
-  __syncthreads();
-  int c = 0;
-  for (int p0 = 0; p0 < m; p0 += nb) {
-    const int pn = min(nb, m - p0), rows = m - p0;
-    for (int q = tid; q < pn * rows; q += DT) {
-      const int jj = q / rows, i = p0 + q % rows;
-      P[jj * m + i] = Wm[i + (int64_t)(p0 + jj) * m];
-    }
-    __syncthreads();
-    for (int jj = 0; jj < pn; ++jj) {
-      const int j = p0 + jj;
-      double2* pc = P + jj * m;
-      const double d = pc[j].x;
-      if (d > tol * sd[j]) {
-        const double idj = rsqrt_nr(d), lj = d * idj;
-        double2* lcol = Lf + (int64_t)j * m;
-        for (int i = j + 1 + tid; i < m; i += DT) {
-          const double2 l = make_double2(pc[i].x * idj, pc[i].y * idj);
-          pc[i] = l;
-          lcol[i] = l;
-        }
-        if (tid == 0) {
-          lcol[j] = make_double2(lj, 0.0);
-          kp[j] = 1;
-        }
-        __syncthreads();
-        // rest of the panel: P(i,kk) -= l_i conj(l_(p0+kk)), i >= p0+kk
-        for (int kk = jj + 1 + wid; kk < pn; kk += DW) {
-          const double2 lk = pc[p0 + kk];
-          double2* pk = P + kk * m;
-          for (int i = p0 + kk + lane; i < m; i += 64) {
-            const double2 li = pc[i];
-            pk[i] = make_double2(pk[i].x - (li.x * lk.x + li.y * lk.y), pk[i].y - (li.y * lk.x - li.x * lk.y));
-          }
-        }
-        __syncthreads();
-        ++c;
-      } else {
-        // only column jj's own rows are written; the next column reads
-        // column jj+1, and the trailing update waits for a barrier
-        for (int i = j + tid; i < m; i += DT) pc[i] = make_double2(0.0, 0.0);
-        if (tid == 0) kp[j] = 0;
-      }
-    }
-    __syncthreads();
-    // trailing update W(i,k) -= sum_jj P(i,jj) conj(P(k,jj)), i >= k >= p0+pn
-    for (int k = p0 + pn + wid; k < m; k += DW) {
-      double2* wk = Wm + (int64_t)k * m;
-      for (int i = k + lane; i < m; i += 64) {
-        double2 acc = wk[i];
-        for (int jj = 0; jj < pn; ++jj) {
-          const double2 li = P[jj * m + i], lk = P[jj * m + k];
-          acc.x -= li.x * lk.x + li.y * lk.y;
-          acc.y -= li.y * lk.x - li.x * lk.y;
-        }
-        wk[i] = acc;
-      }
-    }
-    __syncthreads();
-  }
-  // upper triangle zero; dropped rows and columns -> identity
-  for (int k = wid; k < m; k += DW) {
-    double2* lcol = Lf + (int64_t)k * m;
-    for (int i = lane; i < m; i += 64)
-      if (i < k || !kp[i] || !kp[k]) lcol[i] = make_double2(i == k ? 1.0 : 0.0, 0.0);
-  }
-  for (int i = tid; i < m; i += DT) keepall[(int64_t)kz * m + i] = kp[i];
-  if (tid == 0) {
-    naall[kz] = c;
-    okall[kz] = c >= nev ? 1 : 0;
-  }
-}
-
-// Inverse of a lower-triangular m x m matrix, one wavefront per column j:
-// forward substitution on e_j with the solution and the current column of L
-// in registers (row i lives in lane i % 64, slot i / 64); the pivot and x_k
-// are read across lanes with readlane.  The columns of L are L2 reads: D of
-// them are kept in flight in a register ring (slot d holds column k0 + d and
-// is refilled with column k0 + d + D once used), so a step waits for a load
-// issued D steps earlier instead of one.  TR = rows per lane (m <= 64 TR).
-constexpr int TR = 10;  // largest rows per lane: m <= 640
-
-__device__ __forceinline__ double readlane_d(double v, int l) {
-  const long long b = __double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// rows i >= c of column c of L (zero elsewhere, and for c >= m)
-template <int NR>
-__device__ __forceinline__ void trinv_load(const double2* __restrict__ L, int m, int c, int lane, double2 (&col)[NR]) {
-#pragma unroll
-  for (int t = 0; t < NR; ++t) {
-    const int i = lane + 64 * t;
-    col[t] = (c < m && i >= c && i < m) ? L[i + (int64_t)c * m] : make_double2(0.0, 0.0);
-  }
-}
-
-template <int NR, int D>
-__global__ __launch_bounds__(64) void k_trinv(const double2* __restrict__ Lall, int m,
-                                              double2* __restrict__ Linvall) {
-  const int j = blockIdx.x, lane = threadIdx.x;
-  const int64_t mm = (int64_t)m * m;
-  const double2* L = Lall + blockIdx.y * mm;
-  double2 x[NR], ring[D][NR];
-#pragma unroll
-  for (int t = 0; t < NR; ++t) {
-    const int i = lane + 64 * t;
-    x[t] = make_double2(i == j ? 1.0 : 0.0, 0.0);
-  }
-#pragma unroll
-  for (int d = 0; d < D; ++d) trinv_load<NR>(L, m, j + d, lane, ring[d]);
-  for (int k0 = j; k0 < m; k0 += D) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int k = k0 + d;
-      if (k >= m) break;  // uniform over the wavefront
-      const int tk = k >> 6, lk = k & 63;
-      double2 xo = make_double2(0.0, 0.0), dg = make_double2(1.0, 0.0);
-#pragma unroll
-      for (int t = 0; t < NR; ++t)
-        if (t == tk) {
-          xo = x[t];
-          dg = ring[d][t];
-        }
-      xo = make_double2(readlane_d(xo.x, lk), readlane_d(xo.y, lk));
-      dg = make_double2(readlane_d(dg.x, lk), readlane_d(dg.y, lk));
-      const double den = 1.0 / (dg.x * dg.x + dg.y * dg.y);
-      const double2 xk = make_double2((xo.x * dg.x + xo.y * dg.y) * den, (xo.y * dg.x - xo.x * dg.y) * den);
-#pragma unroll
-      for (int t = 0; t < NR; ++t) {
-        const int i = lane + 64 * t;
-        if (i > k) {
-          const double2 u = zmul(ring[d][t], xk);
-          x[t] = make_double2(x[t].x - u.x, x[t].y - u.y);
-        } else if (i == k) {
-          x[t] = xk;
-        }
-      }
-      trinv_load<NR>(L, m, k + D, lane, ring[d]);
-    }
-  }
-  double2* out = Linvall + blockIdx.y * mm + (int64_t)j * m;
-#pragma unroll
-  for (int t = 0; t < NR; ++t) {
-    const int i = lane + 64 * t;
-    if (i < m) out[i] = x[t];
-  }
-}
-
-// B = A^H
-__global__ void k_conj_transpose(const double2* __restrict__ A, int m, double2* __restrict__ B) {
-  const int64_t mm = (int64_t)m * m;
-  A += blockIdx.y * mm;
-  B += blockIdx.y * mm;
+// Lower triangle of W <- D (S + S^H)/2 D with D = 1/sqrt(diag S) (dsc), and
+// Linv, LinvH <- 0
+__global__ void k_chol_prep(const double2* __restrict__ Sall, int m, double* __restrict__ dscall,
+                            double2* __restrict__ Wall, double2* __restrict__ Linvall,
+                            double2* __restrict__ LinvHall) {
+  const int64_t mm = (int64_t)m * m, o = blockIdx.y * mm;
+  const double2* S = Sall + o;
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < mm; q += (int64_t)gridDim.x * blockDim.x) {
     const int r = (int)(q % m), c = (int)(q / m);
-    const double2 a = A[c + (int64_t)r * m];
-    B[q] = make_double2(a.x, -a.y);
+    Linvall[o + q] = LinvHall[o + q] = make_double2(0.0, 0.0);
+    if (r < c) continue;
+    const double dr = diag_scale(S, m, r);
+    if (r == c) {
+      dscall[(int64_t)blockIdx.y * m + r] = dr;
+      Wall[o + q] = make_double2(S[q].x * (dr * dr), 0.0);
+    } else {
+      const double f = 0.5 * dr * diag_scale(S, m, c);
+      const double2 a = S[q], b = S[c + (int64_t)r * m];
+      Wall[o + q] = make_double2((a.x + b.x) * f, (a.y - b.y) * f);
+    }
   }
 }
 
-// Hc = (D H D) on the kept rows and columns, 0 elsewhere
+// Cholesky factor with dropped columns and its inverse, one launch per panel
+// of CB columns: the factor L of the unit-diagonal W = L L^H, where column j
+// is kept if its updated pivot exceeds tol and replaced by the identity
+// column and row otherwise, is never stored; what the launches leave is
+// Linv = L^-1 (and LinvH, its conjugate transpose), from the forward
+// elimination of the identity carried along with the factorisation.
+//
+// A workgroup owns one CT x CT tile: a lower tile of the trailing W (right of
+// and below the panel) or a tile (trailing rows, columns done so far) of the
+// eliminated identity R.  Each one factors the CB x CB diagonal block of the
+// panel for itself (one wavefront, a row per lane, pivots and columns by
+// readlane), meanwhile another wavefront has loaded the tile's CT rows of the
+// panel and either the CT rows of its columns (W tile) or the CT columns of
+// the panel rows of R (R tile) and solves them against the block, one row or
+// column per lane; then the tile takes its rank-CB update.  The panel columns
+// of W and the panel rows of R are only read, X = L11^-1 R goes to Linv and
+// LinvH, so no workgroup waits for another within a launch.
+//
+// Bound: the serial chain of a launch (launch, two loads, 16 pivots of about
+// 400 cycles, a 16-step substitution).  The single-workgroup factorisation it
+// replaces was bound by its one CU: 203 us at m = 160 and 4650 us at m = 600,
+// plus 57 and 552 us for the inverse (one wavefront per column) and 13 and
+// 139 us for the scaling (one workgroup).
+constexpr int CB = 16, CT = 32, CNT = 256;
+
+__global__ __launch_bounds__(CNT) void k_chol_panel(double2* __restrict__ Wall, double2* __restrict__ Rall,
+                                                    double2* __restrict__ Linvall, double2* __restrict__ LinvHall,
+                                                    int m, int p0, double tol, int nev, int* __restrict__ keepall,
+                                                    int* __restrict__ naall, int* __restrict__ okall) {
+  __shared__ double2 L11[CB][CB];      // rows of the panel's factor
+  __shared__ double idiag[CB];         // 1 / L_jj, 0 where dropped
+  __shared__ double2 La[CB][CT + 1];   // [panel column][tile row]
+  __shared__ double2 Lb[CB][CT + 1];   // [panel column or row][tile column]
+  const int64_t mm = (int64_t)m * m, o = blockIdx.y * mm;
+  double2* W = Wall + o;
+  double2* Rm = Rall + o;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int pn = min(CB, m - p0), p1 = p0 + pn;
+  const int nt = (m - p1 + CT - 1) / CT;  // tile rows of the trailing part
+  // tile: W tiles (bi, bj <= bi) first, then R tiles (bi, cb); with nothing
+  // trailing only X is formed (tile row 0 without rows)
+  int bi = 0, bj = blockIdx.x;
+  const int nw = nt * (nt + 1) / 2;
+  const bool wt = bj < nw;
+  if (wt) {
+    while (bj > bi) bj -= ++bi;
+  } else {
+    const int ncb = (p1 + CT - 1) / CT;
+    bj -= nw;
+    bi = bj / ncb;
+    bj -= bi * ncb;
+  }
+  const int r0 = p1 + bi * CT, c0 = wt ? p1 + bj * CT : bj * CT, cend = wt ? m : p1;
+  // this thread's tile elements: row tr, columns tc + 8 q
+  const int tr = tid % CT, tc = tid / CT;
+  double2* T = wt ? W : Rm;
+  double2 t[CT * CT / CNT];
+#pragma unroll
+  for (int q = 0; q < CT * CT / CNT; ++q) {
+    const int r = r0 + tr, c = c0 + tc + (CNT / CT) * q;
+    // the panel's own columns of R have not been touched: zero
+    t[q] = (r < m && c < cend && (wt || c < p0)) ? T[r + (int64_t)c * m] : make_double2(0.0, 0.0);
+  }
+  double2 x[CB];
+  if (wid == 0) {
+    // lanes 0..31: the tile's rows of the panel; 32..63: the rows of its
+    // columns (W tile) or its columns of the panel's rows of R (R tile)
+    const int h = lane / CT, l = lane % CT;
+    const int row = (h == 0 ? r0 : c0) + l;
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+      double2 v = make_double2(0.0, 0.0);
+      if (h == 0 || wt) {
+        if (row < m && j < pn) v = W[row + (int64_t)(p0 + j) * m];
+      } else if (j < pn) {
+        if (row < p0) v = Rm[(p0 + j) + (int64_t)row * m];
+        else if (row == p0 + j) v = make_double2(1.0, 0.0);
+      }
+      x[j] = v;
+    }
+  } else if (wid == 1) {
+    double2 a[CB];
+#pragma unroll
+    for (int k = 0; k < CB; ++k)
+      a[k] = (lane < pn && k <= lane) ? W[(p0 + lane) + (int64_t)(p0 + k) * m] : make_double2(0.0, 0.0);
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+      const double d = read_lane(a[j].x, j);
+      double idj = 0.0;
+      if (j < pn && d > tol) {
+        idj = rsqrt_nr(d);
+        const double2 l = make_double2(a[j].x * idj, a[j].y * idj);
+#pragma unroll
+        for (int k = j + 1; k < CB; ++k) {
+          const double kr = read_lane(l.x, k), ki = read_lane(l.y, k);
+          a[k] = make_double2(a[k].x - (l.x * kr + l.y * ki), a[k].y - (l.y * kr - l.x * ki));
+        }
+        a[j] = l;
+      } else {
+        a[j] = make_double2(0.0, 0.0);
+      }
+      if (lane == 0) idiag[j] = idj;
+    }
+    if (lane < CB) {
+#pragma unroll
+      for (int k = 0; k < CB; ++k) L11[lane][k] = a[k];
+    }
+  }
+  __syncthreads();
+  if (wid == 0) {
+    const int h = lane / CT, l = lane % CT;
+    const bool left = h == 0 || wt;  // rows: x L11^H = w; columns: L11 x = r
+#pragma unroll
+    for (int j = 0; j < CB; ++j) {
+      double2 s = x[j];
+#pragma unroll
+      for (int k = 0; k < j; ++k) {
+        const double2 b = L11[j][k];
+        const double bi_ = left ? -b.y : b.y;  // x_k conj(L_jk) or L_jk x_k
+        s = make_double2(s.x - (x[k].x * b.x - x[k].y * bi_), s.y - (x[k].x * bi_ + x[k].y * b.x));
+      }
+      const double id = idiag[j];
+      x[j] = make_double2(s.x * id, s.y * id);
+      // a dropped row of L is the identity row: x = e_j there
+      if (!left && id == 0.0) x[j] = make_double2(c0 + l == p0 + j ? 1.0 : 0.0, 0.0);
+    }
+#pragma unroll
+    for (int j = 0; j < CB; ++j) (h == 0 ? La : Lb)[j][l] = x[j];
+    if (!wt && bi == 0 && h == 1 && c0 + l < p1) {
+      const int c = c0 + l;
+      double2* li = Linvall + o + (int64_t)c * m + p0;
+      double2* lh = LinvHall + o + (int64_t)p0 * m + c;
+#pragma unroll
+      for (int j = 0; j < CB; ++j)
+        if (j < pn) {
+          li[j] = x[j];
+          lh[(int64_t)j * m] = make_double2(x[j].x, -x[j].y);
+        }
+    }
+  }
+  __syncthreads();
+  if (r0 < m) {
+#pragma unroll
+    for (int q = 0; q < CT * CT / CNT; ++q) {
+      const int cc = tc + (CNT / CT) * q;
+#pragma unroll
+      for (int j = 0; j < CB; ++j) {
+        // W(r,c) -= L_rj conj(L_cj); R(r,c) -= L_rj X_jc.  An R tile uses the
+        // dropped rows' X only through L_rj = 0.
+        const double2 a = La[j][tr], b = Lb[j][cc];
+        const double by = wt ? -b.y : b.y;
+        t[q] = make_double2(t[q].x - (a.x * b.x - a.y * by), t[q].y - (a.x * by + a.y * b.x));
+      }
+      const int r = r0 + tr, c = c0 + cc;
+      if (r < m && c < cend) T[r + (int64_t)c * m] = t[q];
+    }
+  }
+  if (blockIdx.x == 0) {
+    int* keep = keepall + (int64_t)blockIdx.y * m;
+    if (tid < pn) keep[p0 + tid] = idiag[tid] != 0.0 ? 1 : 0;
+    if (tid == 0) {
+      int c = p0 == 0 ? 0 : naall[blockIdx.y];
+      for (int j = 0; j < pn; ++j) c += idiag[j] != 0.0 ? 1 : 0;
+      naall[blockIdx.y] = c;
+      okall[blockIdx.y] = c >= nev ? 1 : 0;
+    }
+  }
+}
+
+// Hc = D (H + H^H)/2 D on the kept rows and columns, 0 elsewhere
 __global__ void k_scale_mask(const double2* __restrict__ H, const double* __restrict__ dsc,
                              const int* __restrict__ keep, int m, double2* __restrict__ Hc) {
   const int64_t mm = (int64_t)m * m;
@@ -1430,8 +1418,9 @@ __global__ void k_scale_mask(const double2* __restrict__ H, const double* __rest
   keep += (int64_t)kz * m;
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < mm; q += (int64_t)gridDim.x * blockDim.x) {
     const int r = (int)(q % m), c = (int)(q / m);
-    const double f = (keep[r] && keep[c]) ? dsc[r] * dsc[c] : 0.0;
-    Hc[q] = make_double2(H[q].x * f, H[q].y * f);
+    const double f = (keep[r] && keep[c]) ? dsc[r] * dsc[c] * 0.5 : 0.0;
+    const double2 a = H[q], b = H[c + (int64_t)r * m];
+    Hc[q] = make_double2((a.x + b.x) * f, (a.y - b.y) * f);
   }
 }
 
@@ -1440,7 +1429,10 @@ __global__ void k_scale_mask(const double2* __restrict__ H, const double* __rest
 // Row sums: R = min(m, DT) rows per pass over consecutive threads (coalesced
 // column reads), the columns split over DT / R thread groups whose parts are
 // added through LDS.
-__global__ __launch_bounds__(DT) void k_big_diag(double2* __restrict__ Aall, const int* __restrict__ keepall, int m) {
+// Nothing to do, and nothing read, where every column was kept.
+__global__ __launch_bounds__(DT) void k_big_diag(double2* __restrict__ Aall, const int* __restrict__ keepall,
+                                                 const int* __restrict__ naall, int m) {
+  if (naall[blockIdx.x] == m) return;
   __shared__ double red[DW];
   __shared__ double part[DT];
   const int kz = blockIdx.x;
@@ -1524,38 +1516,16 @@ void hermitize_gpu(double2* A, int m, int batch, hipStream_t s) {
   DEREK_HIP(hipGetLastError());
 }
 
-void unit_diag_gpu(double2* S, int m, double* dsc, int batch, hipStream_t s) {
-  DEREK_REQUIRE(m <= 8192, "unit_diag: matrix too large");
-  // one workgroup per matrix: S is scaled in place after its diagonal is read
-  hipLaunchKernelGGL(k_unit_diag, dim3(1, batch), dim3(1024), sizeof(double) * m, s, S, m, dsc);
-  DEREK_HIP(hipGetLastError());
-}
-
-void chol_drop_gpu(const double2* S, int m, double tol, int nev, double2* Wm, double2* Lf, int* keep, int* na,
-                   int* ok, int batch, hipStream_t s) {
-  constexpr size_t kLds = 60 * 1024;
-  const size_t per_row = sizeof(double2) + sizeof(double) + sizeof(int);
-  DEREK_REQUIRE(m >= 1 && (size_t)m * per_row <= kLds, "chol_drop: matrix too large");
-  const int nb = (int)std::min<size_t>(16, (kLds - (sizeof(double) + sizeof(int)) * m) / (sizeof(double2) * m));
-  const size_t lds = sizeof(double2) * (size_t)nb * m + (sizeof(double) + sizeof(int)) * m;
-  hipLaunchKernelGGL(k_chol_drop, dim3(batch), dim3(DT), lds, s, S, m, nb, tol, nev, Wm, Lf, keep, na, ok);
-  DEREK_HIP(hipGetLastError());
-}
-
-void trinv_gpu(const double2* L, int m, double2* Linv, int batch, hipStream_t s) {
-  DEREK_REQUIRE(m <= 64 * TR, "trinv: matrix too large");
-  const dim3 grid((unsigned)m, batch);
-  if (m <= 64)
-    hipLaunchKernelGGL((k_trinv<1, 8>), grid, dim3(64), 0, s, L, m, Linv);
-  else if (m <= 192)
-    hipLaunchKernelGGL((k_trinv<3, 8>), grid, dim3(64), 0, s, L, m, Linv);
-  else
-    hipLaunchKernelGGL((k_trinv<TR, 4>), grid, dim3(64), 0, s, L, m, Linv);
-  DEREK_HIP(hipGetLastError());
-}
-
-void conj_transpose_gpu(const double2* A, int m, double2* B, int batch, hipStream_t s) {
-  hipLaunchKernelGGL(k_conj_transpose, mgrid(m, batch), dim3(256), 0, s, A, m, B);
+void chol_inverse_gpu(const double2* S, int m, double tol, int nev, double2* Wm, double2* R, double2* Linv,
+                      double2* LinvH, double* dsc, int* keep, int* na, int* ok, int batch, hipStream_t s) {
+  DEREK_REQUIRE(m >= 1 && m <= 8192, "chol_inverse: matrix too large");
+  hipLaunchKernelGGL(k_chol_prep, mgrid(m, batch), dim3(256), 0, s, S, m, dsc, Wm, Linv, LinvH);
+  for (int p0 = 0; p0 < m; p0 += CB) {
+    const int p1 = std::min(m, p0 + CB), nt = (int)ceil_div(m - p1, CT);
+    const int tiles = nt * (nt + 1) / 2 + std::max(1, nt) * (int)ceil_div(p1, CT);
+    hipLaunchKernelGGL(k_chol_panel, dim3(tiles, batch), dim3(CNT), 0, s, Wm, R, Linv, LinvH, m, p0, tol, nev, keep, na,
+                       ok);
+  }
   DEREK_HIP(hipGetLastError());
 }
 
@@ -1565,8 +1535,8 @@ void scale_mask_gpu(const double2* H, const double* dsc, const int* keep, int m,
   DEREK_HIP(hipGetLastError());
 }
 
-void big_diag_gpu(double2* A, const int* keep, int m, int batch, hipStream_t s) {
-  hipLaunchKernelGGL(k_big_diag, dim3(batch), dim3(DT), 0, s, A, keep, m);
+void big_diag_gpu(double2* A, const int* keep, const int* na, int m, int batch, hipStream_t s) {
+  hipLaunchKernelGGL(k_big_diag, dim3(batch), dim3(DT), 0, s, A, keep, na, m);
   DEREK_HIP(hipGetLastError());
 }
 

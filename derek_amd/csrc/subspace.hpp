@@ -8,7 +8,7 @@ namespace derek {
 // Scratch for batches of up to `batch` m x m problems with nev wanted pairs.
 struct DenseWork {
   int m = 0, nev = 0, batch = 0;
-  double2 *Wm = nullptr, *Lf = nullptr, *Linv = nullptr, *LinvH = nullptr, *Hc = nullptr, *T = nullptr,
+  double2 *Wm = nullptr, *R = nullptr, *Linv = nullptr, *LinvH = nullptr, *Hc = nullptr, *T = nullptr,
           *A = nullptr, *C = nullptr, *Z = nullptr;
   double *dsc = nullptr, *wtmp = nullptr, *hwork = nullptr;
   int *keep = nullptr, *na = nullptr, *ok = nullptr;
