@@ -43,7 +43,8 @@ template <> struct Mfma<float> {
   __device__ static __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
 };
 
-constexpr int OV_PAD = 66;   // LDS row pitch
+constexpr int OV_PAD = 66;     // LDS row pitch
+constexpr int kOvBlocks = 5;   // 16 x 16 blocks of C per wavefront at most (k_overlap_dealt)
 
 constexpr int kXcds = 8;  // MI355X: 8 XCDs, each with its own L2
 
@@ -177,6 +178,191 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         const double q1 = (double)p1[a][b][r], q2 = (double)p2[a][b][r], q3 = (double)p3[a][b][r];
         if (i < g.m && j < g.n) P[(int64_t)j * g.m + i] = make_double2(q1 + q2, q3 - q1 + q2);
       }
+}
+
+// row groups of the wavefronts of a tile of nblk needed blocks
+__host__ __device__ constexpr int ov_row_groups(int nblk) { return nblk <= 4 ? 4 : (nblk <= 2 * kOvBlocks ? 2 : 1); }
+
+// Whether the tiles of an m x n overlap take the quarter layout: matrix-core
+// steps per slab of the busiest wavefront, summed over the tiles, against the
+// dealt layout's, whose single-use operands cost 9 % per step on full tiles
+// (161214 x 600 x 300: 4.00 against 3.68 ms).
+inline bool ov_quarter(int m, int n, bool herm) {
+  const int tm = (int)ceil_div(m, OV_T), tn = (int)ceil_div(n, OV_T);
+  int64_t quarter = 0, dealt = 0;
+  for (int ti = 0; ti < tm; ++ti)
+    for (int tj = herm ? ti : 0; tj < tn; ++tj) {
+      const int na = std::min(4, (int)ceil_div(m - ti * OV_T, 16)), nb = std::min(4, (int)ceil_div(n - tj * OV_T, 16));
+      const int nblk = herm && ti == tj ? na * (na + 1) / 2 : na * nb, ks = ov_row_groups(nblk);
+      quarter += std::min(2, na) * std::min(2, nb) * 4;
+      dealt += ceil_div(nblk, 4 / ks) * (4 / ks);
+    }
+  return 8 * quarter <= 9 * dealt;
+}
+
+// The same overlap with the 16 x 16 blocks that C needs (inside C; on a
+// diagonal tile of a Hermitian result a <= b) dealt evenly to the wavefronts;
+// with few of them the wavefronts also split each slab's rows (ksp groups,
+// group kgrp takes every ksp-th step of four rows, the sums are added at the
+// end).  A 24-column tile then keeps all four matrix cores busy where a
+// quarter per wavefront leaves three idle.  Measured in FP64, per call: 20
+// columns of 1503 rows 42 -> 10 us (with more row chunks); 48 columns of 17 x
+// 17.5k rows 159 -> 109 us, now near the HBM time of the operands; 160 and 80
+// columns of 62669 rows 212 -> 174 us.  Every operand is read from LDS for
+// each use: full tiles (161214 x 600 x 300) ran 9 % slower than by quarters.
+template <typename R>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_overlap_dealt(const cx_t<R>* __restrict__ X, int64_t ldx, int64_t sx,
+                                                 const cx_t<R>* __restrict__ Y, int64_t ldy, int64_t sy,
+                                                 const int* __restrict__ npwk, OvGeom g,
+                                                 double2* __restrict__ part) {
+  using M = Mfma<R>;
+  using A4 = typename M::acc;
+  using C = cx_t<R>;
+  // slab operands for the three real products of the complex product
+  // conj(x) y (Gauss):  P1 = xr yr,  P2 = xi yi,  P3 = (xr - xi)(yr + yi);
+  // Re = P1 + P2,  Im = P3 - P1 + P2
+  __shared__ __align__(16) R sl[6][OV_KS][OV_PAD];
+  auto xr = sl[0], xi = sl[1], xs = sl[2], yr = sl[3], yi = sl[4], ys = sl[5];
+  // work item: tile fastest, then row chunk, then k-point; the tiles of one
+  // chunk share an XCD and read the same rows through its L2
+  const int64_t w = xcd_item(blockIdx.x, gridDim.x);
+  const int chunk = (int)((w / g.ntiles) % g.nchunk);
+  const int kz = (int)(w / ((int64_t)g.ntiles * g.nchunk));
+  X += kz * sx;
+  Y += kz * sy;
+  const int64_t npw = npwk ? (int64_t)npwk[kz] : g.npw;
+  // tile coordinates
+  int ti, tj;
+  int t = (int)(w % g.ntiles);
+  if (g.herm) {
+    ti = 0;
+    while (t >= g.tm - ti) { t -= g.tm - ti; ++ti; }
+    tj = ti + t;
+  } else {
+    ti = t % g.tm;
+    tj = t / g.tm;
+  }
+  const int i0 = ti * OV_T, j0 = tj * OV_T;
+  const int64_t r0 = (int64_t)chunk * g.kch;
+  const int64_t r1 = std::min<int64_t>(npw, r0 + g.kch);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int na = min(OV_T / 16, (g.m - i0 + 15) / 16), nbk = min(OV_T / 16, (g.n - j0 + 15) / 16);
+  const bool tri = g.herm && ti == tj;
+  const int nblk = tri ? na * (na + 1) / 2 : na * nbk;
+  const int ksp = ov_row_groups(nblk);
+  const int wpg = 4 / ksp, kgrp = wave / wpg;
+  const int per = (nblk + wpg - 1) / wpg;
+  const int q0 = (wave % wpg) * per, nq = max(0, min(per, nblk - q0));
+  constexpr int NQ = kOvBlocks;
+  int ba[NQ], bb[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    int e = max(0, min(q0 + q, nblk - 1));
+    if (tri) {
+      int c = 0;
+      while (e > c) e -= ++c;
+      ba[q] = e * 16;
+      bb[q] = c * 16;
+    } else {
+      ba[q] = (e % na) * 16;
+      bb[q] = (e / na) * 16;
+    }
+  }
+  A4 p1[NQ], p2[NQ], p3[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    p1[q] = A4{0, 0, 0, 0};
+    p2[q] = A4{0, 0, 0, 0};
+    p3[q] = A4{0, 0, 0, 0};
+  }
+  const int lrow = threadIdx.x & 15, lcol = threadIdx.x >> 4;  // 16 rows x 16 column groups
+  // the next slab is loaded into registers while the current one is multiplied
+  C px[4], py[4];
+  auto gload = [&](int64_t k0) {
+    const int64_t gr = k0 + lrow;
+    const bool rok = gr < r1;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int c = lcol + 16 * q;
+      px[q] = (rok && i0 + c < g.m) ? X[(int64_t)(i0 + c) * ldx + gr] : cmk<C>(0, 0);
+      py[q] = (rok && j0 + c < g.n) ? Y[(int64_t)(j0 + c) * ldy + gr] : cmk<C>(0, 0);
+    }
+  };
+  if (r0 < r1) gload(r0);
+  for (int64_t k0 = r0; k0 < r1; k0 += OV_KS) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int c = lcol + 16 * q;
+      xr[lrow][c] = px[q].x;
+      xi[lrow][c] = px[q].y;
+      xs[lrow][c] = px[q].x - px[q].y;
+      yr[lrow][c] = py[q].x;
+      yi[lrow][c] = py[q].y;
+      ys[lrow][c] = py[q].x + py[q].y;
+    }
+    __syncthreads();
+    if (k0 + OV_KS < r1) gload(k0 + OV_KS);
+    // the operands of the next block are read while the current one is multiplied
+    R o[2][6];
+    auto fetch = [&](int kk, int q, R* v) {
+      const int k = kk * 4 + (lane >> 4), ii = ba[q] + (lane & 15), jj = bb[q] + (lane & 15);
+      v[0] = xr[k][ii];
+      v[1] = yr[k][jj];
+      v[2] = xi[k][ii];
+      v[3] = yi[k][jj];
+      v[4] = xs[k][ii];
+      v[5] = ys[k][jj];
+    };
+    for (int kk = kgrp; kk < OV_KS / 4; kk += ksp) {
+      fetch(kk, 0, o[0]);
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        if (q < nq) {
+          if (q + 1 < nq) fetch(kk, q + 1 < NQ ? q + 1 : q, o[(q + 1) & 1]);
+          const R* v = o[q & 1];
+          p1[q] = M::op(v[0], v[1], p1[q]);
+          p2[q] = M::op(v[2], v[3], p2[q]);
+          p3[q] = M::op(v[4], v[5], p3[q]);
+        }
+    }
+    __syncthreads();
+  }
+  // the row groups' sums meet in LDS (the slab buffers), group 0 adds them
+  double2* ex = reinterpret_cast<double2*>(&sl[0][0][0]);
+  static_assert(sizeof(sl) >= 3 * 256 * sizeof(double2) && alignof(R) <= 16, "exchange of one block per wavefront");
+  double2* P = part + ((int64_t)kz * g.nchunk + chunk) * g.m * g.n;
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    double2 v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const double q1 = (double)p1[q][r], q2 = (double)p2[q][r], q3 = (double)p3[q][r];
+      v[r] = make_double2(q1 + q2, q3 - q1 + q2);
+    }
+    // one block of every wavefront at a time: 3 groups x 256 values at most
+    // (ksp 4), 2 wavefronts x 256 (ksp 2)
+    if (ksp > 1) {
+      const int w0 = wave % wpg;
+      if (kgrp > 0 && q < nq)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) ex[(((kgrp - 1) * wpg + w0) * 4 + r) * 64 + lane] = v[r];
+      __syncthreads();
+      if (kgrp == 0 && q < nq)
+        for (int h = 1; h < ksp; ++h)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const double2 u = ex[(((h - 1) * wpg + w0) * 4 + r) * 64 + lane];
+            v[r] = make_double2(v[r].x + u.x, v[r].y + u.y);
+          }
+      __syncthreads();
+    }
+    if (kgrp == 0 && q < nq)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = i0 + ba[q] + M::row(lane, r), j = j0 + bb[q] + (lane & 15);
+        if (i < g.m && j < g.n) P[(int64_t)j * g.m + i] = v[r];
+      }
+  }
 }
 
 // ---- complex64 data on the BF16 matrix cores --------------------------
@@ -491,8 +677,10 @@ void overlap(const cx_t<R>* X, int64_t ldx, int64_t sx, const cx_t<R>* Y, int64_
     else if (bf16_terms == 2)
       hipLaunchKernelGGL((k_overlap_bf16<2, 128>), grid, b128, 0, s, X, ldx, sx, Y, ldy, sy, npwk, g, work);
   }
-  if (bf16_terms == 0)
+  if (bf16_terms == 0 && ov_quarter(m, n, hermitian))
     hipLaunchKernelGGL(k_overlap<R>, grid, dim3(256), 0, s, X, ldx, sx, Y, ldy, sy, npwk, g, work);
+  else if (bf16_terms == 0)
+    hipLaunchKernelGGL(k_overlap_dealt<R>, grid, dim3(256), 0, s, X, ldx, sx, Y, ldy, sy, npwk, g, work);
   DEREK_HIP(hipGetLastError());
   const int64_t mn = (int64_t)m * n;
   hipLaunchKernelGGL(k_overlap_reduce, dim3((unsigned)std::min<int64_t>(4096, ceil_div(mn, RD_E)), batch),
