@@ -874,9 +874,13 @@ int32_t derek_hip_rotate(derek_ctx* c, int64_t npw, int32_t m, int32_t n, const 
     } else {
       float2* fx = c->tD.get<float2>((size_t)(m + n) * npw);
       float2* fz = fx + (size_t)m * npw;
+      const int64_t slots = rotate_work_slots(m, n, 1);
+      double2* work = c->ovwork.get<double2>(slots);
       convert<float, double>(fx, dx, (int64_t)m * npw, c->s);
       c->timed(KC_ROTATE, (double)(m + n) * npw * 8.0, 8.0 * npw * m * n,
-               [&] { rotate<float>(fx, npw, 0, du, m, 0, m, n, npw, nullptr, fz, npw, 0, 1, c->s, c->gemm_bf16); });
+               [&] {
+                 rotate<float>(fx, npw, 0, du, m, 0, m, n, npw, nullptr, fz, npw, 0, 1, c->s, c->gemm_bf16, work, slots);
+               });
       convert<double, float>(dz, fz, (int64_t)n * npw, c->s);
     }
     DEREK_HIP(hipMemcpyAsync(Z, dz, (size_t)n * npw * sizeof(double2), hipMemcpyDeviceToHost, c->s));
@@ -1117,7 +1121,9 @@ int32_t derek_hip_get_tuning(derek_ctx* c, int32_t out[8]) {
     out[4] = c->fused;
     out[5] = c->zsl ? c->zsl : (c->prec == DEREK_FP64 ? 16 : 32);
     out[6] = c->ov_rounds;
-    out[7] = c->ov_tile;
+    // the C tile edge in use; left to the size, the one of the engine's 2nb x 2nb overlaps
+    out[7] = c->ov_tile ? c->ov_tile : 64;
+    if (!c->ov_tile && c->gemm_bf16 == 2 && c->scf && overlap_wide(2 * c->nb, 2 * c->nb, c->max_npw, out[2])) out[7] = 128;
   });
 }
 

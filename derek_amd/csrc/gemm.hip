@@ -552,6 +552,343 @@ __global__ __launch_bounds__(64 * kBfWaves<TT>) __attribute__((amdgpu_waves_per_
       }
 }
 
+// ---- two-term BF16 products of interleaved complex values ----------------
+// For large blocks the complex products are real ones of twice the depth: an
+// operand column is its interleaved (re, im) sequence, split once into a high
+// and a low bf16 term while its slab is staged, and
+//   conj(x) y:  Re = (xr, xi) . (yr, yi),   Im = (xr, xi) . (yi, -yr)
+//   x u:        Re = (xr, -xi) . (ur, ui),  Im = (xi, xr) . (ur, ui)
+// so an operand's other form is a half-word rotation and a sign flip of
+// registers.  Four real products per complex one, where the
+// kernels above take Gauss's three: a third more matrix-core work, but two
+// thirds of the LDS traffic and of the split's vector work, which is what
+// bounded those (10-25 % matrix-core busy), two accumulators per block
+// instead of three, and no cancellation between the products (error against
+// the exact product 4.5e-6 of the largest element against 6.9e-6 at 3001
+// rows).  A wavefront owns 64 x 64 of C or Z: 96 matrix-core instructions per
+// 16 complex rows for 16 operand fragments read.
+constexpr int CX_KS = 16;  // complex rows per slab: one 16x16x32 MFMA of interleaved values
+
+typedef __bf16 bfp __attribute__((ext_vector_type(2)));
+typedef float fp2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+
+typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+
+// term t of the complex value with the FP32 bits (re, im) as one dword (re low, im high)
+__device__ __forceinline__ void cx_split(unsigned re, unsigned im, unsigned (&t)[2]) {
+  const fp2 f = {__builtin_bit_cast(float, re), __builtin_bit_cast(float, im)};
+  const bfp h = __builtin_convertvector(f, bfp);
+  const fp2 hf = __builtin_convertvector(h, fp2);
+  const bfp l = __builtin_convertvector(f - hf, bfp);
+  t[0] = __builtin_bit_cast(unsigned, h);
+  t[1] = __builtin_bit_cast(unsigned, l);
+}
+// (re, im) -> (im, -re)
+__device__ __forceinline__ u4 cx_swap(u4 v) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = __builtin_amdgcn_alignbit(v[e], v[e], 16) ^ 0x80000000u;
+  return v;
+}
+__device__ __forceinline__ f4 cx_mfma(u4 a, u4 b, f4 c) {
+  return mfma_bf16(__builtin_bit_cast(bf8, a), __builtin_bit_cast(bf8, b), c);
+}
+// LDS slot (16 bytes: four complex values of one term) of column c, row group
+// g of a slab; the XOR keeps the 16 lanes of an access on distinct banks
+__device__ __forceinline__ int cx_slot(int c, int g) { return c * 4 + (g ^ ((c >> 2) & 3)); }
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_overlap_cx(
+    const float2* __restrict__ X, int64_t ldx, int64_t sx, const float2* __restrict__ Y, int64_t ldy, int64_t sy,
+    const int* __restrict__ npwk, OvGeom g, double2* __restrict__ part) {
+  constexpr int TT = 128;
+  __shared__ u4 lx[2][2][TT * 4], ly[2][2][TT * 4];  // [buffer][term][slot]
+  const int64_t w = xcd_item(blockIdx.x, gridDim.x);
+  const int chunk = (int)((w / g.ntiles) % g.nchunk);
+  const int kz = (int)(w / ((int64_t)g.ntiles * g.nchunk));
+  X += kz * sx;
+  Y += kz * sy;
+  const int64_t npw = npwk ? (int64_t)npwk[kz] : g.npw;
+  int ti, tj;
+  int t = (int)(w % g.ntiles);
+  if (g.herm) {
+    ti = 0;
+    while (t >= g.tm - ti) { t -= g.tm - ti; ++ti; }
+    tj = ti + t;
+  } else {
+    ti = t % g.tm;
+    tj = t / g.tm;
+  }
+  const int i0 = ti * TT, j0 = tj * TT;
+  const int64_t r0 = (int64_t)chunk * g.kch;
+  const int64_t r1 = std::min<int64_t>(npw, r0 + g.kch);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ri = (wave & 1) * 64, cj = (wave >> 1) * 64;
+  // 16-column blocks of this wavefront inside C; none below the diagonal of a
+  // Hermitian result
+  int na = max(0, min(4, (g.m - i0 - ri + 15) / 16)), nb = max(0, min(4, (g.n - j0 - cj + 15) / 16));
+  if (g.herm && ti == tj && ri > cj) nb = 0;
+  f4 re[4][4], im[4][4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) re[a][b] = im[a][b] = f4{0, 0, 0, 0};
+  // staging: pass q, column 32 q + thread / 8, rows 2 (thread % 8) and the
+  // next, one 16-byte buffer load (columns past C: out of range, zero); only
+  // the last slab of a chunk masks rows
+  const int sc = threadIdx.x >> 3, sp = threadIdx.x & 7;
+  const int64_t lastx = (int64_t)(min(TT, g.m - i0) - 1) * ldx, lasty = (int64_t)(min(TT, g.n - j0) - 1) * ldy;
+  uint32_t ox[4], oy[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int c = 32 * q + sc;
+    ox[q] = i0 + c < g.m ? (uint32_t)(c * ldx + 2 * sp) * 8u : kOob;
+    oy[q] = j0 + c < g.n ? (uint32_t)(c * ldy + 2 * sp) * 8u : kOob;
+  }
+  u4 px[4], py[4];
+  auto gload = [&](int64_t k0) {
+    const int rows = (int)min((int64_t)CX_KS, r1 - k0) - 2 * sp;  // of this lane's two
+    const auto rx = buf_rsrc(X + (int64_t)i0 * ldx + k0, (uint32_t)((lastx + r1 - k0) * 8));
+    const auto ry = buf_rsrc(Y + (int64_t)j0 * ldy + k0, (uint32_t)((lasty + r1 - k0) * 8));
+    if (r1 - k0 >= CX_KS) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        px[q] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)ox[q], 0, 0);
+        py[q] = __builtin_amdgcn_raw_buffer_load_b128(ry, (int)oy[q], 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const u2 zero = {0u, 0u};
+        const u2 x0 = rows > 0 ? __builtin_amdgcn_raw_buffer_load_b64(rx, (int)ox[q], 0, 0) : zero;
+        const u2 x1 = rows > 1 ? __builtin_amdgcn_raw_buffer_load_b64(rx, (int)ox[q] + 8, 0, 0) : zero;
+        const u2 y0 = rows > 0 ? __builtin_amdgcn_raw_buffer_load_b64(ry, (int)oy[q], 0, 0) : zero;
+        const u2 y1 = rows > 1 ? __builtin_amdgcn_raw_buffer_load_b64(ry, (int)oy[q] + 8, 0, 0) : zero;
+        px[q] = u4{x0[0], x0[1], x1[0], x1[1]};
+        py[q] = u4{y0[0], y0[1], y1[0], y1[1]};
+      }
+    }
+  };
+  auto put = [&](u4 (&l)[2][TT * 4], int c, u4 v) {
+    unsigned t0[2], t1[2];
+    cx_split(v[0], v[1], t0);
+    cx_split(v[2], v[3], t1);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      reinterpret_cast<uint2*>(&l[q][cx_slot(c, sp >> 1)])[sp & 1] = make_uint2(t0[q], t1[q]);
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      put(lx[buf], 32 * q + sc, px[q]);
+      put(ly[buf], 32 * q + sc, py[q]);
+    }
+  };
+  const int lc = lane & 15, kg = lane >> 4;
+  if (r0 < r1) {
+    gload(r0);
+    stage(0);
+  }
+  __syncthreads();
+  int buf = 0;
+  for (int64_t k0 = r0; k0 < r1; k0 += CX_KS, buf ^= 1) {
+    const bool more = k0 + CX_KS < r1;
+    if (more) gload(k0 + CX_KS);
+    u4 A[4][2];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) A[a][q] = lx[buf][q][cx_slot(ri + a * 16 + lc, kg)];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      if (b < nb) {
+        u4 B[2], D[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          B[q] = ly[buf][q][cx_slot(cj + b * 16 + lc, kg)];
+          D[q] = cx_swap(B[q]);
+        }
+        // smallest terms first
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+          if (a < na) {
+            re[a][b] = cx_mfma(A[a][0], B[1], re[a][b]);
+            im[a][b] = cx_mfma(A[a][0], D[1], im[a][b]);
+            re[a][b] = cx_mfma(A[a][1], B[0], re[a][b]);
+            im[a][b] = cx_mfma(A[a][1], D[0], im[a][b]);
+            re[a][b] = cx_mfma(A[a][0], B[0], re[a][b]);
+            im[a][b] = cx_mfma(A[a][0], D[0], im[a][b]);
+          }
+      }
+    if (more) stage(buf ^ 1);
+    __syncthreads();
+  }
+  double2* P = part + ((int64_t)kz * g.nchunk + chunk) * g.m * g.n;
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      if (a < na && b < nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = i0 + ri + a * 16 + Mfma<float>::row(lane, r), j = j0 + cj + b * 16 + lc;
+          if (i < g.m && j < g.n) P[(int64_t)j * g.m + i] = make_double2((double)re[a][b][r], (double)im[a][b][r]);
+        }
+}
+
+// Z = X U, 128 rows x 128 columns per workgroup, 64 x 64 per wavefront.  U is
+// split once per call (k_rotate_split) into the LDS images of its slabs, 16
+// rows x 128 columns in two terms, which each workgroup copies in 16-byte
+// pieces; X's rows go straight into the A fragments (lane: one row, four
+// columns of X).
+constexpr int RC_ROWS = 128, RC_COLS = 128;
+constexpr int RC_IMG = 2 * RC_COLS * 4;  // 16-byte slots of one slab image: [term][slot]
+
+// image (column block, slab) of matrix kz at img + ((kz*ncb + block)*nslab + slab)*RC_IMG
+__global__ __launch_bounds__(256) void k_rotate_split(const double2* __restrict__ U, int ldu, int64_t su, int m, int n,
+                                                      u4* __restrict__ img) {
+  const int nslab = gridDim.x, slab = blockIdx.x, cb = blockIdx.y;
+  U += blockIdx.z * su;
+  img += (((int64_t)blockIdx.z * gridDim.y + cb) * nslab + slab) * RC_IMG;
+  for (int s = threadIdx.x; s < RC_COLS * 4; s += 256) {
+    const int c = s >> 2, g = s & 3, col = cb * RC_COLS + c;
+    u4 h, l;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int k = slab * CX_KS + 4 * g + e;
+      const double2 v = (k < m && col < n) ? U[(int64_t)col * ldu + k] : make_double2(0.0, 0.0);
+      unsigned t[2];
+      cx_split(__builtin_bit_cast(unsigned, (float)v.x), __builtin_bit_cast(unsigned, (float)v.y), t);
+      h[e] = t[0];
+      l[e] = t[1];
+    }
+    img[cx_slot(c, g)] = h;
+    img[RC_COLS * 4 + cx_slot(c, g)] = l;
+  }
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_rotate_cx(
+    const float2* __restrict__ X, const float2* __restrict__ X2, int64_t ldx, int64_t sx, const u4* __restrict__ img,
+    int m, int n, int64_t npw, const int* __restrict__ npwk, float2* __restrict__ Z, float2* __restrict__ Z2,
+    int64_t ldz, int64_t sz) {
+  __shared__ u4 lu[2][RC_IMG];
+  const int ncb = (int)ceil_div(n, RC_COLS), nslab = (int)ceil_div(m, CX_KS);
+  const int64_t nrb = ceil_div(npw, RC_ROWS);
+  const int64_t w = xcd_item(blockIdx.x, gridDim.x);
+  const int64_t rb = (w / ncb) % nrb;
+  const int kz = (int)(w / (ncb * nrb));
+  const int64_t nrow = npwk ? (int64_t)npwk[kz] : npw;
+  if (rb * RC_ROWS >= nrow) return;
+  X = (blockIdx.y ? X2 : X) + kz * sx;
+  Z = (blockIdx.y ? Z2 : Z) + kz * sz;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int cb = (int)(w % ncb), j0 = cb * RC_COLS;
+  img += ((int64_t)kz * ncb + cb) * nslab * RC_IMG;
+  const int64_t g0 = rb * RC_ROWS + wave * 32;
+  const int lc = lane & 15, kg = lane >> 4;
+  const int na = (int)max((int64_t)0, min((int64_t)2, (nrow - g0 + 15) / 16));
+  const int nb = min(8, (n - j0 + 15) / 16);
+  f4 re[2][8], im[2][8];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 8; ++b) re[a][b] = im[a][b] = f4{0, 0, 0, 0};
+  // X: lane offsets of row lc of the wavefront's block, columns 4 kg + e.
+  // Rows past the k-point's only reach rows of Z that are not stored; columns
+  // past m read zero.
+  uint32_t xo[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) xo[e] = (uint32_t)((4 * kg + e) * ldx + lc) * 8u;
+  constexpr int UQ = RC_IMG / 256;
+  u4 pu[UQ];
+  u2 p0[2][4] = {}, p1[2][4] = {};
+  auto uload = [&](int s) {
+    const u4* is = img + (int64_t)s * RC_IMG + threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < UQ; ++q) pu[q] = is[q * 256];
+  };
+  auto xload = [&](int s, u2 (&px)[2][4]) {
+    if (na == 0 || s >= nslab) return;
+    const int k0 = s * CX_KS;
+    // in range: rows past the k-point's of all columns but the last, zero past that
+    const auto rx = buf_rsrc(X + (int64_t)k0 * ldx + g0, (uint32_t)(((m - 1 - k0) * ldx + nrow - g0) * 8));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t o = k0 + 4 * kg + e < m ? xo[e] : kOob;
+#pragma unroll
+      for (int a = 0; a < 2; ++a) px[a][e] = __builtin_amdgcn_raw_buffer_load_b64(rx, (int)(o + a * 128), 0, 0);
+    }
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < UQ; ++q) lu[buf][q * 256 + threadIdx.x] = pu[q];
+  };
+  auto step = [&](int s, u2 (&px)[2][4]) {
+    const int buf = s & 1;
+    // (xr, -xi) for Re and (xi, xr) for Im against the same (ur, ui)
+    u4 A[2][2], D[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        unsigned t[2];
+        cx_split(px[a][e][0], px[a][e][1], t);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          A[a][q][e] = t[q] ^ 0x80000000u;
+          D[a][q][e] = __builtin_amdgcn_alignbit(t[q], t[q], 16);
+        }
+      }
+    const bool more = s + 1 < nslab;
+    if (more) uload(s + 1);
+    xload(s + 2, px);
+#pragma unroll
+    for (int b = 0; b < 8; ++b)
+      if (b < nb) {
+        u4 B[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) B[q] = lu[buf][q * RC_COLS * 4 + cx_slot(b * 16 + lc, kg)];
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          re[a][b] = cx_mfma(A[a][0], B[1], re[a][b]);
+          im[a][b] = cx_mfma(D[a][0], B[1], im[a][b]);
+        }
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          re[a][b] = cx_mfma(A[a][1], B[0], re[a][b]);
+          im[a][b] = cx_mfma(D[a][1], B[0], im[a][b]);
+        }
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          re[a][b] = cx_mfma(A[a][0], B[0], re[a][b]);
+          im[a][b] = cx_mfma(D[a][0], B[0], im[a][b]);
+        }
+      }
+    if (more) stage(buf ^ 1);
+    __syncthreads();
+  };
+  xload(0, p0);
+  xload(1, p1);
+  uload(0);
+  stage(0);
+  __syncthreads();
+  for (int s = 0; s < nslab; s += 2) {
+    step(s, p0);
+    if (s + 1 < nslab) step(s + 1, p1);
+  }
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const int j = j0 + b * 16 + lc;
+    if (j >= n) continue;
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t gg = g0 + a * 16 + Mfma<float>::row(lane, r);
+        if (gg < nrow) Z[(int64_t)j * ldz + gg] = make_float2(re[a][b][r], im[a][b][r]);
+      }
+  }
+}
+
 // resident 256-thread workgroups of `kern` on the current device (CUs x
 // per-CU occupancy)
 static int resident_slots(const void* kern, int threads) {
@@ -572,6 +909,11 @@ template <int NT, int TT> static int ov_slots_bf16() {
   return slots;
 }
 
+static int ov_slots_cx() {
+  static const int slots = resident_slots(reinterpret_cast<const void*>(k_overlap_cx), 256);
+  return slots;
+}
+
 // resident slots of every overlap kernel (FP64, FP32, BF16 with 1..3 terms
 // on 64- and 128-wide tiles)
 constexpr int kOvKernels = 8;
@@ -583,7 +925,7 @@ static void overlap_slots(int out[kOvKernels]) {
   out[4] = ov_slots_bf16<3, 64>();
   out[5] = ov_slots_bf16<1, 128>();
   out[6] = ov_slots_bf16<2, 128>();
-  out[7] = out[6];
+  out[7] = ov_slots_cx();
 }
 
 int64_t overlap_work_elems(int m, int n, int64_t npw, int batch) {
@@ -640,6 +982,16 @@ __global__ __launch_bounds__(RD_E * RD_G) void k_overlap_reduce(const double2* _
   }
 }
 
+// Two-term overlaps whose tile edge is left to the size take k_overlap_cx
+// once both sides exceed 64 columns and the rows keep every CU busy (8 x
+// 161214 rows, 600 columns 9.1 -> 5.4 ms, 300 columns 2.7 -> 2.1 ms; 64 x
+// 17529 rows, 96 columns 0.47 -> 0.30 ms, 48 columns 0.17 -> 0.21 ms; one
+// k-point of 62669 rows, 160 columns 85 and 82 us, 320 columns 177 and 186
+// us), the 64-wide k_overlap_bf16 otherwise.
+bool overlap_wide(int m, int n, int64_t npw, int batch) {
+  return std::min(m, n) > 64 && npw * batch >= 131072;
+}
+
 template <typename R>
 void overlap(const cx_t<R>* X, int64_t ldx, int64_t sx, const cx_t<R>* Y, int64_t ldy, int64_t sy, int m, int n,
              int64_t npw, const int* npwk, double2* C, int ldc, int64_t sc, int batch, double2* work,
@@ -649,14 +1001,19 @@ void overlap(const cx_t<R>* X, int64_t ldx, int64_t sx, const cx_t<R>* Y, int64_
   DEREK_REQUIRE(!hermitian || m == n, "overlap: hermitian needs a square result");
   DEREK_REQUIRE(bf16_terms == 0 || (std::is_same<R, float>::value && bf16_terms >= 1 && bf16_terms <= 3),
                 "overlap: bf16 terms must be 0, or 1..3 for complex64 data");
-  DEREK_REQUIRE(tile == 64 || tile == 128, "overlap: tile must be 64 or 128");
+  DEREK_REQUIRE(tile == 0 || tile == 64 || tile == 128, "overlap: tile must be 64 or 128 (0: by size)");
+  // a tile's columns span less than 2 GiB (32-bit offsets)
+  const bool cx = tile == 0 && bf16_terms == 2 && overlap_wide(m, n, npw, batch) &&
+                  128 * std::max(ldx, ldy) * 8 < (int64_t)kOob;
+  if (tile == 0) tile = 64;
   // the 128-wide tile exists for the BF16 kernels with 1 or 2 terms (three
   // terms of a 128-wide tile need 180 KB of LDS)
-  const int tt = bf16_terms && bf16_terms < 3 ? tile : 64;
-  const int slots = bf16_terms == 1   ? (tt == 128 ? ov_slots_bf16<1, 128>() : ov_slots_bf16<1, 64>())
-                    : bf16_terms == 2 ? (tt == 128 ? ov_slots_bf16<2, 128>() : ov_slots_bf16<2, 64>())
-                    : bf16_terms == 3 ? ov_slots_bf16<3, 64>()
-                                      : ov_slots<R>();
+  const int tt = cx ? 128 : (bf16_terms && bf16_terms < 3 ? tile : 64);
+  const int slots = cx                  ? ov_slots_cx()
+                    : bf16_terms == 1   ? (tt == 128 ? ov_slots_bf16<1, 128>() : ov_slots_bf16<1, 64>())
+                    : bf16_terms == 2   ? (tt == 128 ? ov_slots_bf16<2, 128>() : ov_slots_bf16<2, 64>())
+                    : bf16_terms == 3   ? ov_slots_bf16<3, 64>()
+                                        : ov_slots<R>();
   DEREK_REQUIRE(rounds == 1 || rounds == 2 || rounds == 4, "overlap: rounds must be 1, 2 or 4");
   OvGeom g = ov_geom(m, n, npw, hermitian, batch, slots, bf16_terms ? BF_KS : OV_KS, rounds, tt);
   ov_limit_chunks(g, max_chunks, bf16_terms ? BF_KS : OV_KS);
@@ -666,7 +1023,9 @@ void overlap(const cx_t<R>* X, int64_t ldx, int64_t sx, const cx_t<R>* Y, int64_
   const dim3 grid((unsigned)items);
   if constexpr (std::is_same<R, float>::value) {
     const dim3 b64(64 * kBfWaves<64>), b128(64 * kBfWaves<128>);
-    if (bf16_terms == 1 && tt == 64)
+    if (cx)
+      hipLaunchKernelGGL(k_overlap_cx, grid, dim3(256), 0, s, X, ldx, sx, Y, ldy, sy, npwk, g, work);
+    else if (bf16_terms == 1 && tt == 64)
       hipLaunchKernelGGL((k_overlap_bf16<1, 64>), grid, b64, 0, s, X, ldx, sx, Y, ldy, sy, npwk, g, work);
     else if (bf16_terms == 2 && tt == 64)
       hipLaunchKernelGGL((k_overlap_bf16<2, 64>), grid, b64, 0, s, X, ldx, sx, Y, ldy, sy, npwk, g, work);
@@ -693,10 +1052,11 @@ constexpr int RT_COLS = 64;
 constexpr int RT_KS = 16;
 
 template <typename R>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_rotate(const cx_t<R>* __restrict__ X, int64_t ldx, int64_t sx,
-                                                const double2* __restrict__ U, int ldu, int64_t su, int m, int n,
-                                                int64_t npw, const int* __restrict__ npwk, cx_t<R>* __restrict__ Z,
-                                                int64_t ldz, int64_t sz) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_rotate(const cx_t<R>* __restrict__ X, const cx_t<R>* __restrict__ X2,
+                                                int64_t ldx, int64_t sx, const double2* __restrict__ U, int ldu,
+                                                int64_t su, int m, int n, int64_t npw, const int* __restrict__ npwk,
+                                                cx_t<R>* __restrict__ Z, cx_t<R>* __restrict__ Z2, int64_t ldz,
+                                                int64_t sz) {
   using M = Mfma<R>;
   using A4 = typename M::acc;
   using C = cx_t<R>;
@@ -715,9 +1075,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t g0 = rb * RT_ROWS + wave * 16;
   if (rb * RT_ROWS >= nrow) return;
-  X += kz * sx;
+  X = (blockIdx.y ? X2 : X) + kz * sx;
   U += kz * su;
-  Z += kz * sz;
+  Z = (blockIdx.y ? Z2 : Z) + kz * sz;
   const int j0 = (int)(w % ncb) * RT_COLS;
   // 16-column blocks past n, and a wavefront whose 16 rows are all past the
   // k-point's plane waves, skip the matrix cores (wave-uniform)
@@ -799,8 +1159,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // A operand (8 consecutive k of the lane's row) is split in registers.
 template <int NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_rotate_bf16(
-    const float2* __restrict__ X, int64_t ldx, int64_t sx, const double2* __restrict__ U, int ldu, int64_t su, int m,
-    int n, int64_t npw, const int* __restrict__ npwk, float2* __restrict__ Z, int64_t ldz, int64_t sz) {
+    const float2* __restrict__ X, const float2* __restrict__ X2, int64_t ldx, int64_t sx,
+    const double2* __restrict__ U, int ldu, int64_t su, int m, int n, int64_t npw, const int* __restrict__ npwk,
+    float2* __restrict__ Z, float2* __restrict__ Z2, int64_t ldz, int64_t sz) {
   // x u = P1 - P2 + i (P3 - P1 - P2), P1 = xr ur, P2 = xi ui, P3 = (xr + xi)(ur + ui)
   __shared__ bf8 lu[3][NT][64][BF_P];
   const int ncb = (int)ceil_div(n, RT_COLS);
@@ -811,9 +1172,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   const int64_t nrow = npwk ? (int64_t)npwk[kz] : npw;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (rb * RT_ROWS >= nrow) return;
-  X += kz * sx;
+  X = (blockIdx.y ? X2 : X) + kz * sx;
   U += kz * su;
-  Z += kz * sz;
+  Z = (blockIdx.y ? Z2 : Z) + kz * sz;
   const int j0 = (int)(w % ncb) * RT_COLS;
   // 16-column blocks past n, and a wavefront whose 16 rows are all past the
   // k-point's plane waves, skip the matrix cores (wave-uniform)
@@ -902,26 +1263,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   }
 }
 
+int64_t rotate_work_slots(int m, int n, int batch) {
+  return ceil_div(m, CX_KS) * ceil_div(n, RC_COLS) * RC_IMG * batch;
+}
+
 template <typename R>
-void rotate(const cx_t<R>* X, int64_t ldx, int64_t sx, const double2* U, int ldu, int64_t su, int m, int n,
-            int64_t npw, const int* npwk, cx_t<R>* Z, int64_t ldz, int64_t sz, int batch, hipStream_t s,
-            int bf16_terms) {
+void rotate2(const cx_t<R>* X, const cx_t<R>* X2, int64_t ldx, int64_t sx, const double2* U, int ldu, int64_t su, int m,
+             int n, int64_t npw, const int* npwk, cx_t<R>* Z, cx_t<R>* Z2, int64_t ldz, int64_t sz, int batch,
+             hipStream_t s, int bf16_terms, void* work, int64_t work_slots) {
   DEREK_REQUIRE(m > 0 && n > 0 && batch > 0, "rotate: empty block");
   DEREK_REQUIRE(bf16_terms == 0 || (std::is_same<R, float>::value && bf16_terms >= 1 && bf16_terms <= 3),
                 "rotate: bf16 terms must be 0, or 1..3 for complex64 data");
   const int64_t items = ceil_div(npw, RT_ROWS) * ceil_div(n, RT_COLS) * batch;
   DEREK_REQUIRE(items < (int64_t)1 << 31, "rotate: too many workgroups");
-  const dim3 grid((unsigned)items);
+  const unsigned two = X2 ? 2 : 1;
+  const dim3 grid((unsigned)items, two);
   if constexpr (std::is_same<R, float>::value) {
-    if (bf16_terms == 1)
-      hipLaunchKernelGGL(k_rotate_bf16<1>, grid, dim3(256), 0, s, X, ldx, sx, U, ldu, su, m, n, npw, npwk, Z, ldz, sz);
-    else if (bf16_terms == 2)
-      hipLaunchKernelGGL(k_rotate_bf16<2>, grid, dim3(256), 0, s, X, ldx, sx, U, ldu, su, m, n, npw, npwk, Z, ldz, sz);
-    else if (bf16_terms == 3)
-      hipLaunchKernelGGL(k_rotate_bf16<3>, grid, dim3(256), 0, s, X, ldx, sx, U, ldu, su, m, n, npw, npwk, Z, ldz, sz);
+    // two terms: the 128-row workgroups once there is one per CU (600 -> 300
+    // columns of 8 x 161214 rows 10.2 -> 5.3 ms, 48 -> 24 of 64 x 17529 0.248
+    // -> 0.183 ms; with 125 workgroups, 80 -> 40 of 4 x 4000 rows, 13 against
+    // 18 us), a buffer for the split U and 32-bit offsets
+    const int64_t wide = ceil_div(npw, RC_ROWS) * ceil_div(n, RC_COLS) * batch;
+    if (bf16_terms == 2 && wide * two >= 256 && work && rotate_work_slots(m, n, batch) <= work_slots &&
+        (int64_t)m * ldx * 8 < (int64_t)kOob) {
+      u4* img = reinterpret_cast<u4*>(work);
+      hipLaunchKernelGGL(k_rotate_split, dim3((unsigned)ceil_div(m, CX_KS), (unsigned)ceil_div(n, RC_COLS), batch),
+                         dim3(256), 0, s, U, ldu, su, m, n, img);
+      hipLaunchKernelGGL(k_rotate_cx, dim3((unsigned)wide, two), dim3(256), 0, s, X, X2, ldx, sx, img, m, n, npw, npwk, Z,
+                         Z2, ldz, sz);
+    } else if (bf16_terms == 1) {
+      hipLaunchKernelGGL(k_rotate_bf16<1>, grid, dim3(256), 0, s, X, X2, ldx, sx, U, ldu, su, m, n, npw, npwk, Z, Z2, ldz,
+                         sz);
+    } else if (bf16_terms == 2) {
+      hipLaunchKernelGGL(k_rotate_bf16<2>, grid, dim3(256), 0, s, X, X2, ldx, sx, U, ldu, su, m, n, npw, npwk, Z, Z2, ldz,
+                         sz);
+    } else if (bf16_terms == 3) {
+      hipLaunchKernelGGL(k_rotate_bf16<3>, grid, dim3(256), 0, s, X, X2, ldx, sx, U, ldu, su, m, n, npw, npwk, Z, Z2, ldz,
+                         sz);
+    }
   }
   if (bf16_terms == 0)
-    hipLaunchKernelGGL(k_rotate<R>, grid, dim3(256), 0, s, X, ldx, sx, U, ldu, su, m, n, npw, npwk, Z, ldz, sz);
+    hipLaunchKernelGGL(k_rotate<R>, grid, dim3(256), 0, s, X, X2, ldx, sx, U, ldu, su, m, n, npw, npwk, Z, Z2, ldz, sz);
   DEREK_HIP(hipGetLastError());
 }
 
@@ -931,9 +1313,11 @@ template void overlap<double>(const double2*, int64_t, int64_t, const double2*, 
 template void overlap<float>(const float2*, int64_t, int64_t, const float2*, int64_t, int64_t, int, int, int64_t,
                              const int*, double2*, int, int64_t, int, double2*, int64_t, bool, hipStream_t, int,
                              int64_t, int, int);
-template void rotate<double>(const double2*, int64_t, int64_t, const double2*, int, int64_t, int, int, int64_t,
-                             const int*, double2*, int64_t, int64_t, int, hipStream_t, int);
-template void rotate<float>(const float2*, int64_t, int64_t, const double2*, int, int64_t, int, int, int64_t,
-                            const int*, float2*, int64_t, int64_t, int, hipStream_t, int);
+template void rotate2<double>(const double2*, const double2*, int64_t, int64_t, const double2*, int, int64_t, int, int,
+                              int64_t, const int*, double2*, double2*, int64_t, int64_t, int, hipStream_t, int, void*,
+                              int64_t);
+template void rotate2<float>(const float2*, const float2*, int64_t, int64_t, const double2*, int, int64_t, int, int,
+                             int64_t, const int*, float2*, float2*, int64_t, int64_t, int, hipStream_t, int, void*,
+                             int64_t);
 
 }  // namespace derek

@@ -49,6 +49,9 @@ template <typename R> void run(int64_t npw, int nb, int batch, int terms = 0, in
   check(hipGetLastError(), "fill");
   const int64_t cap = std::max(overlap_work_elems(m2, m2, npw, batch), overlap_work_elems(nb, nb, npw, batch));
   check(hipMalloc(&work, sizeof(double2) * cap), "hipMalloc");
+  const int64_t slots = rotate_work_slots(m2, nb, batch);
+  double2* rwork = nullptr;
+  check(hipMalloc(&rwork, sizeof(double2) * slots), "hipMalloc");
   hipEvent_t a, b;
   check(hipEventCreate(&a), "hipEventCreate");
   check(hipEventCreate(&b), "hipEventCreate");
@@ -86,7 +89,7 @@ template <typename R> void run(int64_t npw, int nb, int batch, int terms = 0, in
     });
     std::snprintf(w, sizeof w, "rotate %d->%d", m, nb);
     timeit(w, 8.0 * m * nb * npw * batch, [&] {
-      rotate<R>(X, ld, ks, U, m2, (int64_t)m2 * m2, m, nb, npw, nullptr, Z, ld, ks, batch, 0, terms);
+      rotate<R>(X, ld, ks, U, m2, (int64_t)m2 * m2, m, nb, npw, nullptr, Z, ld, ks, batch, 0, terms, rwork, slots);
     });
   }
   check(hipFree(X), "hipFree");
@@ -94,6 +97,7 @@ template <typename R> void run(int64_t npw, int nb, int batch, int terms = 0, in
   check(hipFree(S), "hipFree");
   check(hipFree(U), "hipFree");
   check(hipFree(work), "hipFree");
+  check(hipFree(rwork), "hipFree");
 }
 
 int main(int argc, char** argv) {

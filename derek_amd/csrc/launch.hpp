@@ -62,7 +62,9 @@ void transpose_xz(const double* v, double* t64, float* t32, int nx, int ny, int 
 // `work` (work_cap double2, checked) must hold overlap_work_elems(m, n, npw, batch),
 // or batch * max_chunks * m * n when max_chunks > 0 caps the row chunks;
 // `rounds` (1, 2, 4): rounds of resident workgroups the row chunks fill at least;
-// `tile` (64, 128): the C tile edge of the BF16 kernels (the others take 64).
+// `tile` (64, 128): the C tile edge of the BF16 kernels (the others take 64);
+// 0: by size, 64 or, for the large two-term overlaps (overlap_wide), the
+// 128-wide kernel on interleaved values.
 // bf16_terms (complex64 data only): 0 multiplies on the FP32 matrix cores;
 // 1..3 on the BF16 ones with every FP32 value split into that many bf16
 // terms (1: plain BF16, 2: ~16 significant bits, 3: ~FP32), FP32 accumulation.
@@ -75,11 +77,23 @@ void overlap(const cx_t<R>* X, int64_t ldx, int64_t sx, const cx_t<R>* Y, int64_
              int64_t npw, const int* npwk, double2* C, int ldc, int64_t sc, int batch, double2* work,
              int64_t work_cap, bool hermitian, hipStream_t s, int bf16_terms = 0, int64_t max_chunks = 0,
              int rounds = 2, int tile = 64);
+bool overlap_wide(int m, int n, int64_t npw, int batch);
 // Z (npw x n, ldz) = X (npw x m, ldx) * U (m x n, FP64, column-major, ldu),
-// U rounded to R; bf16_terms as for overlap.
+// U rounded to R; bf16_terms as for overlap.  rotate2 also forms Z2 = X2 U
+// (X2 nullable) in the same launch.  work: rotate_work_slots(m, n, batch)
+// 16-byte slots for the split U of the large two-term rotations, which
+// otherwise (null or too small) take the kernel that splits U as it goes.
+int64_t rotate_work_slots(int m, int n, int batch);
 template <typename R>
-void rotate(const cx_t<R>* X, int64_t ldx, int64_t sx, const double2* U, int ldu, int64_t su, int m, int n,
-            int64_t npw, const int* npwk, cx_t<R>* Z, int64_t ldz, int64_t sz, int batch, hipStream_t s,
-            int bf16_terms = 0);
+void rotate2(const cx_t<R>* X, const cx_t<R>* X2, int64_t ldx, int64_t sx, const double2* U, int ldu, int64_t su, int m,
+             int n, int64_t npw, const int* npwk, cx_t<R>* Z, cx_t<R>* Z2, int64_t ldz, int64_t sz, int batch,
+             hipStream_t s, int bf16_terms = 0, void* work = nullptr, int64_t work_slots = 0);
+template <typename R>
+inline void rotate(const cx_t<R>* X, int64_t ldx, int64_t sx, const double2* U, int ldu, int64_t su, int m, int n,
+                   int64_t npw, const int* npwk, cx_t<R>* Z, int64_t ldz, int64_t sz, int batch, hipStream_t s,
+                   int bf16_terms = 0, void* work = nullptr, int64_t work_slots = 0) {
+  rotate2<R>(X, nullptr, ldx, sx, U, ldu, su, m, n, npw, npwk, Z, nullptr, ldz, sz, batch, s, bf16_terms, work,
+             work_slots);
+}
 
 }  // namespace derek

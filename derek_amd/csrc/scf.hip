@@ -42,6 +42,8 @@ struct ScfEngine {
   void *Y = nullptr, *HY = nullptr, *Y2 = nullptr, *HY2 = nullptr;
   double2 *S = nullptr, *H = nullptr, *U = nullptr, *ovw = nullptr;
   int64_t ovw_cap = 0;  // double2 elements of ovw
+  double2* rotw = nullptr;  // split U of the two-term BF16 rotations (complex64 phase)
+  int64_t rotw_slots = 0;
   DenseWork dw;
   double *eps = nullptr, *ekin = nullptr, *rn = nullptr, *occ = nullptr, *occw = nullptr, *stats_partial = nullptr;
   double *rho_in = nullptr, *rho_out = nullptr, *vh = nullptr, *vxc = nullptr, *vhxc = nullptr, *tmp1 = nullptr,
@@ -148,14 +150,16 @@ void ov_block(derek_ctx* c, const cx_t<R>* X, int ca, const cx_t<R>* Yp, int cb,
   });
 }
 
-// Z[kz] (n columns) = X[kz] (m columns) U[kz] (m x n, ld m, stride su)
+// Z[kz] (n columns) = X[kz] (m columns) U[kz] (m x n, ld m, stride su), and
+// Z2 = X2 U with the same U (X2 nullable) in one launch
 template <typename R>
-void rot(derek_ctx* c, const cx_t<R>* X, const double2* Uc, int m, int n, int64_t su, int k0, int nkc, cx_t<R>* Z) {
+void rot(derek_ctx* c, const cx_t<R>* X, const cx_t<R>* X2, const double2* Uc, int m, int n, int64_t su, int k0, int nkc,
+         cx_t<R>* Z, cx_t<R>* Z2) {
   ScfEngine& E = *c->scf;
-  const double npw = npw_sum(c, k0, nkc);
+  const double npw = (X2 ? 2.0 : 1.0) * npw_sum(c, k0, nkc);
   c->timed(KC_ROTATE, (double)(m + n) * npw * sizeof(cx_t<R>), 8.0 * npw * m * n, [&] {
-    rotate<R>(X, E.ldk, E.kstride, Uc, m, su, m, n, c->max_npw, c->d_npw + k0, Z, E.ldk, E.kstride, nkc, c->s,
-              bf16_terms<R>(c));
+    rotate2<R>(X, X2, E.ldk, E.kstride, Uc, m, su, m, n, c->max_npw, c->d_npw + k0, Z, Z2, E.ldk, E.kstride, nkc, c->s,
+               bf16_terms<R>(c), E.rotw, E.rotw_slots);
   });
 }
 
@@ -202,8 +206,7 @@ template <typename R> int davidson_chunk(derek_ctx* c, int k0, int nkc, int nit,
   } else {
     c->timed(KC_DENSE, 0, 0, [&] { rr_solve(E.dw, H, nb, nkc, eps, U, s); });
   }
-  rot<R>(c, Y, U, nb, nb, (int64_t)nb * nb, k0, nkc, Y2);
-  rot<R>(c, HY, U, nb, nb, (int64_t)nb * nb, k0, nkc, HY2);
+  rot<R>(c, Y, HY, U, nb, nb, (int64_t)nb * nb, k0, nkc, Y2, HY2);
   std::swap(Y, Y2);
   std::swap(HY, HY2);
   ++swaps;
@@ -237,8 +240,7 @@ template <typename R> int davidson_chunk(derek_ctx* c, int k0, int nkc, int nit,
       c->timed(KC_OTHER, 0, 0, [&] { subspace_blocks(S, H, eps, m2, nb, nkc, s); });
     }
     c->timed(KC_DENSE, 0, 0, [&] { gen_solve(E.dw, S, H, m2, nb, nkc, drop, eps, U, s); });
-    rot<R>(c, Y, U, m2, nb, (int64_t)m2 * nb, k0, nkc, Y2);
-    rot<R>(c, HY, U, m2, nb, (int64_t)m2 * nb, k0, nkc, HY2);
+    rot<R>(c, Y, HY, U, m2, nb, (int64_t)m2 * nb, k0, nkc, Y2, HY2);
     std::swap(Y, Y2);
     std::swap(HY, HY2);
     ++swaps;
@@ -510,10 +512,12 @@ template <typename R> void autotune(derek_ctx* c) {
       return tb;
     };
     float bestg = time_ov();
-    // tile edge first (BF16 overlaps only), then the rounds at that edge
-    if (bf16_terms<R>(c) > 0) {
+    // tile edge first (BF16 overlaps only), then the rounds at that edge; an
+    // edge left to the size stays so for two terms, whose large overlaps have
+    // a kernel of their own
+    if (bf16_terms<R>(c) > 0 && (c->ov_tile || bf16_terms<R>(c) != 2)) {
       const int t0 = c->ov_tile;
-      c->ov_tile = t0 == 64 ? 128 : 64;
+      c->ov_tile = t0 == 128 ? 64 : 128;
       const float t = time_ov();
       if (t < kGain * bestg) bestg = t;
       else c->ov_tile = t0;
@@ -592,6 +596,10 @@ void scf_init(derek_ctx* c, const derek_scf_params& p) {
   // 2nb x 2nb, for full batches and the last, shorter one
   E.ovw_cap = engine_overlap_work_elems(nb, nk, E.kc, c->max_npw);
   E.ovw = E.alloc<double2>(E.ovw_cap);
+  if (E.fp32) {
+    E.rotw_slots = rotate_work_slots(E.m2, nb, E.kc);
+    E.rotw = E.alloc<double2>(E.rotw_slots);
+  }
   for (double** q : {&E.eps, &E.ekin, &E.rn, &E.occ, &E.occw}) *q = E.alloc<double>((size_t)nk * nb);
   E.stats_partial = E.alloc<double>((size_t)E.kc * nb * band_stats_chunks(c->max_npw) * 2);
   for (double** q : {&E.rho_in, &E.rho_out, &E.vh, &E.vxc, &E.vhxc, &E.tmp1, &E.tmp2}) *q = E.alloc<double>(c->N);
@@ -632,7 +640,7 @@ void scf_init(derek_ctx* c, const derek_scf_params& p) {
       c->sync();
       for (int v : ok)
         if (!v) throw NumericError("initial wavefunctions are linearly dependent");
-      rot<R>(c, Yk, U, nb, nb, (int64_t)nb * nb, k0, nkc, Y2k);
+      rot<R>(c, Yk, nullptr, U, nb, nb, (int64_t)nb * nb, k0, nkc, Y2k, nullptr);
       const size_t pitch = (size_t)E.kstride * sizeof(C);
       DEREK_HIP(hipMemcpy2DAsync(Yk, pitch, Y2k, pitch, (size_t)nb * E.ldk * sizeof(C), nkc, hipMemcpyDeviceToDevice,
                                  c->s));
