@@ -177,7 +177,7 @@ void derek_ctx::apply_h(int k0, int nkc, PwBlock<R> psi, PwBlock<R> hpsi, int nb
   const int64_t nyz = (int64_t)dims[1] * dims[2];
   const bool fz = use_slab<R>(kFusedHpsi);
   for_item_launches(this, k0, nkc, nbands, [&](int ka, int kk, int kn, int b0, int nbb) {
-    PwBatch B{d_maps, ka, kn, nbb, nst_max, nax_max, zsl};
+    PwBatch B{d_maps, ka, kn, nbb, nst_max, nax_max, zsl, quarter};
     cx_t<R>* S = sticks<R>(kn * nbb);
     double npw = 0, nst = 0, nax = 0;
     for (int k = ka; k < ka + kn; ++k) {
@@ -218,7 +218,7 @@ void derek_ctx::density(int k0, int nkc, PwBlock<R> psi, int nbands, const doubl
   const bool fz = use_slab<R>(kFusedDensity);
   bool first = true;
   for_item_launches(this, k0, nkc, nbands, [&](int ka, int kk, int kn, int b0, int nbb) {
-    PwBatch B{d_maps, ka, kn, nbb, nst_max, nax_max, zsl};
+    PwBatch B{d_maps, ka, kn, nbb, nst_max, nax_max, zsl, quarter};
     cx_t<R>* S = sticks<R>(kn * nbb);
     double npw = 0, nst = 0, nax = 0;
     for (int k = ka; k < ka + kn; ++k) {
@@ -660,6 +660,7 @@ int32_t derek_hip_set_basis(derek_ctx* c, int32_t k, int64_t npw, const int32_t*
     K.maps.npw = h.npw;
     K.maps.nst = h.nst;
     K.maps.nax = h.nax;
+    K.quarter = h.quarter;
     K.maps.perm = q;
     q += npw;
     K.maps.pw_z = q;
@@ -684,8 +685,10 @@ int32_t derek_hip_set_basis(derek_ctx* c, int32_t k, int64_t npw, const int32_t*
     DEREK_HIP(hipMemcpy(c->d_wk + k, &weight, sizeof(double), hipMemcpyHostToDevice));
     c->nst_max = 0;
     c->nax_max = 0;
+    c->quarter = true;
     for (const KState& s : c->ks)
       if (s.set) {
+        c->quarter = c->quarter && s.quarter;
         c->nst_max = std::max(c->nst_max, s.maps.nst);
         c->nax_max = std::max(c->nax_max, s.maps.nax);
       }

@@ -108,6 +108,7 @@ struct KState {
   double* kin = nullptr;
   double weight = 0.0;
   bool set = false;
+  bool quarter = false;         // plane waves in the grid's outer quarters (PwBatch::quarter)
   PwMaps maps;                  // sphere maps (device pointers into mapbuf)
   int32_t* mapbuf = nullptr;
 };
@@ -136,6 +137,7 @@ struct derek_ctx {
   derek::PwMaps* d_maps = nullptr;  // device table of every k-point's maps
   int* d_npw = nullptr;             // [nk]
   double* d_wk = nullptr;           // [nk] k-point weights
+  bool quarter = false;             // KState::quarter of every k-point
   int nst_max = 0, nax_max = 0;     // largest stick count (rounded up to 16) / plane count over the k-points
   double* gsq = nullptr;
   double* vext = nullptr;

@@ -13,6 +13,21 @@
 // many threads the workgroup has.  Forward transforms after an inverse one run
 // the stages backwards (decimation in frequency).
 //
+// Q: the plane waves lie in the outer quarters of every axis (PwBatch::quarter,
+// true for a sphere on a grid at least twice as fine as it needs).  The
+// inverse transforms then take literal zeros for the digits that cannot hold
+// input (this file and pw_fft.hip are compiled without signed zeros, so the
+// additions fold away) and the forward ones drop the outputs that nobody
+// reads: about a sixth of the arithmetic and half of the first loads and last
+// stores, with the same values.  Measured together with the coprime register
+// transforms (fft.hpp): the fused y/x pass on 144^3 complex64 2466 -> 2121 us,
+// on 108^3 complex128 617 -> 543, on 72^3 complex64 324 -> 299; the x pass of
+// 256 bands on 65^3 complex128 393 -> 352 us.
+// The z passes bring each stick row once and wait for HBM (70 to 80 % of their
+// cycles), so lengths in the code gain nothing over lengths as arguments:
+// 72^3 complex64 43 and 47 us (inverse, forward) against 50 and 50 with
+// compiled lengths, 144^3 418 and 552 against 428 and 534.
+//
 // Bound: HBM for the y and z passes, the vector ALU for the x pass in FP64.
 // The Stockham kernels these replace (ping-pong LDS, one division per element,
 // two or three passes over LDS per stage) took 2340 us for the x pass of 256
@@ -40,7 +55,7 @@ __device__ __forceinline__ void slot_table(int* slot, TwoStage q, int pitch) {
   for (int z = threadIdx.x; z < q.n; z += AT) slot[z] = ((z % q.r1) * q.r2 + z / q.r1) * pitch;
 }
 
-template <int SGN, int SL, typename C>
+template <int SGN, int SL, bool Q, typename C>
 __device__ __forceinline__ void any_z_stages(C* buf, const C* twl, TwoStage q, int pitch) {
   with_radix(q.r1, [&](auto rc) {
     constexpr int R1 = decltype(rc)::value;
@@ -50,7 +65,7 @@ __device__ __forceinline__ void any_z_stages(C* buf, const C* twl, TwoStage q, i
       C* p = buf + j * pitch + l;
       C v[R1];
 #pragma unroll
-      for (int r = 0; r < R1; ++r) v[r] = p[r * step];
+      for (int r = 0; r < R1; ++r) v[r] = (!Q || SGN < 0 || quarter_has(r, R1)) ? p[r * step] : cmk<C>(0, 0);
       dftR<R1, SGN>(v, (const C*)nullptr, 0);
 #pragma unroll
       for (int r = 0; r < R1; ++r) p[r * step] = v[r];
@@ -67,14 +82,15 @@ __device__ __forceinline__ void any_z_stages(C* buf, const C* twl, TwoStage q, i
       for (int r = 0; r < R2; ++r) u[r] = r ? cmul(p[r * pitch], twid<SGN>(twl, k * r)) : p[0];
       dftR<R2, SGN>(u, (const C*)nullptr, 0);
 #pragma unroll
-      for (int r = 0; r < R2; ++r) p[r * pitch] = u[r];
+      for (int r = 0; r < R2; ++r)
+        if (!Q || SGN > 0 || quarter_has(r, R2)) p[r * pitch] = u[r];
     }
   });
   __syncthreads();
 }
 
 // psi[b][perm[p]] -> S
-template <typename R, bool ZM, int SL>
+template <typename R, bool ZM, int SL, bool Q>
 __global__ __launch_bounds__(AT) void k_any_z_inv(PwBatch B, PwBlock<R> psi, TwoStage q, const cx_t<R>* __restrict__ tw,
                                                   cx_t<R>* __restrict__ S) {
   using C = cx_t<R>;
@@ -90,13 +106,16 @@ __global__ __launch_bounds__(AT) void k_any_z_inv(PwBatch B, PwBlock<R> psi, Two
   const int lines = min(SL, m.nst - s0);
   for (int t = tid; t < n; t += AT) twl[t] = tw[t];
   slot_table(slot, q, pitch);
-  for (int e = tid; e < n * pitch; e += AT) buf[e] = cmk<C>(0, 0);
+  // the inputs that stage 1 reads: all, or the digits of the outer quarters
+  const int lo = Q ? (q.r1 + 3) / 4 * q.r2 : n, hi = Q ? max(lo, 3 * q.r1 / 4 * q.r2) : n;
+  for (int e = tid; e < lo * pitch; e += AT) buf[e] = cmk<C>(0, 0);
+  for (int e = hi * pitch + tid; e < n * pitch; e += AT) buf[e] = cmk<C>(0, 0);
   __syncthreads();
   const int p0 = m.st_pw[s0], p1 = m.st_pw[s0 + lines];
   const C* pb = psi.p + blockIdx.z * psi.ks + (int64_t)band * psi.ld;
   for (int p = p0 + tid; p < p1; p += AT) buf[m.pw_z[p] * pitch + (m.pw_st[p] - s0)] = pb[m.perm[p]];
   __syncthreads();
-  any_z_stages<+1, SL>(buf, twl, q, pitch);
+  any_z_stages<+1, SL, Q>(buf, twl, q, pitch);
   const int64_t item = (int64_t)blockIdx.z * B.nbb + band;
   if constexpr (ZM) {
     const int l = tid % SL;
@@ -111,7 +130,7 @@ __global__ __launch_bounds__(AT) void k_any_z_inv(PwBatch B, PwBlock<R> psi, Two
 }
 
 // hpsi[b][perm[p]] = (z FFT of the stick)[pw_z[p]] + kin[perm[p]] psi[b][perm[p]]
-template <typename R, bool ZM, int SL>
+template <typename R, bool ZM, int SL, bool Q>
 __global__ __launch_bounds__(AT) void k_any_z_fwd(PwBatch B, const cx_t<R>* __restrict__ S, TwoStage q,
                                                   const cx_t<R>* __restrict__ tw, PwBlock<R> psi, PwBlock<R> hpsi) {
   using C = cx_t<R>;
@@ -140,7 +159,7 @@ __global__ __launch_bounds__(AT) void k_any_z_fwd(PwBatch B, const cx_t<R>* __re
         buf[z * pitch + l] = l < lines ? nt_load(src + (int64_t)l * n + z) : cmk<C>(0, 0);
   }
   __syncthreads();
-  any_z_stages<-1, SL>(buf, twl, q, pitch);
+  any_z_stages<-1, SL, Q>(buf, twl, q, pitch);
   const int p0 = m.st_pw[s0], p1 = m.st_pw[s0 + lines];
   const C* pb = psi.p + blockIdx.z * psi.ks + (int64_t)band * psi.ld;
   C* hb = hpsi.p + blockIdx.z * hpsi.ks + (int64_t)band * hpsi.ld;
@@ -167,7 +186,7 @@ __device__ __forceinline__ void column_tables(C* twl, uint32_t* row, const C* __
 
 // stage 1 of an inverse or forward transform: rows from a buffer resource
 // (row[i]: byte offset of index i) into slots
-template <int SGN, typename C, int CP, typename Rs>
+template <int SGN, bool Q, typename C, int CP, typename Rs>
 __device__ __forceinline__ void column_in(C* buf, const uint32_t* row, TwoStage q, const Rs& rs, int cols) {
   with_radix(q.r1, [&](auto rc) {
     constexpr int R1 = decltype(rc)::value;
@@ -176,7 +195,8 @@ __device__ __forceinline__ void column_in(C* buf, const uint32_t* row, TwoStage 
       const uint32_t lo = l < cols ? (uint32_t)l * (uint32_t)sizeof(C) : kOob;
       C v[R1];
 #pragma unroll
-      for (int r = 0; r < R1; ++r) v[r] = buf_ld<C, CP>(rs, row[j + q.r2 * r] + lo);
+      for (int r = 0; r < R1; ++r)
+        v[r] = (!Q || quarter_has(r, R1)) ? buf_ld<C, CP>(rs, row[j + q.r2 * r] + lo) : cmk<C>(0, 0);
       dftR<R1, SGN>(v, (const C*)nullptr, 0);
       C* p = buf + j * AL + l;
 #pragma unroll
@@ -204,7 +224,7 @@ __device__ __forceinline__ void column_out(const C* buf, const C* twl, TwoStage 
 }
 
 // y pass: SGN +1 sticks of plane a -> y rows of P, -1 y rows -> sticks
-template <typename R, int SGN>
+template <typename R, int SGN, bool Q>
 __global__ __launch_bounds__(AT) void k_any_y(PwBatch B, cx_t<R>* __restrict__ S, cx_t<R>* __restrict__ P, int nz,
                                               int ztiles, int bpw, TwoStage q, const cx_t<R>* __restrict__ tw) {
   using C = cx_t<R>;
@@ -233,21 +253,22 @@ __global__ __launch_bounds__(AT) void k_any_y(PwBatch B, cx_t<R>* __restrict__ S
     const int64_t item = (int64_t)blockIdx.z * B.nbb + band;
     const auto rst = buf_rsrc(S + item * B.nst_cap * nz + z0, st_bytes);
     const auto rpl = buf_rsrc(P + (item * B.nax_cap + a) * n * nz + z0, pl_bytes);
-    column_in<SGN, C, 0>(buf, in, q, SGN > 0 ? rst : rpl, cols);
+    column_in<SGN, Q && (SGN > 0), C, 0>(buf, in, q, SGN > 0 ? rst : rpl, cols);
     __syncthreads();
     const auto ro = SGN > 0 ? rpl : rst;
     column_out<SGN>(buf, twl, q, [&](auto rc, int k, int l, const C* u) {
       constexpr int R2 = decltype(rc)::value;
       const uint32_t lo = l < cols ? (uint32_t)l * (uint32_t)sizeof(C) : kOob;
 #pragma unroll
-      for (int i = 0; i < R2; ++i) buf_st<C>(ro, out[k + q.r1 * i] + lo, u[i]);
+      for (int i = 0; i < R2; ++i)
+        if (!Q || SGN > 0 || quarter_has(i, R2)) buf_st<C>(ro, out[k + q.r1 * i] + lo, u[i]);
     });
     __syncthreads();
   }
 }
 
 // x pass: inverse of the active rows, * V * vscale, forward, active rows back
-template <typename R>
+template <typename R, bool Q>
 __global__ __launch_bounds__(AT) void k_any_x_vmul(PwBatch B, cx_t<R>* __restrict__ P, int64_t nyz, int bpw, TwoStage q,
                                                    const cx_t<R>* __restrict__ tw, const R* __restrict__ vloc,
                                                    R vscale) {
@@ -273,7 +294,7 @@ __global__ __launch_bounds__(AT) void k_any_x_vmul(PwBatch B, cx_t<R>* __restric
   const int bb0 = blockIdx.y * bpw, bb1 = min(B.nbb, bb0 + bpw);
   for (int band = bb0; band < bb1; ++band) {
     const auto rs = buf_rsrc(P + ((int64_t)blockIdx.z * B.nbb + band) * B.nax_cap * nyz + c0, bytes);
-    column_in<+1, C, kNt>(buf, row, q, rs, cols);
+    column_in<+1, Q, C, kNt>(buf, row, q, rs, cols);
     __syncthreads();
     column_out<+1>(buf, twl, q, [&](auto rc, int k, int l, C* u) {
       constexpr int R2 = decltype(rc)::value;
@@ -298,7 +319,8 @@ __global__ __launch_bounds__(AT) void k_any_x_vmul(PwBatch B, cx_t<R>* __restric
         for (int r = 0; r < R1; ++r) v[r] = p[r * q.r2 * AL];
         dftR<R1, -1>(v, (const C*)nullptr, 0);
 #pragma unroll
-        for (int r = 0; r < R1; ++r) buf_st<C, kNt>(rs, row[j + q.r2 * r] + lo, v[r]);
+        for (int r = 0; r < R1; ++r)
+          if (!Q || quarter_has(r, R1)) buf_st<C, kNt>(rs, row[j + q.r2 * r] + lo, v[r]);
       }
     });
     __syncthreads();
@@ -306,7 +328,7 @@ __global__ __launch_bounds__(AT) void k_any_x_vmul(PwBatch B, cx_t<R>* __restric
 }
 
 // x pass for the density: rho[x*nyz + c] = keep*rho + sum_items occ |inverse x|^2
-template <typename R>
+template <typename R, bool Q>
 __global__ __launch_bounds__(AT) void k_any_x_density(PwBatch B, const cx_t<R>* __restrict__ P, int64_t nyz, TwoStage q,
                                                       const cx_t<R>* __restrict__ tw, const double* __restrict__ occ,
                                                       int occ_ks, double* __restrict__ rho, int keep) {
@@ -332,7 +354,7 @@ __global__ __launch_bounds__(AT) void k_any_x_density(PwBatch B, const cx_t<R>* 
       const double w = occ[(int64_t)kz * occ_ks + band];
       if (w == 0.0) continue;  // uniform over the workgroup
       const auto rs = buf_rsrc(P + ((int64_t)kz * B.nbb + band) * B.nax_cap * nyz + c0, bytes);
-      column_in<+1, C, 0>(buf, row, q, rs, cols);
+      column_in<+1, Q, C, 0>(buf, row, q, rs, cols);
       __syncthreads();
       column_out<+1>(buf, twl, q, [&](auto rc, int k, int l, const C* u) {
         constexpr int R2 = decltype(rc)::value;
@@ -389,7 +411,7 @@ template <typename R, bool ZM, int SL>
 bool z_inv_sl(const PwBatch& B, PwBlock<R> psi, const Axis<R>& az, cx_t<R>* S, TwoStage q, hipStream_t s) {
   const size_t lds = any_z_lds<R, SL>(q.n, ZM);
   if (lds > kLdsMax) return false;
-  auto kern = k_any_z_inv<R, ZM, SL>;
+  auto kern = B.quarter ? k_any_z_inv<R, ZM, SL, true> : k_any_z_inv<R, ZM, SL, false>;
   allow_lds_any(kern, lds);
   hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(B.nst_cap, SL), B.nbb, B.nkc), dim3(AT), lds, s, B, psi, q, az.tw, S);
   return true;
@@ -400,7 +422,7 @@ bool z_fwd_sl(const PwBatch& B, const cx_t<R>* S, const Axis<R>& az, PwBlock<R> 
               hipStream_t s) {
   const size_t lds = any_z_lds<R, SL>(q.n, ZM);
   if (lds > kLdsMax) return false;
-  auto kern = k_any_z_fwd<R, ZM, SL>;
+  auto kern = B.quarter ? k_any_z_fwd<R, ZM, SL, true> : k_any_z_fwd<R, ZM, SL, false>;
   allow_lds_any(kern, lds);
   hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(B.nst_cap, SL), B.nbb, B.nkc), dim3(AT), lds, s, B, S, q, az.tw, psi,
                      hpsi);
@@ -438,7 +460,8 @@ bool any_y(const PwBatch& B, cx_t<R>* S, cx_t<R>* P, const Axis<R>& ay, int nz, 
   if (!q.r1 || lds > kLdsMax) return false;
   const int ztiles = (int)ceil_div(nz, AL);
   dim3 grid((unsigned)(B.nax_cap * ztiles), (unsigned)ceil_div(B.nbb, bands_per_wg), B.nkc);
-  auto kern = sign > 0 ? k_any_y<R, +1> : k_any_y<R, -1>;
+  auto kern = sign > 0 ? (B.quarter ? k_any_y<R, +1, true> : k_any_y<R, +1, false>)
+                       : (B.quarter ? k_any_y<R, -1, true> : k_any_y<R, -1, false>);
   allow_lds_any(kern, lds);
   hipLaunchKernelGGL(kern, grid, dim3(column_threads(q)), lds, s, B, S, P, nz, ztiles, bands_per_wg, q, ay.tw);
   return true;
@@ -452,7 +475,7 @@ bool any_x_vmul(const PwBatch& B, cx_t<R>* P, const Axis<R>& ax, int64_t nyz, co
       (sizeof(cx_t<R>) * (AL + 1) + sizeof(R) * AL + sizeof(uint32_t)) * (size_t)q.n;
   if (!q.r1 || lds > kLdsMax) return false;
   dim3 grid((unsigned)ceil_div(nyz, AL), (unsigned)ceil_div(B.nbb, bands_per_wg), B.nkc);
-  auto kern = k_any_x_vmul<R>;
+  auto kern = B.quarter ? k_any_x_vmul<R, true> : k_any_x_vmul<R, false>;
   allow_lds_any(kern, lds);
   hipLaunchKernelGGL(kern, grid, dim3(column_threads(q)), lds, s, B, P, nyz, bands_per_wg, q, ax.tw, vloc, vscale);
   return true;
@@ -464,7 +487,7 @@ bool any_x_density(const PwBatch& B, const cx_t<R>* P, const Axis<R>& ax, int64_
   const TwoStage q = two_stage(ax.n);
   const size_t lds = (sizeof(cx_t<R>) * (AL + 1) + sizeof(double) * AL + sizeof(uint32_t)) * (size_t)q.n;
   if (!q.r1 || lds > kLdsMax) return false;
-  auto kern = k_any_x_density<R>;
+  auto kern = B.quarter ? k_any_x_density<R, true> : k_any_x_density<R, false>;
   allow_lds_any(kern, lds);
   hipLaunchKernelGGL(kern, dim3((unsigned)ceil_div(nyz, AL)), dim3(column_threads(q)), lds, s, B, P, nyz, q, ax.tw, occ,
                      occ_ks, rho, keep);

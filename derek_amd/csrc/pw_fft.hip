@@ -646,68 +646,6 @@ __global__ __launch_bounds__(Split<N>::NT) void k_py_fwd2(PwBatch B, const cx_t<
   }
 }
 
-// z passes on sticks for the two-stage lengths: SL sticks per workgroup,
-// TPL = max(R1, R2) threads per stick; the sticks are padded lines of one
-// LDS buffer (the plane-wave scatter / gather needs them there anyway), the
-// two DFT stages run in registers with one transpose through that buffer.
-// SL sticks per workgroup, 16 (FP64) or 32 (FP32): with the stick capacity
-// a multiple of 16, every workgroup's segment of a z-major row is two whole
-// 128-byte lines, so no line is written by two workgroups.  (32 FP64 sticks
-// need 57 KB of LDS at N = 108 and cut the z passes to two workgroups per
-// CU, which was slower.)
-template <int N, int SL_> struct StickSplit {
-  static constexpr int R1 = Split<N>::R1, R2 = Split<N>::R2;
-  static constexpr int TPL = R1 > R2 ? R1 : R2;
-  static constexpr int SL = SL_;       // sticks per workgroup
-  static constexpr int NT = SL * TPL;
-  // intermediate pitch between the stages: sub-transform j's outputs start
-  // at slot j (R1 + 1), so the lanes' stage-1 stores stride by an odd count
-  // (a stride of R1 = 12 complex128 is 48 dwords: lanes j and j + 4 would
-  // share banks)
-  static constexpr int IP = R1 + 1;
-  // padded line pitch (odd), room for the padded intermediate
-  static constexpr int LS = ((N + 1 > R2 * IP ? N + 1 : R2 * IP)) | 1;
-  static constexpr size_t lds(size_t csize) { return csize * ((size_t)N + (size_t)SL * LS); }
-};
-
-// sticks per workgroup of a batch: its choice, or 16 (FP64) / 32 (FP32)
-template <typename R> int stick_block(const PwBatch& B) { return B.zsl ? B.zsl : (sizeof(R) == 8 ? 16 : 32); }
-
-// S1 + S2 of one transform on a padded LDS line, in place; thread (line, j)
-// with j < TPL, `act` false for lines past the block's last stick
-template <int SGN, typename C, int N>
-__device__ __forceinline__ void stick_two_stage(C* line, const C* twl, int j, bool act) {
-  using SS = StickSplit<N, 1>;
-  constexpr int R1 = SS::R1, R2 = SS::R2, IP = SS::IP;
-  C v[R1];
-  if (act && j < R2) {
-#pragma unroll
-    for (int r = 0; r < R1; ++r) v[r] = line[j + R2 * r];
-    dftR<R1, SGN>(v, twl, N);
-  }
-  __syncthreads();
-  if (act && j < R2) {
-#pragma unroll
-    for (int k = 0; k < R1; ++k) line[j * IP + k] = v[k];
-  }
-  __syncthreads();
-  C u[R2];
-  if (act && j < R1) {
-#pragma unroll
-    for (int r = 0; r < R2; ++r) {
-      const C y = line[r * IP + j];
-      u[r] = r ? cmul(y, SGN > 0 ? cconj(twl[(j * r) % N]) : twl[(j * r) % N]) : y;
-    }
-    dftR<R2, SGN>(u, twl, N);
-  }
-  __syncthreads();
-  if (act && j < R1) {
-#pragma unroll
-    for (int k = 0; k < R2; ++k) line[j + R1 * k] = u[k];
-  }
-  __syncthreads();
-}
-
 // (major, minor) task of a workgroup of a (gridDim.x majors x gridDim.y
 // minors) grid, for workgroups that share data through their major index
 // (the complex128 fused pass: the V rows of a z plane).  The dispatcher deals
@@ -725,92 +663,6 @@ __device__ __forceinline__ void xcd_task(int& major, int& minor) {
   const int t = x * (T / 8) + min(x, T % 8) + s;
   major = t / (int)gridDim.y;
   minor = t % (int)gridDim.y;
-}
-
-// psi[b][perm[p]] -> S[item][s][:] for the block's sticks
-template <typename R, int N, bool ZM, int SL_>
-__global__ __launch_bounds__((StickSplit<N, SL_>::NT)) void k_sticks_z_inv2(PwBatch B, PwBlock<R> psi,
-                                                                     const cx_t<R>* __restrict__ tw,
-                                                                     cx_t<R>* __restrict__ S) {
-  using C = cx_t<R>;
-  using SS = StickSplit<N, SL_>;
-  constexpr int NT = SS::NT, SL = SS::SL, LS = SS::LS, TPL = SS::TPL;
-  extern __shared__ __align__(16) unsigned char smem[];
-  const PwMaps m = B.mt[B.k0 + blockIdx.z];
-  const int s0 = blockIdx.x * SL;
-  if (s0 >= m.nst) return;
-  C* twl = reinterpret_cast<C*>(smem);
-  C* buf = twl + N;
-  const int lines = min(SL, m.nst - s0);
-  const int band = blockIdx.y;
-  for (int t = threadIdx.x; t < N; t += NT) twl[t] = tw[t];
-  for (int e = threadIdx.x; e < lines * LS; e += NT) buf[e] = cmk<C>(0, 0);
-  __syncthreads();
-  const int p0 = m.st_pw[s0], p1 = m.st_pw[s0 + lines];
-  const C* pb = psi.p + blockIdx.z * psi.ks + (int64_t)band * psi.ld;
-  for (int p = p0 + threadIdx.x; p < p1; p += NT) buf[(m.pw_st[p] - s0) * LS + m.pw_z[p]] = pb[m.perm[p]];
-  __syncthreads();
-  const int line = threadIdx.x / TPL, j = threadIdx.x % TPL;
-  stick_two_stage<+1, C, N>(buf + line * LS, twl, j, line < lines);
-  if constexpr (ZM) {
-    // z-major sticks: row z of the item holds every stick at that z
-    C* dst = S + ((int64_t)blockIdx.z * B.nbb + band) * B.nst_cap * N + s0;
-    for (int e = threadIdx.x; e < lines * N; e += NT) {
-      const int z = e / lines, q = e - z * lines;
-      nt_store(dst + (int64_t)z * B.nst_cap + q, buf[q * LS + z]);
-    }
-  } else {
-    C* dst = S + (((int64_t)blockIdx.z * B.nbb + band) * B.nst_cap + s0) * N;
-    for (int e = threadIdx.x; e < lines * N; e += NT) {
-      const int q = e / N;
-      nt_store(dst + e, buf[q * LS + (e - q * N)]);
-    }
-  }
-}
-
-// hpsi[b][perm[p]] = (z FFT of the stick)[pw_z[p]] + kin[perm[p]] psi[b][perm[p]]
-template <typename R, int N, bool ZM, int SL_>
-__global__ __launch_bounds__((StickSplit<N, SL_>::NT)) void k_sticks_z_fwd2(PwBatch B, const cx_t<R>* __restrict__ S,
-                                                                     const cx_t<R>* __restrict__ tw, PwBlock<R> psi,
-                                                                     PwBlock<R> hpsi) {
-  using C = cx_t<R>;
-  using SS = StickSplit<N, SL_>;
-  constexpr int NT = SS::NT, SL = SS::SL, LS = SS::LS, TPL = SS::TPL;
-  extern __shared__ __align__(16) unsigned char smem[];
-  const PwMaps m = B.mt[B.k0 + blockIdx.z];
-  const int s0 = blockIdx.x * SL;
-  if (s0 >= m.nst) return;
-  C* twl = reinterpret_cast<C*>(smem);
-  C* buf = twl + N;
-  const int lines = min(SL, m.nst - s0);
-  const int band = blockIdx.y;
-  for (int t = threadIdx.x; t < N; t += NT) twl[t] = tw[t];
-  if constexpr (ZM) {
-    const C* src = S + ((int64_t)blockIdx.z * B.nbb + band) * B.nst_cap * N + s0;
-    for (int e = threadIdx.x; e < lines * N; e += NT) {
-      const int z = e / lines, q = e - z * lines;
-      buf[q * LS + z] = nt_load(src + (int64_t)z * B.nst_cap + q);
-    }
-  } else {
-    const C* src = S + (((int64_t)blockIdx.z * B.nbb + band) * B.nst_cap + s0) * N;
-    for (int e = threadIdx.x; e < lines * N; e += NT) {
-      const int q = e / N;
-      buf[q * LS + (e - q * N)] = nt_load(src + e);
-    }
-  }
-  __syncthreads();
-  const int line = threadIdx.x / TPL, j = threadIdx.x % TPL;
-  stick_two_stage<-1, C, N>(buf + line * LS, twl, j, line < lines);
-  const int p0 = m.st_pw[s0], p1 = m.st_pw[s0 + lines];
-  const C* pb = psi.p + blockIdx.z * psi.ks + (int64_t)band * psi.ld;
-  C* hb = hpsi.p + blockIdx.z * hpsi.ks + (int64_t)band * hpsi.ld;
-  for (int p = p0 + threadIdx.x; p < p1; p += NT) {
-    const int g = m.perm[p];
-    const C v = buf[(m.pw_st[p] - s0) * LS + m.pw_z[p]];
-    const C x = pb[g];
-    const R t = (R)m.kin[g];
-    hb[g] = cmk<C>(v.x + t * x.x, v.y + t * x.y);
-  }
 }
 
 // ---------------------------------------------------------------- launchers
@@ -835,55 +687,10 @@ template <typename R> static void check_offsets(const PwBatch& B, int64_t nyz, i
                 "one item's sticks or planes exceed 2 GiB");
 }
 
-template <typename R, int N, int SL>
-static void sticks_z_inv2_sl(const PwBatch& B, PwBlock<R> psi, const Axis<R>* ax, cx_t<R>* S, bool zmajor,
-                             hipStream_t s) {
-  using SS = StickSplit<N, SL>;
-  const size_t lds = SS::lds(sizeof(cx_t<R>));
-  check_lds_pw(lds, N);
-  auto kern = zmajor ? k_sticks_z_inv2<R, N, true, SL> : k_sticks_z_inv2<R, N, false, SL>;
-  allow_lds_pw(kern, lds);
-  dim3 grid((unsigned)ceil_div(B.nst_cap, SS::SL), B.nbb, B.nkc);
-  hipLaunchKernelGGL(kern, grid, dim3(SS::NT), lds, s, B, psi, ax[2].tw, S);
-}
-
-template <typename R, int N, int SL>
-static void sticks_z_fwd2_sl(const PwBatch& B, const cx_t<R>* S, const Axis<R>* ax, PwBlock<R> psi, PwBlock<R> hpsi,
-                             bool zmajor, hipStream_t s) {
-  using SS = StickSplit<N, SL>;
-  const size_t lds = SS::lds(sizeof(cx_t<R>));
-  check_lds_pw(lds, N);
-  auto kern = zmajor ? k_sticks_z_fwd2<R, N, true, SL> : k_sticks_z_fwd2<R, N, false, SL>;
-  allow_lds_pw(kern, lds);
-  dim3 grid((unsigned)ceil_div(B.nst_cap, SS::SL), B.nbb, B.nkc);
-  hipLaunchKernelGGL(kern, grid, dim3(SS::NT), lds, s, B, S, ax[2].tw, psi, hpsi);
-}
-
-template <typename R, int N>
-static void sticks_z_inv2(const PwBatch& B, PwBlock<R> psi, const Axis<R>* ax, cx_t<R>* S, bool zmajor,
-                          hipStream_t s) {
-  if (stick_block<R>(B) == 32) sticks_z_inv2_sl<R, N, 32>(B, psi, ax, S, zmajor, s);
-  else sticks_z_inv2_sl<R, N, 16>(B, psi, ax, S, zmajor, s);
-}
-
-template <typename R, int N>
-static void sticks_z_fwd2(const PwBatch& B, const cx_t<R>* S, const Axis<R>* ax, PwBlock<R> psi, PwBlock<R> hpsi,
-                          bool zmajor, hipStream_t s) {
-  if (stick_block<R>(B) == 32) sticks_z_fwd2_sl<R, N, 32>(B, S, ax, psi, hpsi, zmajor, s);
-  else sticks_z_fwd2_sl<R, N, 16>(B, S, ax, psi, hpsi, zmajor, s);
-}
-
 template <typename R>
 void sticks_z_inv(const PwBatch& B, PwBlock<R> psi, const Axis<R>* ax, int nz, cx_t<R>* S, bool zmajor,
                   hipStream_t s) {
   check_batch(B);
-  switch (nz) {
-    case 32: sticks_z_inv2<R, 32>(B, psi, ax, S, zmajor, s); DEREK_HIP(hipGetLastError()); return;
-    case 72: sticks_z_inv2<R, 72>(B, psi, ax, S, zmajor, s); DEREK_HIP(hipGetLastError()); return;
-    case 108: sticks_z_inv2<R, 108>(B, psi, ax, S, zmajor, s); DEREK_HIP(hipGetLastError()); return;
-    case 144: sticks_z_inv2<R, 144>(B, psi, ax, S, zmajor, s); DEREK_HIP(hipGetLastError()); return;
-    default: break;
-  }
   if (any_z_inv<R>(B, psi, ax[2], S, zmajor, s)) {
     DEREK_HIP(hipGetLastError());
     return;
@@ -966,13 +773,6 @@ template <typename R>
 void sticks_z_fwd(const PwBatch& B, const cx_t<R>* S, const Axis<R>* ax, int nz, PwBlock<R> psi, PwBlock<R> hpsi,
                   bool zmajor, hipStream_t s) {
   check_batch(B);
-  switch (nz) {
-    case 32: sticks_z_fwd2<R, 32>(B, S, ax, psi, hpsi, zmajor, s); DEREK_HIP(hipGetLastError()); return;
-    case 72: sticks_z_fwd2<R, 72>(B, S, ax, psi, hpsi, zmajor, s); DEREK_HIP(hipGetLastError()); return;
-    case 108: sticks_z_fwd2<R, 108>(B, S, ax, psi, hpsi, zmajor, s); DEREK_HIP(hipGetLastError()); return;
-    case 144: sticks_z_fwd2<R, 144>(B, S, ax, psi, hpsi, zmajor, s); DEREK_HIP(hipGetLastError()); return;
-    default: break;
-  }
   if (any_z_fwd<R>(B, S, ax[2], psi, hpsi, zmajor, s)) {
     DEREK_HIP(hipGetLastError());
     return;
@@ -1137,7 +937,7 @@ template <typename R, int N, bool VM = false> struct Slab {
 // (j2 in the R2-thread stages, k1 in the R1-thread stages, and its line in
 // each), its twiddles exp(-2 pi i k1 r / N) and the LDS rows of the active
 // planes at x = j2 + R2 r (-1 if none).
-template <typename R, int N, bool VM = false> struct SlabThread {
+template <typename R, int N, bool VM, bool Q> struct SlabThread {
   using C = cx_t<R>;
   using SL = Slab<R, N, VM>;
   static constexpr int R1 = SL::R1, R2 = SL::R2, R2P = SL::R2P, NT = SL::NT, LR = SL::LR;
@@ -1149,6 +949,10 @@ template <typename R, int N, bool VM = false> struct SlabThread {
   int nax, j2, lj, k1, lk;
   C tk[R2];
   int xr[R1];
+
+  // digits of x and y (j2 + R2 r, or k1 + R1 k) that the sphere can reach
+  static constexpr bool in1(int r) { return !Q || quarter_has(r, R1); }
+  static constexpr bool in2(int k) { return !Q || quarter_has(k, R2); }
 
   // LDS tables of the k-point's maps (two barriers)
   __device__ __forceinline__ void init(const PwBatch& B, const PwMaps& m, const C* __restrict__ tw,
@@ -1179,7 +983,7 @@ template <typename R, int N, bool VM = false> struct SlabThread {
   template <typename Rs> __device__ __forceinline__ void load_a1(const Rs& rs, int a, C* v) const {
     const int16_t* ty = sty + a * N + j2;
 #pragma unroll
-    for (int r = 0; r < R1; ++r) v[r] = buf_ld<C>(rs, stick_off(ty[R2 * r]));
+    for (int r = 0; r < R1; ++r) v[r] = in1(r) ? buf_ld<C>(rs, stick_off(ty[R2 * r])) : cmk<C>(0, 0);
   }
   // y inverse of every active plane from a stick row into A (two barriers);
   // with PRE, `pre` holds the first item's inputs
@@ -1218,7 +1022,7 @@ template <typename R, int N, bool VM = false> struct SlabThread {
       const int py = pos(y0 + lj);
       C v[R1];
 #pragma unroll
-      for (int r = 0; r < R1; ++r) v[r] = xr[r] >= 0 ? A[xr[r] + py] : cmk<C>(0, 0);
+      for (int r = 0; r < R1; ++r) v[r] = (in1(r) && xr[r] >= 0) ? A[xr[r] + py] : cmk<C>(0, 0);
       dftR<R1, +1>(v, (const C*)nullptr, N);
       C* row = X + lj * LPX + j2;
 #pragma unroll
@@ -1235,12 +1039,12 @@ template <typename R, int N, bool VM = false> struct SlabThread {
   }
 };
 
-template <typename R, int N>
+template <typename R, int N, bool Q>
 __global__ __launch_bounds__((Slab<R, N, true>::NT)) void k_slab_vmul(PwBatch B, cx_t<R>* __restrict__ S, int nz, int bpw,
                                                               const cx_t<R>* __restrict__ tw,
                                                               const R* __restrict__ vt) {
   using C = cx_t<R>;
-  using ST = SlabThread<R, N, true>;
+  using ST = SlabThread<R, N, true, Q>;
   constexpr int R1 = ST::R1, R2 = ST::R2, LR = ST::LR, NR = Slab<R, N, true>::NR, LJ = ST::LJ, LK = ST::LK;
   constexpr int LPA = ST::LPA, LPX = ST::LPX;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -1304,7 +1108,7 @@ __global__ __launch_bounds__((Slab<R, N, true>::NT)) void k_slab_vmul(PwBatch B,
         dftR<R1, -1>(v, (const C*)nullptr, N);
 #pragma unroll
         for (int k = 0; k < R1; ++k)
-          if (t.xr[k] >= 0) A[t.xr[k] + py] = v[k];
+          if (ST::in1(k) && t.xr[k] >= 0) A[t.xr[k] + py] = v[k];
       }
       __syncthreads();
     }
@@ -1332,7 +1136,8 @@ __global__ __launch_bounds__((Slab<R, N, true>::NT)) void k_slab_vmul(PwBatch B,
       }
       dftR<R2, -1>(u, (const C*)nullptr, N);
 #pragma unroll
-      for (int k = 0; k < R2; ++k) buf_st<C>(rs, ST::stick_off(ty[R1 * k]), u[k]);
+      for (int k = 0; k < R2; ++k)
+        if (ST::in2(k)) buf_st<C>(rs, ST::stick_off(ty[R1 * k]), u[k]);
     }
     __syncthreads();
   }
@@ -1342,13 +1147,13 @@ __global__ __launch_bounds__((Slab<R, N, true>::NT)) void k_slab_vmul(PwBatch B,
 // the y and x inverse transforms as in k_slab_vmul, then
 // part[p][z][y][x] = sum over the group's bands of occ |psi(r)|^2 in FP64
 // (p = k-point slot * groups + group); k_slab_rho_sum adds the partials.
-template <typename R, int N>
+template <typename R, int N, bool Q>
 __global__ __launch_bounds__((Slab<R, N>::NT)) void k_slab_density(PwBatch B, const cx_t<R>* __restrict__ S, int nz,
                                                                  int bpg, const cx_t<R>* __restrict__ tw,
                                                                  const double* __restrict__ occ, int occ_ks,
                                                                  double* __restrict__ part) {
   using C = cx_t<R>;
-  using ST = SlabThread<R, N>;
+  using ST = SlabThread<R, N, false, Q>;
   constexpr int R1 = ST::R1, R2 = ST::R2, LR = ST::LR, NR = Slab<R, N>::NR;
   extern __shared__ __align__(16) unsigned char smem[];
   const PwMaps m = B.mt[B.k0 + blockIdx.z];
@@ -1431,7 +1236,7 @@ template <typename R, int N> static bool slab_fits(int nax_cap) {
 
 template <typename R> bool slab_supported(int nx, int ny, int nz, int nax_cap, int nst_cap) {
   if (nx != ny || nax_cap < 1 || nax_cap > nx || nst_cap > 32767) return false;
-  if (nz != 32 && nz != 72 && nz != 108 && nz != 144) return false;  // z-major stick kernels
+  if (!two_stage(nz).r1) return false;  // z-major stick kernels
   switch (nx) {
     case 32: return slab_fits<R, 32>(nax_cap);
     case 72: return slab_fits<R, 72>(nax_cap);
@@ -1446,7 +1251,7 @@ static void slab_vmul_n(const PwBatch& B, cx_t<R>* S, const Axis<R>* ax, int nz,
   using SL = Slab<R, N, true>;
   const size_t lds = SL::lds(B.nax_cap);
   check_lds_pw(lds, N);
-  auto kern = k_slab_vmul<R, N>;
+  auto kern = B.quarter ? k_slab_vmul<R, N, true> : k_slab_vmul<R, N, false>;
   allow_lds_pw(kern, lds);
   dim3 grid((unsigned)nz, (unsigned)ceil_div(B.nbb, bpw), B.nkc);
   hipLaunchKernelGGL(kern, grid, dim3(SL::NT), lds, s, B, S, nz, bpw, ax[0].tw, vt);
@@ -1464,7 +1269,6 @@ void slab_vmul(const PwBatch& B, cx_t<R>* S, const Axis<R>* ax, int nz, const R*
     case 72: slab_vmul_n<R, 72>(B, S, ax, nz, vt, bpw, s); break;
     case 108: slab_vmul_n<R, 108>(B, S, ax, nz, vt, bpw, s); break;
     case 144: slab_vmul_n<R, 144>(B, S, ax, nz, vt, bpw, s); break;
-    default: throw ArgError("grid not supported by the fused y/x pass");
   }
   DEREK_HIP(hipGetLastError());
 }
@@ -1478,10 +1282,10 @@ template <typename R, int N> static int slab_density_groups_n(const PwBatch& B, 
     return std::max(1, p.multiProcessorCount);
   }();
   const size_t lds = Slab<R, N>::lds(B.nax_cap);
-  allow_lds_pw(k_slab_density<R, N>, lds);
+  auto kern = B.quarter ? k_slab_density<R, N, true> : k_slab_density<R, N, false>;
+  allow_lds_pw(kern, lds);
   int per = 0;
-  DEREK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(k_slab_density<R, N>),
-                                                         Slab<R, N>::NT, lds));
+  DEREK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(kern), Slab<R, N>::NT, lds));
   // about four rounds of resident workgroups
   const int64_t want = 4LL * std::max(1, per) * cus;
   const int64_t g = (want + (int64_t)nz * B.nkc - 1) / ((int64_t)nz * B.nkc);
@@ -1511,7 +1315,7 @@ static void slab_density_n(const PwBatch& B, const cx_t<R>* S, const Axis<R>* ax
   using SL = Slab<R, N>;
   const size_t lds = SL::lds(B.nax_cap);
   check_lds_pw(lds, N);
-  auto kern = k_slab_density<R, N>;
+  auto kern = B.quarter ? k_slab_density<R, N, true> : k_slab_density<R, N, false>;
   allow_lds_pw(kern, lds);
   dim3 grid((unsigned)nz, (unsigned)groups, B.nkc);
   hipLaunchKernelGGL(kern, grid, dim3(SL::NT), lds, s, B, S, nz, (int)ceil_div(B.nbb, groups), ax[0].tw, occ, occ_ks,

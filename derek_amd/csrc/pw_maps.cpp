@@ -9,7 +9,6 @@
 namespace derek {
 
 PwMapsHost build_pw_maps(const int32_t* idx, int64_t npw, int nx, int ny, int nz) {
-  (void)nx;
   PwMapsHost h;
   h.npw = (int)npw;
   std::vector<int32_t> ord(npw);
@@ -29,6 +28,8 @@ PwMapsHost build_pw_maps(const int32_t* idx, int64_t npw, int nx, int ny, int nz
     const int64_t col = f / nz;  // x*ny + y
     const int64_t x = f / nyz;
     h.pw_z[p] = (int32_t)(f % nz);
+    auto outer = [](int64_t b, int64_t n) { return 4 * b < n || 4 * b >= 3 * n; };
+    h.quarter = h.quarter && outer(x, nx) && outer(col % ny, ny) && outer(f % nz, nz);
     if (col != prev_col) {
       if (x != prev_x) {
         h.pl_st.push_back(h.nst);

@@ -31,14 +31,18 @@ struct PwBatch {
   const PwMaps* mt = nullptr;
   int k0 = 0, nkc = 1, nbb = 1;
   int nst_cap = 0, nax_cap = 0;
-  // sticks per workgroup of the compiled z passes (16 or 32; 0: 16 for
+  // sticks per workgroup of the two-stage z passes (16 or 32; 0: 16 for
   // complex128, 32 for complex64)
   int zsl = 0;
+  // every plane wave of every k-point lies in the outer quarters of all three
+  // axes (fft.hpp: quarter_has)
+  bool quarter = false;
 };
 
 // Host construction of the maps from flat FFT-bin indices (z fastest).
 struct PwMapsHost {
   int npw = 0, nst = 0, nax = 0;
+  bool quarter = true;  // all bins b < n/4 or b >= 3n/4 on each axis
   std::vector<int32_t> perm, pw_z, pw_st, st_pw, st_y, pl_st, ax_x, pl_y;
 };
 PwMapsHost build_pw_maps(const int32_t* fft_index, int64_t npw, int nx, int ny, int nz);

@@ -59,3 +59,41 @@ def test_any_length_apply_h_and_density(dims, precision):
             ref = r0 + oks.density([psi], [occ], [weight], [sets[k]], dims, volume)
             assert_close(ctx.density(k, psi, occ, r0), ref, tol, f"density k={k}")
     ctx.close()
+
+
+def outer(n, rng):
+    """Bins of the outer quarters (b < n/4, b >= 3n/4), the edges always among them."""
+    b = np.array([q for q in range(n) if 4 * q < n or 4 * q >= 3 * n])
+    return np.union1d(b[[0, -1, (n + 3) // 4 - 1]], rng.permutation(b)[:max(1, len(b) // 2)])
+
+
+@pytest.mark.parametrize("dims", DIMS[:-1] + [(72, 72, 105), (32, 32, 65), (108, 108, 21), (144, 144, 10)])
+@pytest.mark.parametrize("precision", [lib.DEREK_FP64, lib.DEREK_MIXED])
+@pytest.mark.parametrize("quarter", [True, False])
+def test_outer_quarters(dims, precision, quarter):
+    """Plane waves in the outer quarters of every axis take the transforms with
+    dropped zero inputs and unread outputs, separate and fused; a single bin
+    outside them (quarter False) takes the full ones."""
+    rng = np.random.default_rng(sum(dims) + 1)
+    nx, ny, nz = dims
+    idx = np.concatenate([(x * ny + y) * nz + outer(nz, rng) for x in outer(nx, rng) for y in outer(ny, rng)])
+    if not quarter:
+        idx = np.append(idx, ((nx // 2) * ny + ny // 2) * nz + nz // 2)
+    idx = rng.permutation(np.unique(idx)).astype(np.int32)[:6000]
+    nb, volume, weight = 3, 21.0, 0.9
+    kin = rng.uniform(0.0, 3.0, len(idx))
+    v = rng.normal(size=nx * ny * nz)
+    tol = 1e-12 if precision == lib.DEREK_FP64 else 5e-5
+    ctx = lib.Context(list(dims), 1, nb, volume, len(idx), precision)
+    ctx.set_basis(0, idx, kin, weight)
+    ctx.set_vloc(v)
+    psi = rng.normal(size=(nb, len(idx))) + 1j * rng.normal(size=(nb, len(idx)))
+    occ = np.array([2.0, 1.3, 0.4])
+    ref = oks.apply_h(psi, idx, kin, v, dims)
+    rref = oks.density([psi], [occ], [weight], [idx], dims, volume)
+    for fused in (True, False):
+        print("outer quarters", dims, precision, quarter, "fused", fused, flush=True)
+        ctx.set_launch(bands_per_wg=2, items_per_launch=256, fused=fused)
+        assert_close(ctx.apply_h(0, psi), ref, tol, "H psi")
+        assert_close(ctx.density(0, psi, occ), rref, tol, "density")
+    ctx.close()
