@@ -956,7 +956,9 @@ __global__ __launch_bounds__(IT) void k_inviter(int n, int nev, int cpw, double*
     emax = fmax(emax, ee[i] * ee[i]);
     tnorm = fmax(tnorm, fabs(dd[i]) + 2.0 * ee[i]);
   }
-  const double pivmin = fmax(DBL_MIN * fmax(1.0, emax), 1e-300);
+  // no pivot below 1e-30 |T|: with 1e-300 (the pivot of a decoupled row at its
+  // own eigenvalue) the solution's norm overflowed and the vector came out zero
+  const double pivmin = fmax(fmax(DBL_MIN * fmax(1.0, emax), 1e-300), 1e-30 * tnorm);
   const int t0 = W.cstart[c], t1 = W.cstart[c + 1];
   double prev = -1e300;
   for (int t = t0; t < t1; ++t) {

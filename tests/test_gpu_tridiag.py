@@ -1,0 +1,44 @@
+"""Eigenpairs of matrices whose tridiagonal form splits.
+
+Bounds: Householder reduction, bisection and inverse iteration are backward
+stable, with errors of a few n eps |A|; the bounds are those of the other
+eigenvalue tests (1e-12 n for the values, 1e-11 sqrt(n) for residual and
+orthogonality, relative to the largest eigenvalue).
+"""
+import numpy as np
+import pytest
+
+from derek_amd import lib
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = lib.Context((8, 8, 8), 1, 4, 1.0, 1)
+    yield c
+    c.close()
+
+
+def check(ctx, A):
+    n = len(A)
+    w, Z = ctx.heev(A, n)
+    ref = np.linalg.eigvalsh(A)
+    scale = max(np.abs(ref).max(), 1e-300)
+    assert np.max(np.abs(w - ref)) < 1e-12 * scale * n
+    assert np.max(np.abs(A @ Z - Z * w[None, :])) < 1e-11 * scale * np.sqrt(n)
+    assert np.max(np.abs(Z.conj().T @ Z - np.eye(n))) < 1e-11 * np.sqrt(n)
+
+
+@pytest.mark.parametrize("n,seed", [(18, 3), (47, 0), (65, 6), (95, 5)])
+def test_rows_decoupled_from_the_rest(ctx, n, seed):
+    """A diagonal row whose eigenvalue is met to the last bit: the shifted
+    matrix then has an exactly zero pivot."""
+    rng = np.random.default_rng(n + 1000 * seed)
+    A = rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))
+    A = A + A.conj().T
+    k = n // 3
+    A[k:, :] = A[:, k:] = 0
+    A[np.arange(k, n), np.arange(k, n)] = np.arange(k, n)
+    A[n - 1, 0] = A[0, n - 1] = 0.5
+    check(ctx, A)
