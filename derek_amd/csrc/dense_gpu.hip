@@ -3,10 +3,11 @@
 //
 // k_heev: lowest nev eigenpairs of a Hermitian n x n matrix.
 //   1. Householder reduction to real tridiagonal form: while the trailing
-//      matrix exceeds LDS, one multi-workgroup launch per column on the matrix
-//      in global memory (L2 resident); then the last <= 98 columns in LDS in
-//      one workgroup (lower triangle, look-ahead reflector, two barriers per
-//      column).  The reflectors overwrite the eliminated columns.
+//      matrix exceeds 128 columns, one multi-workgroup launch per column on the
+//      matrix in global memory (L2 resident); then the last 128 columns in the
+//      registers of one workgroup (matrix-core rank-2 updates, look-ahead
+//      reflector, two barriers per column).  The reflectors overwrite the
+//      eliminated columns.
 //   2. Phases that make the sub-diagonal real and non-negative (a prefix
 //      product over the workgroup).
 //   3. Sturm-sequence multisection for the lowest nev eigenvalues, one
@@ -20,6 +21,7 @@
 //   skipping every column whose remaining pivot is below tol (dependent on
 //   earlier columns); many workgroups, one launch per panel of columns.
 #include <cfloat>
+#include <type_traits>
 
 #include "dense_gpu.hpp"
 #include "launch.hpp"
@@ -28,8 +30,6 @@ namespace derek {
 
 constexpr int DT = 1024;  // threads per workgroup
 constexpr int DW = DT / 64;
-// LDS of the matrix-resident tridiagonalisation (gfx950: 160 KiB per workgroup)
-constexpr size_t kTridiagLds = 156 * 1024;
 
 __device__ __forceinline__ double2 zmul(double2 a, double2 b) {
   return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
@@ -255,24 +255,25 @@ int64_t heev_work_doubles(int n, int nev) {
 }
 
 // ---- 1. Householder tridiagonalisation + phases
-// Columns 0 .. n-99 (n > 98) take one multi-workgroup launch each
+// Columns 0 .. n-129 (n > 128) take one multi-workgroup launch each
 // (k_wide_step: the rank-2 update of column k's reflector, fused with the
-// next reflector and u = A v for it); the trailing block of at most 98
-// columns is copied to LDS (lower triangle) and reduced by one workgroup
-// per matrix (k_tridiag).
+// next reflector and u = A v for it); the trailing block of at most 128
+// columns is loaded into registers and reduced by one workgroup per matrix
+// (k_tridiag).
 
 // e = |sub| and the phases ph[0] = 1, ph[k+1] = ph[k] f_k, f_k = sub_k/|sub_k|
 // (1 where sub_k = 0), that make D^H T D real.  The phases are a prefix
-// product of unit complex numbers: each thread takes two consecutive f_k
-// (n <= 2048 = 2 DT), the threads' products are scanned across the lanes of
-// each wavefront and then across the wavefronts (s_wave: DW entries).
+// product of unit complex numbers: each thread takes four consecutive f_k
+// (n <= 2048 = 4 TDT), the threads' products are scanned across the lanes of
+// each wavefront and then across the wavefronts (s_wave: TDT / 64 entries).
+constexpr int TDT = 512;  // threads of k_tridiag
 __device__ void tri_phases(HeevWork& W, int n, double2* s_wave) {
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const double2 one = make_double2(1.0, 0.0);
-  double2 f[2], q = one;
+  double2 f[4], q = one;
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int k = 2 * tid + r;
+  for (int r = 0; r < 4; ++r) {
+    const int k = 4 * tid + r;
     f[r] = one;
     if (k + 1 < n) {
       const double2 sk = W.sub[k];
@@ -294,10 +295,10 @@ __device__ void tri_phases(HeevWork& W, int n, double2* s_wave) {
   for (int w = 0; w < wid; ++w) p = zmul(p, s_wave[w]);
   double2 ex = make_double2(__shfl_up(q.x, 1, 64), __shfl_up(q.y, 1, 64));
   if (lane == 0) ex = one;
-  p = zmul(p, ex);  // ph[2 tid]
+  p = zmul(p, ex);  // ph[4 tid]
 #pragma unroll
-  for (int r = 0; r < 2; ++r) {
-    const int k = 2 * tid + r;
+  for (int r = 0; r < 4; ++r) {
+    const int k = 4 * tid + r;
     p = zmul(p, f[r]);
     if (k + 1 < n) W.ph[k + 1] = p;
   }
@@ -307,19 +308,6 @@ __device__ void tri_phases(HeevWork& W, int n, double2* s_wave) {
   }
 }
 
-
-// LDS pitch (in 16-byte elements) of the trailing block in k_tridiag: 2 mod 4,
-// so that the lanes of a column-wise read (eight columns of one row, stride =
-// pitch) and of the update's mirrored rows (stride = pitch + 1) fall on
-// distinct banks
-__host__ __device__ constexpr int tri_pitch(int nb) { return nb + (6 - nb % 4) % 4; }
-
-// LDS bytes of k_tridiag for a trailing block of nb columns: the block, u and
-// the per-column reflector scalars (at least the DW entries of the phase scan)
-static size_t tri_lds(int nb) {
-  return std::max(sizeof(double2) * ((size_t)tri_pitch(nb) * nb + 2 * (size_t)nb) + 8 * (size_t)nb,
-                  sizeof(double2) * DW);
-}
 
 // 1/sqrt(x) for x > 0 within a few ulps: the hardware estimate refined by two
 // Newton steps, a shorter dependent chain than a square root and a division
@@ -345,24 +333,17 @@ __device__ __forceinline__ double read_lane(double x, int l) {
 // is set the caller's lane records alpha and the skip flag.
 __device__ __forceinline__ void tri_scalars(bool rec, int k, double xn2, double2 x0, HeevWork& W, int& skip,
                                             double& iv, double2& v0) {
+  // without branches: the two square roots overlap
   const double a2 = x0.x * x0.x + x0.y * x0.y;
   skip = (xn2 == 0.0 || xn2 - a2 <= 1e-300) ? 1 : 0;
-  iv = 0.0;
-  v0 = make_double2(0.0, 0.0);
-  double2 alpha = x0;
-  if (!skip) {
-    const double xn = xn2 * rsqrt_nr(xn2);
-    double ax0 = 0.0;
-    double2 phs = make_double2(1.0, 0.0);
-    if (a2 > 0.0) {
-      const double ra = rsqrt_nr(a2);
-      ax0 = a2 * ra;
-      phs = make_double2(x0.x * ra, x0.y * ra);
-    }
-    alpha = make_double2(-phs.x * xn, -phs.y * xn);
-    v0 = make_double2(x0.x + phs.x * xn, x0.y + phs.y * xn);
-    iv = rsqrt_nr(2.0 * xn * (xn + ax0));
-  }
+  const double rx = rsqrt_nr(xn2), ra = rsqrt_nr(a2), xn = xn2 * rx;
+  const bool nz = a2 > 0.0;
+  const double ax0 = nz ? a2 * ra : 0.0;
+  const double2 phs = make_double2(nz ? x0.x * ra : 1.0, nz ? x0.y * ra : 0.0);
+  const double r = rsqrt_nr(2.0 * xn * (xn + ax0));
+  const double2 alpha = skip ? x0 : make_double2(-phs.x * xn, -phs.y * xn);
+  iv = skip ? 0.0 : r;
+  v0 = make_double2(skip ? 0.0 : x0.x + phs.x * xn, skip ? 0.0 : x0.y + phs.y * xn);
   if (rec) {
     W.skip[k] = skip;
     W.sub[k] = alpha;
@@ -384,246 +365,245 @@ __device__ __forceinline__ void wide_reflector_scalars(int lane, int k, double x
   }
 }
 
-// Reflector of column c of the LDS block from its values below the diagonal
-// (one wavefront); lane 0 records it and stores its scalars in sc.
-__device__ __forceinline__ void tri_col_reflector(const double2* __restrict__ As, int lda, int nb, int k0, int c,
-                                                  int lane, HeevWork& W, double* sc) {
-  const double2* col = As + c * lda;
-  double part = 0.0;
-  for (int i = c + 1 + lane; i < nb; i += 64) part += col[i].x * col[i].x + col[i].y * col[i].y;
-  part = wave_sum(part);
-  int skip;
-  double iv;
-  double2 v0;
-  tri_scalars(lane == 0, k0 + c, part, col[c + 1], W, skip, iv, v0);
-  if (lane == 0) {
-    sc[0] = skip;
-    sc[1] = iv;
-    sc[2] = v0.x;
-    sc[3] = v0.y;
-  }
+// Sum over the lanes l, l ^ 16, l ^ 32, l ^ 48, every lane gets it.
+__device__ __forceinline__ double cross_row_sum(double x) {
+  auto halves = [](double y, auto swap) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(y);
+    const unsigned lo = (unsigned)(b & 0xffffffffull), hi = (unsigned)(b >> 32);
+    const auto l = swap(lo), h = swap(hi);
+    return __longlong_as_double((long long)(((unsigned long long)h[0] << 32) | l[0])) +
+           __longlong_as_double((long long)(((unsigned long long)h[1] << 32) | l[1]));
+  };
+  x = halves(x, [](unsigned w) { return __builtin_amdgcn_permlane16_swap(w, w, false, false); });
+  return halves(x, [](unsigned w) { return __builtin_amdgcn_permlane32_swap(w, w, false, false); });
 }
 
-// Householder reduction of the trailing block A[k0:, k0:] (nb = n - k0 rows
-// and columns) in LDS, one workgroup per matrix: the whole matrix for k0 = 0,
-// or the tail after the multi-workgroup steps 0..k0-1.  Only the lower
-// triangle is kept; indices below are local to the block.  Column c keeps x
-// while it is reduced; v = x iv (x_{c+1} replaced by v0) is formed where it
-// is read.  Per column c, with its reflector's scalars already in LDS:
-//   1. u = A v with A(i,j) = conj(A(j,i)) above the diagonal: each wavefront
-//      takes eight rows (lane >> 3) times eight column classes (lane & 7,
-//      columns c+1+cl, c+9+cl, ...), summed within the eight lanes by DPP;
-//      the wavefronts' parts of v^H u go to LDS;
-//   2. A -= v w^H + w v^H (w = 2u - 2 gamma v): wavefront 0 updates column
-//      c+1 and forms its reflector (look-ahead) while the other wavefronts
-//      update the lower triangle of rows and columns c+2.., each thread a row
-//      a and its mirror row m-1-a so that the threads share the work evenly.
-// Two barriers per column.  The reflectors are scaled to unit norm when the
-// block is written back.
-__global__ __launch_bounds__(DT) void k_tridiag(double2* __restrict__ Aall, int lda_g, int64_t strideA, int n,
-                                               int k0, int nev, double* __restrict__ work, int64_t strideWork) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int nb = n - k0, lda = tri_pitch(nb);
-  double2* As = reinterpret_cast<double2*>(smem);     // [lda * nb] A(i, j) = As[i + j lda], i >= j
-  double2* us = As + (size_t)lda * nb;                // [nb] u = A v
-  double2* rv0 = us + nb;                             // [nb] v0 iv of column c
-  double* riv = reinterpret_cast<double*>(rv0 + nb);  // [nb] iv of column c (0 without a reflector)
-  __shared__ double s_sc[2][4];                       // skip, iv, v0 of columns c (slot c & 1) and c + 1
-  __shared__ double s_g[DW];                          // the wavefronts' parts of v^H u
+// Sum over the 16 lanes of a row, every lane gets it.
+__device__ __forceinline__ double row_sum(double x) {
+  x += dpp_move<0x128>(x);  // row_ror:8, 4, 2, 1
+  x += dpp_move<0x124>(x);
+  x += dpp_move<0x122>(x);
+  return x + dpp_move<0x121>(x);
+}
+// Lane L of every row of 16 in all lanes of the row.
+template <int L> __device__ __forceinline__ double row_bcast(double x) {
+  return __longlong_as_double(__builtin_amdgcn_update_dpp(0ll, __double_as_longlong(x), 0x150 + L, 0xf, 0xf, true));
+}
+
+// Householder reduction of the trailing block A[k0:, k0:] (nb = n - k0 <= TNB
+// rows and columns) in registers, one workgroup per matrix: the whole matrix
+// for k0 = 0, or the tail after the multi-workgroup steps 0..k0-1.  Indices
+// below are local to the block.  The block, both triangles, lies in 16 x 16
+// accumulator tiles of the FP64 matrix cores: wavefront w holds columns
+// 16 w + (lane & 15), tile t of it the rows 16 t + (lane >> 4) + 4 r.
+// v, u and the next column go through LDS.  Per column c, with v in LDS:
+//   1. u = A^H v = A v: a lane sums its column over its rows (v of the rows
+//      is one LDS read per 64 rows, handed round the 16 columns by DPP), four
+//      lanes share a column; the wavefronts' parts of gamma = v^H u to LDS;
+//   2. A -= v (2u - 2 gamma v)^H + u (2v)^H, the rank-2 update of the
+//      reflector, two matrix instructions per tile: (v, u) of the rows
+//      against the columns' pair for the real part, against i times it for
+//      the imaginary one.  One wavefront first updates column c+1 (a copy in
+//      LDS) and forms its reflector.
+// Two barriers per column; tiles left of and above column c+1 are skipped.
+// v is zero outside rows c+1.. and u outside columns c+1.., so nothing else
+// needs masks, and a column without a reflector is one with v = 0.
+//
+// Bound: the chain from one reflector to the next (two barriers, three
+// reductions, the scalars of tri_scalars: 3100 cycles per column) and, on the
+// first columns, the vector ALU in 1 and the matrix cores in 2 (6300 cycles).
+// The block in LDS (98 columns at most, lower triangle) took 2.9 us per
+// column, 32 us for 20 columns: this takes 2.0 and 24, and the 30 columns
+// more save a launch of 5 us each (k_wide_step).  One matrix of 160 columns:
+// 310 + 62 * 5.0 us -> 250 + 32 * 5.0 us.
+constexpr int TNB = 128;       // rows and columns of the register block
+constexpr int TW = TDT / 64;   // wavefronts, one per 16 columns
+
+__global__ __launch_bounds__(TDT) void k_tridiag(double2* __restrict__ Aall, int lda_g, int64_t strideA, int n,
+                                                int k0, int nev, double* __restrict__ work, int64_t strideWork) {
+  typedef double d4 __attribute__((ext_vector_type(4)));
+  static_assert(TNB == 16 * TW && TNB == 128, "a wavefront per 16 columns, two rows of the block per lane");
+  __shared__ double2 s_vu[2][TNB][2];  // v (unit norm) and u of columns c and c + 1 (slot c & 1)
+  __shared__ double s_col[2][2][TNB];  // column c + 1 (slot (c + 1) & 1; re, im) before the update of step c
+  __shared__ double s_g[TW];           // the wavefronts' parts of v^H u
+  __shared__ double2 s_ph[TW];
+  const int nb = n - k0, nt = (nb + 15) / 16;
   const int mat = blockIdx.x;
   double2* Ag = Aall + mat * strideA + k0 + (int64_t)k0 * lda_g;
   HeevWork W(work + mat * strideWork, n, nev);
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const int nn = nb * nb;
-  for (int q0 = tid; q0 < nn; q0 += 4 * DT) {
-    double2 t[4];
+  const int tid = threadIdx.x, lane = tid & 63, ct = tid >> 6, l16 = lane & 15, lg = lane >> 4;
+  const int j = 16 * ct + l16;  // this lane's column
+  const int look = nt < TW ? TW - 1 : 0;  // the wavefront that forms the reflectors: one without columns, or soon
+  d4 ar[TW], ai[TW];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int q = q0 + r * DT, i = q % nb, j = q / nb;
-      t[r] = make_double2(0.0, 0.0);
-      if (q < nn && i >= j) t[r] = Ag[i + (int64_t)j * lda_g];
-    }
+  for (int t = 0; t < TW; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int q = q0 + r * DT, i = q % nb, j = q / nb;
-      if (q < nn && i >= j) As[i + j * lda] = t[r];
+    for (int r = 0; r < 4; ++r) {  // from the lower triangle
+      const int i = 16 * t + lg + 4 * r;
+      double2 e = make_double2(0.0, 0.0);
+      if (i < nb && j < nb) e = i >= j ? Ag[i + (int64_t)j * lda_g] : Ag[j + (int64_t)i * lda_g];
+      ar[t][r] = e.x;
+      ai[t][r] = i >= j ? e.y : -e.y;
     }
+  // reflector of column c from its values x (rows lane and lane + 64, zero
+  // outside c+1..nb-1): into s_vu and, for the back-transformation, column c
+  auto reflector = [&](int c, const double2* x) {
+    const double part = wave_sum(x[0].x * x[0].x + x[0].y * x[0].y + x[1].x * x[1].x + x[1].y * x[1].y);
+    const int l = (c + 1) & 63;
+    const double2 y = (c + 1) >> 6 ? x[1] : x[0];
+    const double2 x0 = make_double2(read_lane(y.x, l), read_lane(y.y, l));
+    int skip;
+    double iv;
+    double2 v0;
+    tri_scalars(lane == 0, k0 + c, part, x0, W, skip, iv, v0);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int i = lane + 64 * q;
+      const double2 a = i == c + 1 ? v0 : x[q];
+      const double2 v = skip ? make_double2(0.0, 0.0) : make_double2(a.x * iv, a.y * iv);
+      s_vu[c & 1][i][0] = v;
+      if (i > c && i < nb) Ag[i + (int64_t)c * lda_g] = v;
+    }
+  };
+  if (tid < TNB) {
+    s_vu[0][tid][1] = s_vu[1][tid][1] = make_double2(0.0, 0.0);
+    const double2 x = tid < nb && nb > 1 && tid >= 1 ? Ag[tid + lda_g] : make_double2(0.0, 0.0);
+    s_col[1][0][tid] = x.x;
+    s_col[1][1][tid] = x.y;
   }
-  __syncthreads();
-  if (nb > 2 && wid == 0) tri_col_reflector(As, lda, nb, k0, 0, lane, W, s_sc[0]);
-  __syncthreads();
-  for (int c = 0; c + 2 < nb; ++c) {
-    const int m = nb - c - 1;       // trailing rows and columns
-    const bool more = c + 3 < nb;  // column c+1 takes a reflector too
-    const double* sc = s_sc[c & 1];
-    const bool skip = sc[0] != 0.0;
-    const double iv = sc[1];
-    const double2 v0 = make_double2(sc[2], sc[3]);
-    if (tid == 0) {
-      rv0[c] = make_double2(v0.x * iv, v0.y * iv);
-      riv[c] = iv;
+  __syncthreads();  // columns 0 and 1 are read before the reflector overwrites column 0
+  if (ct == look && nb >= 2) {
+    double2 x[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int i = lane + 64 * q;
+      x[q] = i >= 1 && i < nb ? Ag[i] : make_double2(0.0, 0.0);
     }
-    if (skip) {  // nothing changes; column c+1 is read as it stands
-      if (more && wid == 0) tri_col_reflector(As, lda, nb, k0, c + 1, lane, W, s_sc[(c + 1) & 1]);
-      __syncthreads();
-      continue;
-    }
-    const double2* col = As + c * lda;
-    auto vat = [=](int j) {
-      const double2 x = j == c + 1 ? v0 : col[j];
-      return make_double2(x.x * iv, x.y * iv);
-    };
-    // 1. u = A v and the wavefront's part of v^H u
-    double gp = 0.0;
-    for (int i0 = c + 1 + wid * 8; i0 < nb; i0 += DT / 8) {
-      const int i = i0 + (lane >> 3);
-      double sr = 0.0, si = 0.0, tr = 0.0, ti = 0.0;
-      if (i < nb) {
-        for (int j0 = c + 1 + (lane & 7); j0 < nb; j0 += 64) {
-          double2 a[8], b[8];
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            const int j = j0 + 8 * q;
-            a[q] = make_double2(0.0, 0.0);
-            b[q] = make_double2(0.0, 0.0);
-            if (j < nb) {
-              const double2 e = As[j <= i ? i + j * lda : j + i * lda];
-              a[q] = j <= i ? e : make_double2(e.x, -e.y);
-              b[q] = vat(j);
-            }
-          }
-#pragma unroll
-          for (int q = 0; q < 8; q += 2) {
-            sr += a[q].x * b[q].x - a[q].y * b[q].y;
-            si += a[q].x * b[q].y + a[q].y * b[q].x;
-            tr += a[q + 1].x * b[q + 1].x - a[q + 1].y * b[q + 1].y;
-            ti += a[q + 1].x * b[q + 1].y + a[q + 1].y * b[q + 1].x;
-          }
-        }
-      }
-      sr += tr;
-      si += ti;
-      sr += dpp_move<0xb1>(sr);  // quad_perm [1,0,3,2]
-      si += dpp_move<0xb1>(si);
-      sr += dpp_move<0x4e>(sr);  // quad_perm [2,3,0,1]
-      si += dpp_move<0x4e>(si);
-      sr += dpp_move<0x114>(sr);  // row_shr:4: lanes 4..7 of each eight hold the row's sum
-      si += dpp_move<0x114>(si);
-      if ((lane & 7) == 4 && i < nb) {
-        us[i] = make_double2(sr, si);
-        const double2 vi = vat(i);
-        gp += vi.x * sr + vi.y * si;  // Re(conj(v_i) u_i)
-      }
-    }
-    gp = wave_sum(gp);
-    if (lane == 0) s_g[wid] = gp;
-    __syncthreads();
-    double gam = 0.0;
-#pragma unroll
-    for (int w = 0; w < DW; ++w) gam += s_g[w];
-    const double g2 = 2.0 * gam;
-    // 2. the rank-2 update
-    if (wid == 0) {
-      const int j = c + 1;
-      const double2 vj = vat(j), uj = us[j];
-      const double2 wj = make_double2(2.0 * uj.x - g2 * vj.x, 2.0 * uj.y - g2 * vj.y);
-      double part = 0.0;
-      double2 x0 = make_double2(0.0, 0.0);
-      for (int i = j + lane; i < nb; i += 64) {
-        const double2 vi = vat(i), ui = us[i];
-        const double2 wi = make_double2(2.0 * ui.x - g2 * vi.x, 2.0 * ui.y - g2 * vi.y);
-        const double2 t1 = zmul(vi, make_double2(wj.x, -wj.y));
-        const double2 t2 = zmul(wi, make_double2(vj.x, -vj.y));
-        double2& r = As[i + j * lda];
-        r = make_double2(r.x - t1.x - t2.x, r.y - t1.y - t2.y);
-        if (i > j) part += r.x * r.x + r.y * r.y;
-        if (i == j + 1) x0 = r;
-      }
-      if (more) {  // row c+2 of column c+1 lies in lane 1
-        part = wave_sum(part);
-        x0 = make_double2(read_lane(x0.x, 1), read_lane(x0.y, 1));
-        int skip1;
-        double iv1;
-        double2 v01;
-        tri_scalars(lane == 0, k0 + c + 1, part, x0, W, skip1, iv1, v01);
-        if (lane == 0) {
-          double* s = s_sc[(c + 1) & 1];
-          s[0] = skip1;
-          s[1] = iv1;
-          s[2] = v01.x;
-          s[3] = v01.y;
-        }
-      }
-    } else {
-      const int m2 = m - 1;  // rows and columns c+2 .. nb-1
-      const int P = (m2 + 1) / 2, cg = (DT - 64) / P;
-      const int t = tid - 64, p = t % P, g = t / P;
-      if (g < cg) {
-        const int ra = c + 2 + p, rb = c + 1 + m2 - p;  // rows a and m2-1-a of the block
-        const double2 va = vat(ra), ua = us[ra], vb = vat(rb), ub = us[rb];
-        const double2 wa = make_double2(2.0 * ua.x - g2 * va.x, 2.0 * ua.y - g2 * va.y);
-        const double2 wb = make_double2(2.0 * ub.x - g2 * vb.x, 2.0 * ub.y - g2 * vb.y);
-        const int ne = ra == rb ? p + 1 : m2 + 1;  // row a: p + 1 elements, row m2-1-a: m2 - p
-        for (int e0 = g; e0 < ne; e0 += 4 * cg) {
-          int idx[4];
-          double2 r[4], vj[4], uj[4];
-          bool fs[4];
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int e = e0 + q * cg;
-            fs[q] = e <= p;
-            const int i = fs[q] ? ra : rb, j = c + 2 + (fs[q] ? e : e - p - 1);
-            idx[q] = e < ne ? i + j * lda : -1;
-            r[q] = vj[q] = uj[q] = make_double2(0.0, 0.0);
-            if (e < ne) {
-              r[q] = As[idx[q]];
-              vj[q] = vat(j);
-              uj[q] = us[j];
-            }
-          }
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            if (idx[q] < 0) continue;
-            const double2 vi = fs[q] ? va : vb, wi = fs[q] ? wa : wb;
-            const double2 wj = make_double2(2.0 * uj[q].x - g2 * vj[q].x, 2.0 * uj[q].y - g2 * vj[q].y);
-            const double2 t1 = zmul(vi, make_double2(wj.x, -wj.y));
-            const double2 t2 = zmul(wi, make_double2(vj[q].x, -vj[q].y));
-            As[idx[q]] = make_double2(r[q].x - t1.x - t2.x, r[q].y - t1.y - t2.y);
-          }
-        }
-      }
-    }
-    __syncthreads();
-  }
-  __syncthreads();
-  // the reflectors (strict lower triangle, unit norm) for the back-transformation
-  for (int q0 = tid; q0 < nn; q0 += 4 * DT) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int q = q0 + r * DT, i = q % nb, j = q / nb;
-      if (q < nn && i > j && j + 2 < nb) {
-        const double2 x = As[i + j * lda];
-        Ag[i + (int64_t)j * lda_g] = i == j + 1 ? rv0[j] : make_double2(x.x * riv[j], x.y * riv[j]);
-      }
-    }
-  }
-  // the diagonal (rows before k0 were final after their own step) and the
-  // last sub-diagonal element
-  for (int i = tid; i < n; i += DT)
-    W.d[i] = i < k0 ? Aall[mat * strideA + i + (int64_t)i * lda_g].x : As[(i - k0) * (lda + 1)].x;
-  if (tid == 0) {
-    if (nb >= 2) {
-      W.sub[n - 2] = As[(nb - 1) + (nb - 2) * lda];
+    if (nb > 2) {
+      reflector(0, x);
+    } else if (lane == 1) {
+      W.sub[n - 2] = x[0];
       W.skip[n - 2] = 1;
     }
-    W.skip[n - 1] = 1;
   }
+  // the tiles are used here, before the loop: a wait for these loads inside it
+  // would also wait for the reflectors' stores, once per column
+#pragma unroll
+  for (int t = 0; t < TW; ++t) asm volatile("" : "+v"(ar[t]), "+v"(ai[t]));
   __syncthreads();
-  // phases: T' = D^H T D real with off-diagonal |sub| (As is free now)
-  tri_phases(W, n, As);
+  for (int c = 0; c + 2 < nb; ++c) {
+    const int t0 = (c + 1) >> 4;  // first tile row and column still needed
+    double2(*vu)[2] = s_vu[c & 1];
+    if (ct >= t0 && ct < nt) {
+      // v of this lane row's rows: lane 4 (t & 3) + r of half t >> 2 holds row 16 t + lg + 4 r
+      const double2 vh[2] = {vu[4 * l16 + lg][0], vu[64 + 4 * l16 + lg][0]};
+      const double2 vj = vu[j][0];
+      double sr = 0.0, si = 0.0, tr = 0.0, ti = 0.0;
+      auto rows = [&](auto tc, auto rc) {
+        constexpr int t = decltype(tc)::value, r = decltype(rc)::value;
+        const double vx = row_bcast<4 * (t & 3) + r>(vh[t >> 2].x), vy = row_bcast<4 * (t & 3) + r>(vh[t >> 2].y);
+        sr += ar[t][r] * vx;
+        si += ar[t][r] * vy;
+        tr += ai[t][r] * vy;
+        ti += ai[t][r] * vx;
+      };
+      auto tile = [&](auto tc) {
+        if (decltype(tc)::value < t0 || decltype(tc)::value >= nt) return;
+        rows(tc, std::integral_constant<int, 0>{});
+        rows(tc, std::integral_constant<int, 1>{});
+        rows(tc, std::integral_constant<int, 2>{});
+        rows(tc, std::integral_constant<int, 3>{});
+      };
+      tile(std::integral_constant<int, 0>{});
+      tile(std::integral_constant<int, 1>{});
+      tile(std::integral_constant<int, 2>{});
+      tile(std::integral_constant<int, 3>{});
+      tile(std::integral_constant<int, 4>{});
+      tile(std::integral_constant<int, 5>{});
+      tile(std::integral_constant<int, 6>{});
+      tile(std::integral_constant<int, 7>{});
+      sr = cross_row_sum(sr + tr);
+      si = cross_row_sum(si - ti);
+      const double2 u = j > c ? make_double2(sr, si) : make_double2(0.0, 0.0);
+      if (lg == 0) vu[j][1] = u;
+      const double gp = row_sum(vj.x * u.x + vj.y * u.y);  // Re(conj(v_j) u_j)
+      if (lane == 0) s_g[ct] = gp;
+    } else if (lane == 0) {
+      s_g[ct] = 0.0;
+    }
+    __syncthreads();
+    const double g2 = row_sum(s_g[l16 & (TW - 1)]);  // 2 gamma: the row holds every part twice
+    if (ct == look) {
+      __builtin_amdgcn_s_setprio(3);  // ahead of the matrix instructions of its SIMD
+      const int c1 = c + 1;
+      const double2 vj = vu[c1][0], uj = vu[c1][1];
+      const double2 wj = make_double2(2.0 * uj.x - g2 * vj.x, 2.0 * uj.y - g2 * vj.y);
+      double2 x[2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int i = lane + 64 * q;
+        const double2 a = make_double2(s_col[c1 & 1][0][i], s_col[c1 & 1][1][i]), vi = vu[i][0], ui = vu[i][1];
+        const double2 wi = make_double2(2.0 * ui.x - g2 * vi.x, 2.0 * ui.y - g2 * vi.y);
+        const double2 p = zmul(vi, make_double2(wj.x, -wj.y)), s = zmul(wi, make_double2(vj.x, -vj.y));
+        x[q] = i > c1 && i < nb ? make_double2(a.x - p.x - s.x, a.y - p.y - s.y) : make_double2(0.0, 0.0);
+      }
+      if (c1 + 2 < nb) {
+        reflector(c1, x);
+      } else {  // the last sub-diagonal element
+        const double2 y = (c1 + 1) >> 6 ? x[1] : x[0];
+        if (lane == ((c1 + 1) & 63)) {
+          W.sub[n - 2] = y;
+          W.skip[n - 2] = 1;
+        }
+      }
+      __builtin_amdgcn_s_setprio(0);
+    }
+    if (ct >= t0 && ct < nt) {
+      // operands, component k = lane >> 4: (v, u) of a row, negated; the
+      // pair (2u - 2 gamma v, 2v) of the column and i times it
+      const double2 vj = vu[j][0], uj = vu[j][1];
+      const double2 q = lg < 2 ? make_double2(2.0 * (uj.x - g2 * vj.x), 2.0 * (uj.y - g2 * vj.y))
+                               : make_double2(2.0 * vj.x, 2.0 * vj.y);
+      const double b1 = lg & 1 ? q.y : q.x, b2 = lg & 1 ? q.x : -q.y;
+      const double* rows = reinterpret_cast<const double*>(vu);
+#pragma unroll
+      for (int t = 0; t < TW; ++t) {
+        if (t < t0 || t >= nt) continue;
+        const double a = -rows[4 * (16 * t + l16) + lg];
+        ar[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b1, ar[t], 0, 0, 0);
+        ai[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b2, ai[t], 0, 0, 0);
+      }
+      if (ct == (c + 2) >> 4) {
+        double(*col)[TNB] = s_col[c & 1];
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+          if (t < t0 || t >= nt) continue;
+          if (j == c + 2) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              col[0][16 * t + lg + 4 * r] = ar[t][r];
+              col[1][16 * t + lg + 4 * r] = ai[t][r];
+            }
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+  // the diagonal (rows before k0 were final after their own step)
+  for (int i = tid; i < k0; i += TDT) W.d[i] = Aall[mat * strideA + i + (int64_t)i * lda_g].x;
+#pragma unroll
+  for (int t = 0; t < TW; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (t == ct && lg + 4 * r == l16 && j < nb) W.d[k0 + j] = ar[t][r];
+  if (tid == 0) W.skip[n - 1] = 1;
+  __syncthreads();
+  // phases: T' = D^H T D real with off-diagonal |sub|
+  tri_phases(W, n, s_ph);
 }
 
-// ---- 1'. wide tridiagonalisation (matrices that do not fit LDS): one
+// ---- 1'. wide tridiagonalisation (matrices of more than TNB columns): one
 // launch per column, the trailing matrix spread over many workgroups (one
 // wavefront per column).  k_wide_first and k_wide_gemv form reflector 0 and
 // u_0 = A22 v_0; launch k (k_wide_step) applies the rank-2 update of step k
@@ -698,7 +678,7 @@ __global__ __launch_bounds__(WT) void k_wide_gemv(double2* __restrict__ Aall, in
 // reflector k+1 (vb, scal, skip, sub), the updated diagonal entry of column
 // k+1, and reflector k into column k for the back-transformation.  On the
 // last wide step (`last`) column k+1 is updated in place like the others,
-// for the in-LDS reduction that follows.
+// for the one-workgroup reduction that follows.
 __global__ __launch_bounds__(WT) void k_wide_step(double2* __restrict__ Aall, int lda, int64_t strideA, int n,
                                                   int nev, int k, int last, double* __restrict__ work,
                                                   int64_t strideWork) {
@@ -1137,12 +1117,9 @@ void heev_gpu(double2* A, int lda, int64_t strideA, int n, int nev, double* Wv, 
   DEREK_REQUIRE(n >= 1 && nev >= 1 && nev <= n, "heev: need 1 <= nev <= n");
   DEREK_REQUIRE(n <= 2048, "heev: n must be <= 2048");
   {
-    // the largest trailing block the LDS kernel holds
-    int nbl = std::min(n, 98);
-    while (nbl > 1 && tri_lds(nbl) > kTridiagLds) --nbl;
-    const int k0 = n - nbl;
-    // steps 0..k0-1 with two multi-workgroup launches per column while the
-    // trailing matrix is larger than that, then the rest in one workgroup
+    const int k0 = std::max(0, n - TNB);
+    // steps 0..k0-1 with a multi-workgroup launch per column, then the rest in
+    // one workgroup
     if (k0 > 0) {
       hipLaunchKernelGGL(k_wide_first, dim3(batch), dim3(64), 0, s, A, lda, strideA, n, nev, work, strideWork);
       hipLaunchKernelGGL(k_wide_gemv, dim3((unsigned)ceil_div(n - 1, WC), batch), dim3(WT), 0, s, A, lda, strideA, n,
@@ -1153,8 +1130,7 @@ void heev_gpu(double2* A, int lda, int64_t strideA, int n, int nev, double* Wv, 
                            k == k0 - 1 ? 1 : 0, work, strideWork);
       }
     }
-    allow_dynamic_lds(reinterpret_cast<const void*>(k_tridiag), kTridiagLds);
-    hipLaunchKernelGGL(k_tridiag, dim3(batch), dim3(DT), tri_lds(nbl), s, A, lda, strideA, n, k0, nev, work,
+    hipLaunchKernelGGL(k_tridiag, dim3(batch), dim3(TDT), 0, s, A, lda, strideA, n, k0, nev, work,
                        strideWork);
     DEREK_HIP(hipGetLastError());
   }

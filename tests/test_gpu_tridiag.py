@@ -1,4 +1,6 @@
-"""Eigenpairs of matrices whose tridiagonal form splits.
+"""Eigenpairs at the edges of the one-workgroup tridiagonalisation: its 16 x 16
+register tiles, the wavefront that forms the reflectors (an idle one up to 112
+columns), and the 128 columns from which on multi-workgroup steps come first.
 
 Bounds: Householder reduction, bisection and inverse iteration are backward
 stable, with errors of a few n eps |A|; the bounds are those of the other
@@ -28,6 +30,23 @@ def check(ctx, A):
     assert np.max(np.abs(w - ref)) < 1e-12 * scale * n
     assert np.max(np.abs(A @ Z - Z * w[None, :])) < 1e-11 * scale * np.sqrt(n)
     assert np.max(np.abs(Z.conj().T @ Z - np.eye(n))) < 1e-11 * np.sqrt(n)
+
+
+@pytest.mark.parametrize("n", [4, 15, 18, 31, 32, 47, 48, 49, 63, 65, 66, 95, 111, 113, 126, 127, 129, 130, 131, 145])
+def test_tile_edges(ctx, n):
+    print("tridiag", n, flush=True)
+    rng = np.random.default_rng(n)
+    A = rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))
+    A = A + A.conj().T
+    check(ctx, A)
+    check(ctx, 1e-30 * A)
+    # a diagonal block at the end and one dense corner: columns without a
+    # reflector before and after ones with
+    k = n // 3
+    A[k:, :] = A[:, k:] = 0
+    A[np.arange(k, n), np.arange(k, n)] = np.arange(k, n)
+    A[n - 1, 0] = A[0, n - 1] = 0.5
+    check(ctx, A)
 
 
 @pytest.mark.parametrize("n,seed", [(18, 3), (47, 0), (65, 6), (95, 5)])
