@@ -789,6 +789,115 @@ __global__ __launch_bounds__(WT) void k_wide_step(double2* __restrict__ Aall, in
 }
 
 
+// The same step for at most 64 PF trailing rows: a wavefront per column j with
+// everything in registers, loaded at once: v, u, column k+1 and column j.
+// Every wavefront forms reflector k+1 for itself; nothing goes through LDS and
+// there are no barriers.  The wavefront of column k+1 records the reflector.
+// Bound: one round trip of loads that miss the L2 of their XCD (the previous
+// launch wrote them elsewhere), the chain of three reductions, and the launch.
+// n = 600 (128 to 600 rows): 8.2 us a step with the workgroup's LDS copy,
+// 4.6 here; n = 160: 5.0 and 3.8; four matrices of n = 600: 11.9 and 9.1.
+template <int PF>
+__global__ __launch_bounds__(WT) void k_wide_regs(double2* __restrict__ Aall, int lda, int64_t strideA, int n, int nev,
+                                                  int k, int last, double* __restrict__ work, int64_t strideWork) {
+  const int mat = blockIdx.y;
+  HeevWork W(work + mat * strideWork, n, nev);
+  double2* A = Aall + mat * strideA;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int k1 = k + 1, j = k1 + blockIdx.x * WC + wid;
+  if (j >= n) return;
+  const bool own = j == k1;  // records reflectors k and k+1
+  const double2* vg = W.vb + (size_t)(k & 1) * n;
+  const double2* ug = W.uu + (size_t)(k & 1) * n;
+  double2* col = A + (int64_t)j * lda;
+  double2 v[PF], w[PF], c[PF], a[PF];
+#pragma unroll
+  for (int q = 0; q < PF; ++q) {
+    const int i = k1 + lane + 64 * q;
+    v[q] = w[q] = c[q] = a[q] = make_double2(0.0, 0.0);
+    if (i < n) {
+      v[q] = vg[i];
+      w[q] = ug[i];
+      c[q] = A[i + (int64_t)k1 * lda];
+      a[q] = col[i];
+    }
+  }
+  double2 vj = vg[j], wj = ug[j];
+  const bool skip = W.scal[4 * (k & 1)] != 0.0;  // column k needed no reflector: v = u = 0
+  const double2 zero = make_double2(0.0, 0.0);
+  if (skip) {
+    vj = wj = zero;
+#pragma unroll
+    for (int q = 0; q < PF; ++q) v[q] = w[q] = zero;
+  }
+  double gp = 0.0;
+#pragma unroll
+  for (int q = 0; q < PF; ++q) gp += zconjmul(v[q], w[q]).x;
+  const double g2 = 2.0 * wave_sum(gp);
+  auto wof = [=](double2 vi, double2 ui) { return make_double2(2.0 * ui.x - g2 * vi.x, 2.0 * ui.y - g2 * vi.y); };
+  // x - v_i conj(w_j) - w_i conj(v_j)
+  auto upd = [](double2 x, double2 vi, double2 wi, double2 vl, double2 wl) {
+    const double2 t1 = zmul(vi, make_double2(wl.x, -wl.y));
+    const double2 t2 = zmul(wi, make_double2(vl.x, -vl.y));
+    return make_double2(x.x - t1.x - t2.x, x.y - t1.y - t2.y);
+  };
+  wj = wof(vj, wj);
+#pragma unroll
+  for (int q = 0; q < PF; ++q) w[q] = wof(v[q], w[q]);
+  if (own && !skip) {
+#pragma unroll
+    for (int q = 0; q < PF; ++q) {
+      const int i = k1 + lane + 64 * q;
+      if (i < n) A[i + (int64_t)k * lda] = v[q];
+    }
+  }
+  int skip1 = 1;
+  double iv1 = 0.0;
+  if (!last) {
+    // column k+1 below its diagonal (row k+1 is lane 0 of q = 0), its reflector
+    const double2 v1 = make_double2(read_lane(v[0].x, 0), read_lane(v[0].y, 0));
+    const double2 w1 = make_double2(read_lane(w[0].x, 0), read_lane(w[0].y, 0));
+    double part = 0.0;
+#pragma unroll
+    for (int q = 0; q < PF; ++q) {
+      c[q] = upd(c[q], v[q], w[q], v1, w1);
+      if (q == 0 && lane == 0) {
+        if (own && !skip) col[k1] = c[0];  // the diagonal entry
+        c[0] = zero;
+      }
+      part += c[q].x * c[q].x + c[q].y * c[q].y;
+    }
+    part = wave_sum(part);
+    const double2 x0 = make_double2(read_lane(c[0].x, 1), read_lane(c[0].y, 1));
+    double2 v01;
+    wide_reflector_scalars(own ? lane : 1, k1, part, x0, W, skip1, iv1, v01);
+    if (lane == 1) c[0] = v01;
+    if (own) {
+      double2* vb1 = W.vb + (size_t)(k1 & 1) * n;
+#pragma unroll
+      for (int q = 0; q < PF; ++q) {
+        const int i = k1 + lane + 64 * q;
+        if (i > k1 && i < n) vb1[i] = make_double2(c[q].x * iv1, c[q].y * iv1);
+      }
+      return;
+    }
+  }
+  double sr = 0.0, si = 0.0;
+#pragma unroll
+  for (int q = 0; q < PF; ++q) {
+    const int i = k1 + lane + 64 * q;
+    a[q] = upd(a[q], v[q], w[q], vj, wj);
+    if (!skip && i < n) col[i] = a[q];
+    const double2 t = zconjmul(a[q], c[q]);  // row k+1 of c is zero
+    sr += t.x;
+    si += t.y;
+  }
+  if (last) return;
+  sr = wave_sum(sr) * iv1;
+  si = wave_sum(si) * iv1;
+  if (lane == 0) W.uu[(size_t)(k1 & 1) * n + j] = make_double2(sr, si);
+}
+
 // ---- 2. eigenvalues by multisection: one wavefront per eigenvalue; the 64
 // lanes count eigenvalues below 64 interior points, so every step narrows the
 // bracket 65-fold.  When the eigenvalues of a launch fit one round of the CUs,
@@ -1125,9 +1234,15 @@ void heev_gpu(double2* A, int lda, int64_t strideA, int n, int nev, double* Wv, 
       hipLaunchKernelGGL(k_wide_gemv, dim3((unsigned)ceil_div(n - 1, WC), batch), dim3(WT), 0, s, A, lda, strideA, n,
                          nev, 0, work, strideWork);
       for (int k = 0; k < k0; ++k) {
-        dim3 grid((unsigned)ceil_div(n - k - 1, WC), batch);
-        hipLaunchKernelGGL(k_wide_step, grid, dim3(WT), sizeof(double2) * (size_t)n, s, A, lda, strideA, n, nev, k,
-                           k == k0 - 1 ? 1 : 0, work, strideWork);
+        const dim3 grid((unsigned)ceil_div(n - k - 1, WC), batch);
+        const int last = k == k0 - 1 ? 1 : 0, pf = (int)ceil_div(n - k - 1, 64);
+        // in registers while a column and its three companions fit them
+        if (pf > 10)
+          hipLaunchKernelGGL(k_wide_step, grid, dim3(WT), sizeof(double2) * (size_t)n, s, A, lda, strideA, n, nev, k,
+                             last, work, strideWork);
+        else
+          hipLaunchKernelGGL(pf > 7 ? k_wide_regs<10> : (pf > 4 ? k_wide_regs<7> : k_wide_regs<4>), grid, dim3(WT), 0,
+                             s, A, lda, strideA, n, nev, k, last, work, strideWork);
       }
     }
     hipLaunchKernelGGL(k_tridiag, dim3(batch), dim3(TDT), 0, s, A, lda, strideA, n, k0, nev, work,

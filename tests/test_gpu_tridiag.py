@@ -61,3 +61,18 @@ def test_rows_decoupled_from_the_rest(ctx, n, seed):
     A[np.arange(k, n), np.arange(k, n)] = np.arange(k, n)
     A[n - 1, 0] = A[0, n - 1] = 0.5
     check(ctx, A)
+
+
+@pytest.mark.parametrize("n", [192, 256, 257, 258, 320, 448, 449, 450, 577, 640, 641, 642, 700])
+def test_multi_workgroup_steps(ctx, n):
+    """Trailing rows at the edges of the register steps (256, 448 and 640 rows)
+    and beyond them; columns without a reflector among the others."""
+    print("wide steps", n, flush=True)
+    rng = np.random.default_rng(n)
+    A = rng.normal(size=(n, n)) + 1j * rng.normal(size=(n, n))
+    A = A + A.conj().T
+    for q in (1, 2, n - 200, n - 130):
+        if q > 0:  # column q - 1 keeps its diagonal and sub-diagonal only
+            A[q + 1:, :q] = 0
+            A[:q, q + 1:] = 0
+    check(ctx, A)
