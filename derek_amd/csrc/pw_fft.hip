@@ -1143,6 +1143,187 @@ __global__ __launch_bounds__((Slab<R, N, true>::NT)) void k_slab_vmul(PwBatch B,
   }
 }
 
+// ---------------------------------------------------------------- the same pass with a line per few lanes of one wavefront
+// N = R1 R1: the R1 threads of a line are the same in both stages, so a
+// wavefront that keeps whole lines (64 / R1 of them) needs no barrier between
+// the stages of a line: planes wid, wid + nw, ... (in groups of LPW) in A and
+// C, x lines likewise in B, each wavefront with its own lines of X.  Two
+// barriers per band (around B, where the axes change hands) instead of 16,
+// and every wavefront has work in every phase.
+// 144 lines of complex64: twelve wavefronts with 5 lines each; the sticks of
+// a thread's planes (at most two) stay in registers.  Pitch 156 of A and X:
+// the fewest LDS passes over all accesses of the kernel (593 against 744 for
+// 156 / 157, counted over 32 eight-byte banks).
+template <int N> struct Lines {
+  static constexpr int R1 = Split<N>::R1;
+  static_assert(R1 * R1 == N && R1 <= 16, "both stages of a line on the same threads");
+  static constexpr int RP = R1 | 1, L = R1 * RP, LPW = 64 / R1, NG = (N + LPW - 1) / LPW;
+  static constexpr int MAXW = 12, NP = 2;  // wavefronts; groups of planes per wavefront
+  template <typename R> static constexpr size_t lds(int nax_cap, int nw) {
+    return sizeof(cx_t<R>) * ((size_t)nax_cap * L + (size_t)nw * LPW * L) + sizeof(int) * N;
+  }
+  // wavefronts that the LDS holds and the planes need; 0: none
+  template <typename R> static int waves(int nax_cap) {
+    for (int nw = MAXW; nw * LPW * NP >= nax_cap; --nw)
+      if (lds<R>(nax_cap, nw) <= 160 * 1024) return nw;
+    return 0;
+  }
+};
+
+// LDS accesses of one wavefront on lines of its own stay in program order
+__device__ __forceinline__ void line_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <typename R, int N, bool Q>
+__global__ __launch_bounds__(64 * Lines<N>::MAXW) void k_slab_lines(PwBatch B, cx_t<R>* __restrict__ S, int nz, int bpw,
+                                                                  const cx_t<R>* __restrict__ tw,
+                                                                  const R* __restrict__ vt) {
+  using C = cx_t<R>;
+  using G = Lines<N>;
+  constexpr int R1 = G::R1, RP = G::RP, L = G::L, LPW = G::LPW, NP = G::NP;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const PwMaps m = B.mt[B.k0 + blockIdx.z];
+  const int z = blockIdx.x, grp = blockIdx.y, nw = blockDim.x >> 6, nax = m.nax;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int l = lane / R1, d = lane % R1;  // line of the wavefront, digit
+  const bool on = l < LPW;
+  C* A = reinterpret_cast<C*>(smem);
+  C* X = A + (size_t)B.nax_cap * L + (size_t)(wid * LPW + (on ? l : 0)) * L;  // this thread's x line
+  int* xa = reinterpret_cast<int*>(A + ((size_t)B.nax_cap + (size_t)nw * LPW) * L);
+  for (int x = threadIdx.x; x < N; x += blockDim.x) xa[x] = -1;
+  auto has = [](int r) { return !Q || quarter_has(r, R1); };
+  // sticks y = d + R1 r of the thread's planes
+  uint32_t st[NP][R1];
+  C* plane[NP];
+  bool pl[NP];
+#pragma unroll
+  for (int p = 0; p < NP; ++p) {
+    const int a = (wid + nw * p) * LPW + l;
+    pl[p] = on && a < nax;
+    plane[p] = A + (size_t)(pl[p] ? a : 0) * L;
+#pragma unroll
+    for (int r = 0; r < R1; ++r) {
+      const int q = pl[p] && has(r) ? m.pl_y[a * N + d + R1 * r] : -1;
+      st[p][r] = q >= 0 ? (uint32_t)q * (uint32_t)sizeof(C) : kOob;
+    }
+  }
+  C tk[R1];
+#pragma unroll
+  for (int r = 1; r < R1; ++r) tk[r] = tw[(d * r) % N];
+  __syncthreads();
+  for (int a = threadIdx.x; a < nax; a += blockDim.x) xa[m.ax_x[a]] = a;
+  __syncthreads();
+  int xr[R1];  // rows of A of x = d + R1 r
+#pragma unroll
+  for (int r = 0; r < R1; ++r) {
+    const int a = xa[d + R1 * r];
+    xr[r] = a >= 0 ? a * L : -1;
+  }
+  const R* vz = vt + (int64_t)z * N * N;  // V at (x, y, z) in vz[y*N + x]
+  const int bb0 = grp * bpw, bb1 = min(B.nbb, bb0 + bpw);
+  const uint32_t row_bytes = (uint32_t)B.nst_cap * (uint32_t)sizeof(C);
+  auto row_rsrc = [&](int band) {
+    return buf_rsrc(S + (((int64_t)blockIdx.z * B.nbb + band) * nz + z) * B.nst_cap, row_bytes);
+  };
+  C pre[NP][R1];
+  auto load = [&](int band) {
+    const auto rs = row_rsrc(band);
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int r = 0; r < R1; ++r) pre[p][r] = has(r) ? buf_ld<C>(rs, st[p][r]) : cmk<C>(0, 0);
+  };
+  // slots: index d + R1 r of a line lies in slot d RP + r
+  if (Q) load(bb0);
+  for (int band = bb0; band < bb1; ++band) {
+    if (!Q) load(band);
+    // A: y inverse of the wavefront's planes
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+      if (pl[p]) {
+        C* row = plane[p];
+        dftR<R1, +1>(pre[p], (const C*)nullptr, N);
+#pragma unroll
+        for (int k = 0; k < R1; ++k) row[k * RP + d] = pre[p][k];
+        line_fence();
+        C u[R1];
+        row += d * RP;
+#pragma unroll
+        for (int r = 0; r < R1; ++r) u[r] = r ? cmul(row[r], cconj(tk[r])) : row[r];
+        dftR<R1, +1>(u, (const C*)nullptr, N);
+#pragma unroll
+        for (int k = 0; k < R1; ++k) row[k] = u[k];
+      }
+    __syncthreads();
+    // B: x lines, inverse, * V / (nx ny nz), forward
+#pragma unroll 1
+    for (int g = wid; g < G::NG; g += nw) {
+      const int y = g * LPW + l;
+      R vq[R1];  // V of the thread's points, used after the first two stages
+      const R* vy = vz + min(y, N - 1) * N + d;
+#pragma unroll
+      for (int k = 0; k < R1; ++k) vq[k] = vy[R1 * k];
+      if (on && y < N) {
+        const int py = (y % R1) * RP + y / R1;
+        C v[R1];
+#pragma unroll
+        for (int r = 0; r < R1; ++r) v[r] = (has(r) && xr[r] >= 0) ? A[xr[r] + py] : cmk<C>(0, 0);
+        dftR<R1, +1>(v, (const C*)nullptr, N);
+#pragma unroll
+        for (int k = 0; k < R1; ++k) X[k * RP + d] = v[k];
+        line_fence();
+        C u[R1];
+        C* row = X + d * RP;
+#pragma unroll
+        for (int r = 0; r < R1; ++r) u[r] = r ? cmul(row[r], cconj(tk[r])) : row[r];
+        dftR<R1, +1>(u, (const C*)nullptr, N);
+#pragma unroll
+        for (int k = 0; k < R1; ++k) u[k] = cscale(u[k], vq[k]);
+        dftR<R1, -1>(u, (const C*)nullptr, N);
+#pragma unroll
+        for (int k = 0; k < R1; ++k) row[k] = k ? cmul(u[k], tk[k]) : u[k];
+        line_fence();
+#pragma unroll
+        for (int j = 0; j < R1; ++j) v[j] = X[j * RP + d];
+        dftR<R1, -1>(v, (const C*)nullptr, N);
+#pragma unroll
+        for (int k = 0; k < R1; ++k)
+          if (has(k) && xr[k] >= 0) A[xr[k] + py] = v[k];
+        line_fence();
+      }
+    }
+    __syncthreads();
+    if (Q && band + 1 < bb1) load(band + 1);
+    // C: y forward of the wavefront's planes, back to the sticks
+    const auto rs = row_rsrc(band);
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+      if (pl[p]) {
+        C* row = plane[p];
+        C v[R1];
+#pragma unroll
+        for (int r = 0; r < R1; ++r) v[r] = row[d * RP + r];
+        dftR<R1, -1>(v, (const C*)nullptr, N);
+#pragma unroll
+        for (int k = 0; k < R1; ++k) row[d * RP + k] = v[k];
+        line_fence();
+        C u[R1];
+#pragma unroll
+        for (int j = 0; j < R1; ++j) {
+          const C w = row[j * RP + d];
+          u[j] = j ? cmul(w, tk[j]) : w;
+        }
+        dftR<R1, -1>(u, (const C*)nullptr, N);
+#pragma unroll
+        for (int k = 0; k < R1; ++k)
+          if (has(k)) buf_st<C>(rs, st[p][k], u[k]);
+        line_fence();
+      }
+  }
+}
+
 // Density on z-major sticks: per z plane and group of bands of one k-point,
 // the y and x inverse transforms as in k_slab_vmul, then
 // part[p][z][y][x] = sum over the group's bands of occ |psi(r)|^2 in FP64
@@ -1248,6 +1429,17 @@ template <typename R> bool slab_supported(int nx, int ny, int nz, int nax_cap, i
 
 template <typename R, int N>
 static void slab_vmul_n(const PwBatch& B, cx_t<R>* S, const Axis<R>* ax, int nz, const R* vt, int bpw, hipStream_t s) {
+  if constexpr (N == 144 && sizeof(R) == 4) {
+    using G = Lines<N>;
+    if (const int nw = G::template waves<R>(B.nax_cap)) {
+      const size_t lds = G::template lds<R>(B.nax_cap, nw);
+      auto kern = B.quarter ? k_slab_lines<R, N, true> : k_slab_lines<R, N, false>;
+      allow_lds_pw(kern, lds);
+      hipLaunchKernelGGL(kern, dim3((unsigned)nz, (unsigned)ceil_div(B.nbb, bpw), B.nkc), dim3(64 * nw), lds, s, B, S,
+                         nz, bpw, ax[0].tw, vt);
+      return;
+    }
+  }
   using SL = Slab<R, N, true>;
   const size_t lds = SL::lds(B.nax_cap);
   check_lds_pw(lds, N);
