@@ -877,6 +877,8 @@ void planes_x_density(const PwBatch& B, const cx_t<R>* P, const Axis<R>* ax, int
 //   B  x lines in rounds of LR: inverse transform of the active rows,
 //      * V(x, y, z) / (nx ny nz), forward transform, active rows back into A;
 //   C  y forward of each active plane, stick rows written back.
+// (k_slab_vmul at N = 32 and k_slab_density; k_slab_lines below is the pass of
+// H|psi> at the other lengths.)
 // Each length-N transform is two register stages, N = R1 R2: R2 threads
 // (digit j2) take R1-point DFTs over the inputs j2 + R2 r, R1 threads (digit
 // k1) finish with R2-point DFTs; the result with index k1 + R1 k2 sits in
@@ -887,9 +889,7 @@ void planes_x_density(const PwBatch& B, const cx_t<R>* P, const Axis<R>* ax, int
 // x rows in registers for the whole launch.  Compared with the separate y and
 // x passes the active planes stay on chip: HBM sees the stick rows once each
 // way and V once per band group.
-// VM: parameters of k_slab_vmul (false: k_slab_density, whose FP64
-// accumulators need more registers per thread)
-template <typename R, int N, bool VM = false> struct Slab {
+template <typename R, int N> struct Slab {
   static constexpr int R1 = Split<N>::R1, R2 = Split<N>::R2;
   static constexpr int R2P = R2 % 2 ? R2 : R2 + 1;
   static constexpr int L = R1 * R2P;              // slots of a line
@@ -909,18 +909,11 @@ template <typename R, int N, bool VM = false> struct Slab {
   // 360 threads at N = 72 (not 288): the R1- and R2-thread stages then take
   // 40 and 45 planes per pass, so the 33 active planes of a 16 bohr cell at
   // Ecut 20 Ha need one pass per y stage instead of two
-  // complex64 H|psi> at 144 runs 840 threads (70 planes per pass: one pass
-  // per y stage for the 69 active planes of a 30 bohr cell at Ecut 25 Ha,
-  // and 14 waves on the CU that its LDS working set allows)
-  // FP64 H|psi> at 72 runs 720 threads with all 72 x lines in one round
-  // (7 barrier phases per band instead of 13; one 136 KB workgroup per CU)
-  static constexpr bool kWide72 = VM && N == 72 && sizeof(R) == 8;
-  static constexpr int NT =
-      N == 32 ? 256 : (N == 72 ? (kWide72 ? 720 : 360) : (VM && N == 144 && sizeof(R) == 4 ? 840 : 504));
+  static constexpr int NT = N == 32 ? 256 : (N == 72 ? 360 : 504);
   // x lines per round: the complex64 108 case is sized for two workgroups per
   // CU; complex64 at 72 takes the 72 lines in two rounds
   static constexpr int LR =
-      N == 32 ? 32 : (N == 72 ? (kWide72 ? 72 : (sizeof(R) == 4 ? 36 : 24)) : (N == 108 && sizeof(R) == 4 ? 27 : 36));
+      N == 32 ? 32 : (N == 72 ? (sizeof(R) == 4 ? 36 : 24) : (N == 108 && sizeof(R) == 4 ? 27 : 36));
   static constexpr int NR = (N + LR - 1) / LR;
   static constexpr int LJ = NT / R2, LK = NT / R1;  // lines per pass of the R2- / R1-thread stages
   static_assert(NT % R1 == 0 && NT % R2 == 0, "workgroup size must keep each thread's digits");
@@ -937,9 +930,9 @@ template <typename R, int N, bool VM = false> struct Slab {
 // (j2 in the R2-thread stages, k1 in the R1-thread stages, and its line in
 // each), its twiddles exp(-2 pi i k1 r / N) and the LDS rows of the active
 // planes at x = j2 + R2 r (-1 if none).
-template <typename R, int N, bool VM, bool Q> struct SlabThread {
+template <typename R, int N, bool Q> struct SlabThread {
   using C = cx_t<R>;
-  using SL = Slab<R, N, VM>;
+  using SL = Slab<R, N>;
   static constexpr int R1 = SL::R1, R2 = SL::R2, R2P = SL::R2P, NT = SL::NT, LR = SL::LR;
   static constexpr int LPA = SL::LPA, LPX = SL::LPX;
   static constexpr int LJ = SL::LJ, LK = SL::LK;
@@ -985,18 +978,12 @@ template <typename R, int N, bool VM, bool Q> struct SlabThread {
 #pragma unroll
     for (int r = 0; r < R1; ++r) v[r] = in1(r) ? buf_ld<C>(rs, stick_off(ty[R2 * r])) : cmk<C>(0, 0);
   }
-  // y inverse of every active plane from a stick row into A (two barriers);
-  // with PRE, `pre` holds the first item's inputs
-  template <bool PRE, typename Rs> __device__ __forceinline__ void y_inverse(const Rs& rs, const C (&pre)[R1]) {
+  // y inverse of every active plane from a stick row into A (two barriers)
+  template <typename Rs> __device__ __forceinline__ void y_inverse(const Rs& rs) {
     // A1: y = j2 + R2 r from the sticks, output k in slot k R2P + j2
     for (int a = lj; a < nax; a += LJ) {
       C v[R1];
-      if (PRE && a == lj) {
-#pragma unroll
-        for (int r = 0; r < R1; ++r) v[r] = pre[r];
-      } else {
-        load_a1(rs, a, v);
-      }
+      load_a1(rs, a, v);
       dftR<R1, +1>(v, (const C*)nullptr, N);
       C* row = A + a * LPA + j2;
 #pragma unroll
@@ -1040,21 +1027,17 @@ template <typename R, int N, bool VM, bool Q> struct SlabThread {
 };
 
 template <typename R, int N, bool Q>
-__global__ __launch_bounds__((Slab<R, N, true>::NT)) void k_slab_vmul(PwBatch B, cx_t<R>* __restrict__ S, int nz, int bpw,
+__global__ __launch_bounds__((Slab<R, N>::NT)) void k_slab_vmul(PwBatch B, cx_t<R>* __restrict__ S, int nz, int bpw,
                                                               const cx_t<R>* __restrict__ tw,
                                                               const R* __restrict__ vt) {
   using C = cx_t<R>;
-  using ST = SlabThread<R, N, true, Q>;
-  constexpr int R1 = ST::R1, R2 = ST::R2, LR = ST::LR, NR = Slab<R, N, true>::NR, LJ = ST::LJ, LK = ST::LK;
+  using ST = SlabThread<R, N, Q>;
+  constexpr int R1 = ST::R1, R2 = ST::R2, LR = ST::LR, NR = Slab<R, N>::NR, LJ = ST::LJ, LK = ST::LK;
   constexpr int LPA = ST::LPA, LPX = ST::LPX;
   extern __shared__ __align__(16) unsigned char smem[];
   const PwMaps m = B.mt[B.k0 + blockIdx.z];
-  // complex128 runs one workgroup per CU and waits on its V rows: planes
-  // grouped per XCD (measured 4-5 % faster at 108^3; complex64, two
-  // workgroups per CU, keeps the plane-fastest order, which measured 1-2 %
-  // faster for it)
   int z = blockIdx.x, grp = blockIdx.y;
-  if constexpr (sizeof(R) == 8) xcd_task(z, grp);
+  if constexpr (sizeof(R) == 8) xcd_task(z, grp);  // as in k_slab_lines
   ST t;
   t.init(B, m, tw, smem);
   const int nax = t.nax, j2 = t.j2, lj = t.lj, k1 = t.k1, lk = t.lk;
@@ -1066,14 +1049,9 @@ __global__ __launch_bounds__((Slab<R, N, true>::NT)) void k_slab_vmul(PwBatch B,
   auto row_rsrc = [&](int band) {
     return buf_rsrc(S + (((int64_t)blockIdx.z * B.nbb + band) * nz + z) * B.nst_cap, row_bytes);
   };
-  // the first A1 item's sticks of the next band are loaded during phase C
-  // (complex128 at one workgroup per CU, where the registers are free)
-  constexpr bool kPre = sizeof(R) == 8 && N >= 100;
-  C pre[R1];
-  if (kPre && lj < nax) t.load_a1(row_rsrc(bb0), lj, pre);
   for (int band = bb0; band < bb1; ++band) {
     const auto rs = row_rsrc(band);
-    t.template y_inverse<kPre>(rs, pre);
+    t.y_inverse(rs);
 #pragma unroll 1
     for (int q = 0; q < NR; ++q) {
       const int y0 = q * LR, ln = min(LR, N - y0);
@@ -1112,7 +1090,6 @@ __global__ __launch_bounds__((Slab<R, N, true>::NT)) void k_slab_vmul(PwBatch B,
       }
       __syncthreads();
     }
-    if (kPre && band + 1 < bb1 && lj < nax) t.load_a1(row_rsrc(band + 1), lj, pre);
     // C1: y = j2 + R2 r, output k1 back into the slot of y = j2 + R2 k1
     for (int a = lj; a < nax; a += LJ) {
       C* row = A + a * LPA;
@@ -1144,28 +1121,40 @@ __global__ __launch_bounds__((Slab<R, N, true>::NT)) void k_slab_vmul(PwBatch B,
 }
 
 // ---------------------------------------------------------------- the same pass with a line per few lanes of one wavefront
-// N = R1 R1: the R1 threads of a line are the same in both stages, so a
-// wavefront that keeps whole lines (64 / R1 of them) needs no barrier between
-// the stages of a line: planes wid, wid + nw, ... (in groups of LPW) in A and
-// C, x lines likewise in B, each wavefront with its own lines of X.  Two
-// barriers per band (around B, where the axes change hands) instead of 16,
-// and every wavefront has work in every phase.
-// 144 lines of complex64: twelve wavefronts with 5 lines each; the sticks of
-// a thread's planes (at most two) stay in registers.  Pitch 156 of A and X:
-// the fewest LDS passes over all accesses of the kernel (593 against 744 for
-// 156 / 157, counted over 32 eight-byte banks).
-template <int N> struct Lines {
-  static constexpr int R1 = Split<N>::R1;
-  static_assert(R1 * R1 == N && R1 <= 16, "both stages of a line on the same threads");
-  static constexpr int RP = R1 | 1, L = R1 * RP, LPW = 64 / R1, NG = (N + LPW - 1) / LPW;
-  static constexpr int MAXW = 12, NP = 2;  // wavefronts; groups of planes per wavefront
-  template <typename R> static constexpr size_t lds(int nax_cap, int nw) {
+// A wavefront keeps whole lines: LPW = 64 / max(R1, R2) of them, max(R1, R2)
+// lanes each, so no barrier is needed between the stages of a line.  Planes
+// wid, wid + nw, ... (in groups of LPW) in A and C, x lines likewise in B, each
+// wavefront with its own lines of X.  Two barriers per band (around B, where
+// the axes change hands) instead of 16 at N = 144, and every wavefront has work
+// in every phase.  The sticks of a thread's planes (at most two) stay in registers.
+// 256 items, barrier kernel -> this one: 144^3 complex64 2114 -> 1570 us, 72^3
+// complex64 299 -> 211, 72^3 complex128 (64 items) 148 -> 121, 108^3 complex128
+// (100 items) 719 -> 661, complex64 374 -> 357.  At 32 the lines of a plane are
+// one round of the barrier kernel, which stays for it (64 items: 15.1 us in
+// complex128 and 11.4 in complex64 against 17.2 and 11.8).
+// Pitch of A and X at 144: 156, the fewest LDS passes over all accesses of the
+// kernel (593 against 744 for 156 / 157, counted over 32 eight-byte banks).
+template <typename R, int N> struct Lines {
+  static constexpr int R1 = Split<N>::R1, R2 = Split<N>::R2, RM = R1 > R2 ? R1 : R2;
+  static constexpr int R2P = R2 | 1, L = R1 * R2P, LPW = 64 / RM, NG = (N + LPW - 1) / LPW;
+  // wavefronts of a workgroup: four where several workgroups fit a CU (their
+  // wavefronts then spread evenly over the four SIMDs), else as many as fit.
+  // 64 bands at 72: complex64 66 us with four, 90 with six, 97 with five;
+  // complex128 121, 166, 175.  100 bands at 108: complex64 357 with four, 432
+  // with eight; complex128 661 with seven, 693 with six, 735 with four.
+  static constexpr bool kMany = N == 72 || (N == 108 && sizeof(R) == 4);
+  static constexpr int W = kMany ? 4 : (sizeof(R) == 8 ? 8 : 12);
+  static constexpr int MAXW = N == 72 ? 6 : (sizeof(R) == 8 ? 8 : 12);
+  static constexpr int MINW = sizeof(R) == 4 ? (N == 72 ? 4 : 3) : 2;  // wavefronts per SIMD
+  static constexpr int NP = 2;                                         // groups of planes per wavefront
+  static constexpr size_t lds(int nax_cap, int nw) {
     return sizeof(cx_t<R>) * ((size_t)nax_cap * L + (size_t)nw * LPW * L) + sizeof(int) * N;
   }
-  // wavefronts that the LDS holds and the planes need; 0: none
-  template <typename R> static int waves(int nax_cap) {
-    for (int nw = MAXW; nw * LPW * NP >= nax_cap; --nw)
-      if (lds<R>(nax_cap, nw) <= 160 * 1024) return nw;
+  // wavefronts that the planes need and the LDS holds; 0: none
+  static int waves(int nax_cap) {
+    const int need = (int)ceil_div(nax_cap, LPW * NP);
+    for (int nw = std::max(W, need); nw >= need && nw <= MAXW; --nw)
+      if (lds(nax_cap, nw) <= 160 * 1024) return nw;
     return 0;
   }
 };
@@ -1177,48 +1166,67 @@ __device__ __forceinline__ void line_fence() {
 }
 
 template <typename R, int N, bool Q>
-__global__ __launch_bounds__(64 * Lines<N>::MAXW) void k_slab_lines(PwBatch B, cx_t<R>* __restrict__ S, int nz, int bpw,
-                                                                  const cx_t<R>* __restrict__ tw,
-                                                                  const R* __restrict__ vt) {
+__global__ __launch_bounds__((64 * Lines<R, N>::MAXW), (Lines<R, N>::MINW)) void k_slab_lines(PwBatch B, cx_t<R>* __restrict__ S, int nz,
+                                                                        int bpw, const cx_t<R>* __restrict__ tw,
+                                                                        const R* __restrict__ vt) {
   using C = cx_t<R>;
-  using G = Lines<N>;
-  constexpr int R1 = G::R1, RP = G::RP, L = G::L, LPW = G::LPW, NP = G::NP;
+  using G = Lines<R, N>;
+  constexpr int R1 = G::R1, R2 = G::R2, RM = G::RM, R2P = G::R2P, L = G::L, LPW = G::LPW, NP = G::NP;
   extern __shared__ __align__(16) unsigned char smem[];
   const PwMaps m = B.mt[B.k0 + blockIdx.z];
-  const int z = blockIdx.x, grp = blockIdx.y, nw = blockDim.x >> 6, nax = m.nax;
+  // complex128 waits on its V rows: planes grouped per XCD (measured 4-5 %
+  // faster at 108^3; complex64 keeps the plane-fastest order, which measured
+  // 1-2 % faster for it)
+  int z = blockIdx.x, grp = blockIdx.y;
+  if constexpr (sizeof(R) == 8) xcd_task(z, grp);
+  const int nw = blockDim.x >> 6, nax = m.nax;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int l = lane / R1, d = lane % R1;  // line of the wavefront, digit
-  const bool on = l < LPW;
+  const int l = lane / RM, d = lane % RM;  // line of the wavefront; j2 or k1
+  const bool onj = l < LPW && d < R2, onk = l < LPW && d < R1;
   C* A = reinterpret_cast<C*>(smem);
-  C* X = A + (size_t)B.nax_cap * L + (size_t)(wid * LPW + (on ? l : 0)) * L;  // this thread's x line
+  C* X = A + (size_t)B.nax_cap * L + (size_t)(wid * LPW + (l < LPW ? l : 0)) * L;  // this thread's x line
   int* xa = reinterpret_cast<int*>(A + ((size_t)B.nax_cap + (size_t)nw * LPW) * L);
   for (int x = threadIdx.x; x < N; x += blockDim.x) xa[x] = -1;
-  auto has = [](int r) { return !Q || quarter_has(r, R1); };
-  // sticks y = d + R1 r of the thread's planes
-  uint32_t st[NP][R1];
+  auto in1 = [](int r) { return !Q || quarter_has(r, R1); };  // digits that the sphere can reach
+  auto in2 = [](int k) { return !Q || quarter_has(k, R2); };
+  auto pos = [](int y) { return (y % R1) * R2P + y / R1; };  // slot of index y
+  // sticks y = j2 + R2 r (read) and k1 + R1 k (written) of the thread's
+  // planes: the same ones when R1 = R2
+  uint32_t sa[NP][R1], sc[NP][R2];
   C* plane[NP];
-  bool pl[NP];
+  bool pj[NP], pk[NP];
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
     const int a = (wid + nw * p) * LPW + l;
-    pl[p] = on && a < nax;
-    plane[p] = A + (size_t)(pl[p] ? a : 0) * L;
+    pj[p] = onj && a < nax;
+    pk[p] = onk && a < nax;
+    plane[p] = A + (size_t)(pj[p] || pk[p] ? a : 0) * L;
+    const int* py = m.pl_y + (int64_t)a * N + d;
 #pragma unroll
     for (int r = 0; r < R1; ++r) {
-      const int q = pl[p] && has(r) ? m.pl_y[a * N + d + R1 * r] : -1;
-      st[p][r] = q >= 0 ? (uint32_t)q * (uint32_t)sizeof(C) : kOob;
+      const int q = pj[p] && in1(r) ? py[R2 * r] : -1;
+      sa[p][r] = q >= 0 ? (uint32_t)q * (uint32_t)sizeof(C) : kOob;
+    }
+#pragma unroll
+    for (int k = 0; k < R2; ++k) {
+      if constexpr (R1 == R2) {
+        sc[p][k] = sa[p][k];
+      } else {
+        const int q = pk[p] && in2(k) ? py[R1 * k] : -1;
+        sc[p][k] = q >= 0 ? (uint32_t)q * (uint32_t)sizeof(C) : kOob;
+      }
     }
   }
-  C tk[R1];
+  C tk[R2];
 #pragma unroll
-  for (int r = 1; r < R1; ++r) tk[r] = tw[(d * r) % N];
+  for (int r = 1; r < R2; ++r) tk[r] = tw[(d * r) % N];
   __syncthreads();
   for (int a = threadIdx.x; a < nax; a += blockDim.x) xa[m.ax_x[a]] = a;
   __syncthreads();
-  int xr[R1];  // rows of A of x = d + R1 r
+  int xr[R1];  // rows of A of x = j2 + R2 r
 #pragma unroll
   for (int r = 0; r < R1; ++r) {
-    const int a = xa[d + R1 * r];
+    const int a = onj ? xa[d + R2 * r] : -1;
     xr[r] = a >= 0 ? a * L : -1;
   }
   const R* vz = vt + (int64_t)z * N * N;  // V at (x, y, z) in vz[y*N + x]
@@ -1227,100 +1235,111 @@ __global__ __launch_bounds__(64 * Lines<N>::MAXW) void k_slab_lines(PwBatch B, c
   auto row_rsrc = [&](int band) {
     return buf_rsrc(S + (((int64_t)blockIdx.z * B.nbb + band) * nz + z) * B.nst_cap, row_bytes);
   };
+  // the next band's sticks are loaded during phase C where registers are free
+  constexpr bool kPre = Q && sizeof(R) == 4 && N == 144;
   C pre[NP][R1];
   auto load = [&](int band) {
     const auto rs = row_rsrc(band);
 #pragma unroll
     for (int p = 0; p < NP; ++p)
 #pragma unroll
-      for (int r = 0; r < R1; ++r) pre[p][r] = has(r) ? buf_ld<C>(rs, st[p][r]) : cmk<C>(0, 0);
+      for (int r = 0; r < R1; ++r) pre[p][r] = in1(r) ? buf_ld<C>(rs, sa[p][r]) : cmk<C>(0, 0);
   };
-  // slots: index d + R1 r of a line lies in slot d RP + r
-  if (Q) load(bb0);
+  if (kPre) load(bb0);
   for (int band = bb0; band < bb1; ++band) {
-    if (!Q) load(band);
+    if (!kPre) load(band);
     // A: y inverse of the wavefront's planes
 #pragma unroll
-    for (int p = 0; p < NP; ++p)
-      if (pl[p]) {
-        C* row = plane[p];
+    for (int p = 0; p < NP; ++p) {
+      if (pj[p]) {
         dftR<R1, +1>(pre[p], (const C*)nullptr, N);
+        C* row = plane[p] + d;
 #pragma unroll
-        for (int k = 0; k < R1; ++k) row[k * RP + d] = pre[p][k];
-        line_fence();
-        C u[R1];
-        row += d * RP;
-#pragma unroll
-        for (int r = 0; r < R1; ++r) u[r] = r ? cmul(row[r], cconj(tk[r])) : row[r];
-        dftR<R1, +1>(u, (const C*)nullptr, N);
-#pragma unroll
-        for (int k = 0; k < R1; ++k) row[k] = u[k];
+        for (int k = 0; k < R1; ++k) row[k * R2P] = pre[p][k];
       }
+      line_fence();
+      if (pk[p]) {
+        C u[R2];
+        C* row = plane[p] + d * R2P;
+#pragma unroll
+        for (int r = 0; r < R2; ++r) u[r] = r ? cmul(row[r], cconj(tk[r])) : row[r];
+        dftR<R2, +1>(u, (const C*)nullptr, N);
+#pragma unroll
+        for (int k = 0; k < R2; ++k) row[k] = u[k];
+      }
+    }
     __syncthreads();
     // B: x lines, inverse, * V / (nx ny nz), forward
 #pragma unroll 1
     for (int g = wid; g < G::NG; g += nw) {
-      const int y = g * LPW + l;
-      R vq[R1];  // V of the thread's points, used after the first two stages
+      const int y = g * LPW + l, py = pos(y);
+      R vq[R2];  // V of the thread's points, used after the first two stages
       const R* vy = vz + min(y, N - 1) * N + d;
 #pragma unroll
-      for (int k = 0; k < R1; ++k) vq[k] = vy[R1 * k];
-      if (on && y < N) {
-        const int py = (y % R1) * RP + y / R1;
+      for (int k = 0; k < R2; ++k) vq[k] = d < R1 ? vy[R1 * k] : R(0);
+      if (onj && y < N) {
         C v[R1];
 #pragma unroll
-        for (int r = 0; r < R1; ++r) v[r] = (has(r) && xr[r] >= 0) ? A[xr[r] + py] : cmk<C>(0, 0);
+        for (int r = 0; r < R1; ++r) v[r] = (in1(r) && xr[r] >= 0) ? A[xr[r] + py] : cmk<C>(0, 0);
         dftR<R1, +1>(v, (const C*)nullptr, N);
 #pragma unroll
-        for (int k = 0; k < R1; ++k) X[k * RP + d] = v[k];
-        line_fence();
-        C u[R1];
-        C* row = X + d * RP;
+        for (int k = 0; k < R1; ++k) X[k * R2P + d] = v[k];
+      }
+      line_fence();
+      if (onk && y < N) {
+        C u[R2];
+        C* row = X + d * R2P;
 #pragma unroll
-        for (int r = 0; r < R1; ++r) u[r] = r ? cmul(row[r], cconj(tk[r])) : row[r];
-        dftR<R1, +1>(u, (const C*)nullptr, N);
+        for (int r = 0; r < R2; ++r) u[r] = r ? cmul(row[r], cconj(tk[r])) : row[r];
+        dftR<R2, +1>(u, (const C*)nullptr, N);
 #pragma unroll
-        for (int k = 0; k < R1; ++k) u[k] = cscale(u[k], vq[k]);
-        dftR<R1, -1>(u, (const C*)nullptr, N);
+        for (int k = 0; k < R2; ++k) u[k] = cscale(u[k], vq[k]);
+        dftR<R2, -1>(u, (const C*)nullptr, N);
 #pragma unroll
-        for (int k = 0; k < R1; ++k) row[k] = k ? cmul(u[k], tk[k]) : u[k];
-        line_fence();
+        for (int k = 0; k < R2; ++k) row[k] = k ? cmul(u[k], tk[k]) : u[k];
+      }
+      line_fence();
+      if (onj && y < N) {
+        C v[R1];
 #pragma unroll
-        for (int j = 0; j < R1; ++j) v[j] = X[j * RP + d];
+        for (int j = 0; j < R1; ++j) v[j] = X[j * R2P + d];
         dftR<R1, -1>(v, (const C*)nullptr, N);
 #pragma unroll
         for (int k = 0; k < R1; ++k)
-          if (has(k) && xr[k] >= 0) A[xr[k] + py] = v[k];
-        line_fence();
+          if (in1(k) && xr[k] >= 0) A[xr[k] + py] = v[k];
       }
+      line_fence();
     }
     __syncthreads();
-    if (Q && band + 1 < bb1) load(band + 1);
+    if (kPre && band + 1 < bb1) load(band + 1);
     // C: y forward of the wavefront's planes, back to the sticks
     const auto rs = row_rsrc(band);
 #pragma unroll
-    for (int p = 0; p < NP; ++p)
-      if (pl[p]) {
-        C* row = plane[p];
+    for (int p = 0; p < NP; ++p) {
+      C* row = plane[p];
+      if (pj[p]) {
         C v[R1];
 #pragma unroll
-        for (int r = 0; r < R1; ++r) v[r] = row[d * RP + r];
+        for (int r = 0; r < R1; ++r) v[r] = row[pos(d + R2 * r)];
         dftR<R1, -1>(v, (const C*)nullptr, N);
 #pragma unroll
-        for (int k = 0; k < R1; ++k) row[d * RP + k] = v[k];
-        line_fence();
-        C u[R1];
+        for (int k = 0; k < R1; ++k) row[pos(d + R2 * k)] = v[k];
+      }
+      line_fence();
+      if (pk[p]) {
+        C u[R2];
 #pragma unroll
-        for (int j = 0; j < R1; ++j) {
-          const C w = row[j * RP + d];
+        for (int j = 0; j < R2; ++j) {
+          const C w = row[pos(j + R2 * d)];
           u[j] = j ? cmul(w, tk[j]) : w;
         }
-        dftR<R1, -1>(u, (const C*)nullptr, N);
+        dftR<R2, -1>(u, (const C*)nullptr, N);
 #pragma unroll
-        for (int k = 0; k < R1; ++k)
-          if (has(k)) buf_st<C>(rs, st[p][k], u[k]);
-        line_fence();
+        for (int k = 0; k < R2; ++k)
+          if (in2(k)) buf_st<C>(rs, sc[p][k], u[k]);
       }
+      line_fence();
+    }
   }
 }
 
@@ -1334,7 +1353,7 @@ __global__ __launch_bounds__((Slab<R, N>::NT)) void k_slab_density(PwBatch B, co
                                                                  const double* __restrict__ occ, int occ_ks,
                                                                  double* __restrict__ part) {
   using C = cx_t<R>;
-  using ST = SlabThread<R, N, false, Q>;
+  using ST = SlabThread<R, N, Q>;
   constexpr int R1 = ST::R1, R2 = ST::R2, LR = ST::LR, NR = Slab<R, N>::NR;
   extern __shared__ __align__(16) unsigned char smem[];
   const PwMaps m = B.mt[B.k0 + blockIdx.z];
@@ -1352,8 +1371,7 @@ __global__ __launch_bounds__((Slab<R, N>::NT)) void k_slab_density(PwBatch B, co
     const double w = occ[(int64_t)blockIdx.z * occ_ks + band];
     if (w == 0.0) continue;  // uniform over the workgroup
     const auto rs = buf_rsrc(S + (((int64_t)blockIdx.z * B.nbb + band) * nz + z) * B.nst_cap, row_bytes);
-    const C none[R1] = {};
-    t.template y_inverse<false>(rs, none);
+    t.y_inverse(rs);
 #pragma unroll
     for (int q = 0; q < NR; ++q) {
       const int y0 = q * LR, ln = min(LR, N - y0);
@@ -1412,7 +1430,7 @@ __global__ __launch_bounds__(256) void k_slab_rho_sum(const double* __restrict__
 
 // both fused kernels (H|psi> and density) fit the LDS for nax_cap planes
 template <typename R, int N> static bool slab_fits(int nax_cap) {
-  return Slab<R, N>::lds(nax_cap) <= 160 * 1024 && Slab<R, N, true>::lds(nax_cap) <= 160 * 1024;
+  return Slab<R, N>::lds(nax_cap) <= 160 * 1024 && (N == 32 || Lines<R, N>::waves(nax_cap) > 0);
 }
 
 template <typename R> bool slab_supported(int nx, int ny, int nz, int nax_cap, int nst_cap) {
@@ -1429,24 +1447,23 @@ template <typename R> bool slab_supported(int nx, int ny, int nz, int nax_cap, i
 
 template <typename R, int N>
 static void slab_vmul_n(const PwBatch& B, cx_t<R>* S, const Axis<R>* ax, int nz, const R* vt, int bpw, hipStream_t s) {
-  if constexpr (N == 144 && sizeof(R) == 4) {
-    using G = Lines<N>;
-    if (const int nw = G::template waves<R>(B.nax_cap)) {
-      const size_t lds = G::template lds<R>(B.nax_cap, nw);
-      auto kern = B.quarter ? k_slab_lines<R, N, true> : k_slab_lines<R, N, false>;
-      allow_lds_pw(kern, lds);
-      hipLaunchKernelGGL(kern, dim3((unsigned)nz, (unsigned)ceil_div(B.nbb, bpw), B.nkc), dim3(64 * nw), lds, s, B, S,
-                         nz, bpw, ax[0].tw, vt);
-      return;
-    }
+  const dim3 grid((unsigned)nz, (unsigned)ceil_div(B.nbb, bpw), B.nkc);
+  if constexpr (N == 32) {
+    using SL = Slab<R, N>;
+    const size_t lds = SL::lds(B.nax_cap);
+    check_lds_pw(lds, N);
+    auto kern = B.quarter ? k_slab_vmul<R, N, true> : k_slab_vmul<R, N, false>;
+    allow_lds_pw(kern, lds);
+    hipLaunchKernelGGL(kern, grid, dim3(SL::NT), lds, s, B, S, nz, bpw, ax[0].tw, vt);
+  } else {
+    using G = Lines<R, N>;
+    const int nw = G::waves(B.nax_cap);
+    DEREK_REQUIRE(nw > 0, "active planes do not fit the LDS");
+    const size_t lds = G::lds(B.nax_cap, nw);
+    auto kern = B.quarter ? k_slab_lines<R, N, true> : k_slab_lines<R, N, false>;
+    allow_lds_pw(kern, lds);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, B, S, nz, bpw, ax[0].tw, vt);
   }
-  using SL = Slab<R, N, true>;
-  const size_t lds = SL::lds(B.nax_cap);
-  check_lds_pw(lds, N);
-  auto kern = B.quarter ? k_slab_vmul<R, N, true> : k_slab_vmul<R, N, false>;
-  allow_lds_pw(kern, lds);
-  dim3 grid((unsigned)nz, (unsigned)ceil_div(B.nbb, bpw), B.nkc);
-  hipLaunchKernelGGL(kern, grid, dim3(SL::NT), lds, s, B, S, nz, bpw, ax[0].tw, vt);
 }
 
 template <typename R>
