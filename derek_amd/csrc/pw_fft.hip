@@ -1146,6 +1146,7 @@ template <typename R, int N> struct Lines {
   static constexpr int W = kMany ? 4 : (sizeof(R) == 8 ? 8 : 12);
   static constexpr int MAXW = N == 72 ? 6 : (sizeof(R) == 8 ? 8 : 12);
   static constexpr int MINW = sizeof(R) == 4 ? (N == 72 ? 4 : 3) : 2;  // wavefronts per SIMD
+  static constexpr int MIND = sizeof(R) == 4 && N == 72 ? 4 : 2;       // the same, density
   static constexpr int NP = 2;                                         // groups of planes per wavefront
   static constexpr size_t lds(int nax_cap, int nw) {
     return sizeof(cx_t<R>) * ((size_t)nax_cap * L + (size_t)nw * LPW * L) + sizeof(int) * N;
@@ -1165,13 +1166,110 @@ __device__ __forceinline__ void line_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-template <typename R, int N, bool Q>
-__global__ __launch_bounds__((64 * Lines<R, N>::MAXW), (Lines<R, N>::MINW)) void k_slab_lines(PwBatch B, cx_t<R>* __restrict__ S, int nz,
-                                                                        int bpw, const cx_t<R>* __restrict__ tw,
-                                                                        const R* __restrict__ vt) {
+// Per-thread state of the kernels below: the thread's digits (d = j2 in the
+// R2-lane stages, k1 in the R1-lane ones), planes, twiddles, sticks and rows of A.
+template <typename R, int N, bool Q> struct LineThread {
   using C = cx_t<R>;
   using G = Lines<R, N>;
-  constexpr int R1 = G::R1, R2 = G::R2, RM = G::RM, R2P = G::R2P, L = G::L, LPW = G::LPW, NP = G::NP;
+  static constexpr int R1 = G::R1, R2 = G::R2, RM = G::RM, R2P = G::R2P, L = G::L, LPW = G::LPW, NP = G::NP;
+  int nw, wid, l, d;    // wavefronts, this one, its line, digit
+  bool onj, onk;        // lane with work in the R2- / R1-lane stages
+  C *A, *X;             // planes; this thread's x line
+  uint32_t sa[NP][R1];  // sticks y = j2 + R2 r of the thread's planes
+  C* plane[NP];
+  bool pj[NP], pk[NP];
+  C tk[R2];
+  int xr[R1];  // rows of A of x = j2 + R2 r, -1 if inactive
+  // digits that the sphere can reach
+  __device__ static constexpr bool in1(int r) { return !Q || quarter_has(r, R1); }
+  __device__ static constexpr bool in2(int k) { return !Q || quarter_has(k, R2); }
+  __device__ static int pos(int y) { return (y % R1) * R2P + y / R1; }  // slot of index y
+  __device__ static uint32_t off(int q) { return q >= 0 ? (uint32_t)q * (uint32_t)sizeof(C) : kOob; }
+  __device__ __forceinline__ int plane_of(int p) const { return (wid + nw * p) * LPW + l; }
+
+  // two barriers
+  __device__ __forceinline__ void init(const PwBatch& B, const PwMaps& m, const C* __restrict__ tw,
+                                       unsigned char* smem) {
+    nw = blockDim.x >> 6;
+    wid = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, nax = m.nax;
+    l = lane / RM;
+    d = lane % RM;
+    onj = l < LPW && d < R2;
+    onk = l < LPW && d < R1;
+    A = reinterpret_cast<C*>(smem);
+    X = A + (size_t)B.nax_cap * L + (size_t)(wid * LPW + (l < LPW ? l : 0)) * L;
+    int* xa = reinterpret_cast<int*>(A + ((size_t)B.nax_cap + (size_t)nw * LPW) * L);
+    for (int x = threadIdx.x; x < N; x += blockDim.x) xa[x] = -1;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      const int a = plane_of(p);
+      pj[p] = onj && a < nax;
+      pk[p] = onk && a < nax;
+      plane[p] = A + (size_t)(pj[p] || pk[p] ? a : 0) * L;
+#pragma unroll
+      for (int r = 0; r < R1; ++r) sa[p][r] = off(pj[p] && in1(r) ? m.pl_y[a * N + d + R2 * r] : -1);
+    }
+#pragma unroll
+    for (int r = 1; r < R2; ++r) tk[r] = tw[(d * r) % N];
+    __syncthreads();
+    for (int a = threadIdx.x; a < nax; a += blockDim.x) xa[m.ax_x[a]] = a;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R1; ++r) {
+      const int a = onj ? xa[d + R2 * r] : -1;
+      xr[r] = a >= 0 ? a * L : -1;
+    }
+  }
+  // sticks of the thread's plane p
+  template <typename Rs> __device__ __forceinline__ void load(const Rs& rs, int p, C (&v)[R1]) const {
+#pragma unroll
+    for (int r = 0; r < R1; ++r) v[r] = in1(r) ? buf_ld<C>(rs, sa[p][r]) : cmk<C>(0, 0);
+  }
+  // A: y inverse of plane p
+  __device__ __forceinline__ void y_inverse(int p, C (&v)[R1]) {
+    if (pj[p]) {
+      dftR<R1, +1>(v, (const C*)nullptr, N);
+      C* row = plane[p] + d;
+#pragma unroll
+      for (int k = 0; k < R1; ++k) row[k * R2P] = v[k];
+    }
+    line_fence();
+    if (pk[p]) {
+      C u[R2];
+      C* row = plane[p] + d * R2P;
+      second(row, u);
+#pragma unroll
+      for (int k = 0; k < R2; ++k) row[k] = u[k];
+    }
+  }
+  // second inverse stage of a line from the R2 slots at row
+  __device__ __forceinline__ void second(const C* row, C* u) const {
+#pragma unroll
+    for (int r = 0; r < R2; ++r) u[r] = r ? cmul(row[r], cconj(tk[r])) : row[r];
+    dftR<R2, +1>(u, (const C*)nullptr, N);
+  }
+  // first inverse stage of x line y into X
+  __device__ __forceinline__ void x_inverse1(int y, int py) {
+    if (onj && y < N) {
+      C v[R1];
+#pragma unroll
+      for (int r = 0; r < R1; ++r) v[r] = (in1(r) && xr[r] >= 0) ? A[xr[r] + py] : cmk<C>(0, 0);
+      dftR<R1, +1>(v, (const C*)nullptr, N);
+#pragma unroll
+      for (int k = 0; k < R1; ++k) X[k * R2P + d] = v[k];
+    }
+    line_fence();
+  }
+};
+
+template <typename R, int N, bool Q>
+__global__ __launch_bounds__((64 * Lines<R, N>::MAXW), (Lines<R, N>::MINW)) void k_slab_lines(
+    PwBatch B, cx_t<R>* __restrict__ S, int nz, int bpw, const cx_t<R>* __restrict__ tw, const R* __restrict__ vt) {
+  using C = cx_t<R>;
+  using T = LineThread<R, N, Q>;
+  using G = Lines<R, N>;
+  constexpr int R1 = T::R1, R2 = T::R2, R2P = T::R2P, LPW = T::LPW, NP = T::NP;
   extern __shared__ __align__(16) unsigned char smem[];
   const PwMaps m = B.mt[B.k0 + blockIdx.z];
   // complex128 waits on its V rows: planes grouped per XCD (measured 4-5 %
@@ -1179,56 +1277,19 @@ __global__ __launch_bounds__((64 * Lines<R, N>::MAXW), (Lines<R, N>::MINW)) void
   // 1-2 % faster for it)
   int z = blockIdx.x, grp = blockIdx.y;
   if constexpr (sizeof(R) == 8) xcd_task(z, grp);
-  const int nw = blockDim.x >> 6, nax = m.nax;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int l = lane / RM, d = lane % RM;  // line of the wavefront; j2 or k1
-  const bool onj = l < LPW && d < R2, onk = l < LPW && d < R1;
-  C* A = reinterpret_cast<C*>(smem);
-  C* X = A + (size_t)B.nax_cap * L + (size_t)(wid * LPW + (l < LPW ? l : 0)) * L;  // this thread's x line
-  int* xa = reinterpret_cast<int*>(A + ((size_t)B.nax_cap + (size_t)nw * LPW) * L);
-  for (int x = threadIdx.x; x < N; x += blockDim.x) xa[x] = -1;
-  auto in1 = [](int r) { return !Q || quarter_has(r, R1); };  // digits that the sphere can reach
-  auto in2 = [](int k) { return !Q || quarter_has(k, R2); };
-  auto pos = [](int y) { return (y % R1) * R2P + y / R1; };  // slot of index y
-  // sticks y = j2 + R2 r (read) and k1 + R1 k (written) of the thread's
-  // planes: the same ones when R1 = R2
-  uint32_t sa[NP][R1], sc[NP][R2];
-  C* plane[NP];
-  bool pj[NP], pk[NP];
+  T t;
+  t.init(B, m, tw, smem);
+  const int d = t.d, nw = t.nw;
+  uint32_t sc[NP][R2];  // sticks y = k1 + R1 k, written: those read when R1 = R2
 #pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    const int a = (wid + nw * p) * LPW + l;
-    pj[p] = onj && a < nax;
-    pk[p] = onk && a < nax;
-    plane[p] = A + (size_t)(pj[p] || pk[p] ? a : 0) * L;
-    const int* py = m.pl_y + (int64_t)a * N + d;
-#pragma unroll
-    for (int r = 0; r < R1; ++r) {
-      const int q = pj[p] && in1(r) ? py[R2 * r] : -1;
-      sa[p][r] = q >= 0 ? (uint32_t)q * (uint32_t)sizeof(C) : kOob;
-    }
+  for (int p = 0; p < NP; ++p)
 #pragma unroll
     for (int k = 0; k < R2; ++k) {
-      if constexpr (R1 == R2) {
-        sc[p][k] = sa[p][k];
-      } else {
-        const int q = pk[p] && in2(k) ? py[R1 * k] : -1;
-        sc[p][k] = q >= 0 ? (uint32_t)q * (uint32_t)sizeof(C) : kOob;
-      }
+      if constexpr (R1 == R2)
+        sc[p][k] = t.sa[p][k];
+      else
+        sc[p][k] = T::off(t.pk[p] && T::in2(k) ? m.pl_y[t.plane_of(p) * N + d + R1 * k] : -1);
     }
-  }
-  C tk[R2];
-#pragma unroll
-  for (int r = 1; r < R2; ++r) tk[r] = tw[(d * r) % N];
-  __syncthreads();
-  for (int a = threadIdx.x; a < nax; a += blockDim.x) xa[m.ax_x[a]] = a;
-  __syncthreads();
-  int xr[R1];  // rows of A of x = j2 + R2 r
-#pragma unroll
-  for (int r = 0; r < R1; ++r) {
-    const int a = onj ? xa[d + R2 * r] : -1;
-    xr[r] = a >= 0 ? a * L : -1;
-  }
   const R* vz = vt + (int64_t)z * N * N;  // V at (x, y, z) in vz[y*N + x]
   const int bb0 = grp * bpw, bb1 = min(B.nbb, bb0 + bpw);
   const uint32_t row_bytes = (uint32_t)B.nst_cap * (uint32_t)sizeof(C);
@@ -1239,106 +1300,140 @@ __global__ __launch_bounds__((64 * Lines<R, N>::MAXW), (Lines<R, N>::MINW)) void
   constexpr bool kPre = Q && sizeof(R) == 4 && N == 144;
   C pre[NP][R1];
   auto load = [&](int band) {
-    const auto rs = row_rsrc(band);
 #pragma unroll
-    for (int p = 0; p < NP; ++p)
-#pragma unroll
-      for (int r = 0; r < R1; ++r) pre[p][r] = in1(r) ? buf_ld<C>(rs, sa[p][r]) : cmk<C>(0, 0);
+    for (int p = 0; p < NP; ++p) t.load(row_rsrc(band), p, pre[p]);
   };
   if (kPre) load(bb0);
   for (int band = bb0; band < bb1; ++band) {
+    const auto rs = row_rsrc(band);
     if (!kPre) load(band);
-    // A: y inverse of the wavefront's planes
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      if (pj[p]) {
-        dftR<R1, +1>(pre[p], (const C*)nullptr, N);
-        C* row = plane[p] + d;
-#pragma unroll
-        for (int k = 0; k < R1; ++k) row[k * R2P] = pre[p][k];
-      }
-      line_fence();
-      if (pk[p]) {
-        C u[R2];
-        C* row = plane[p] + d * R2P;
-#pragma unroll
-        for (int r = 0; r < R2; ++r) u[r] = r ? cmul(row[r], cconj(tk[r])) : row[r];
-        dftR<R2, +1>(u, (const C*)nullptr, N);
-#pragma unroll
-        for (int k = 0; k < R2; ++k) row[k] = u[k];
-      }
-    }
+    for (int p = 0; p < NP; ++p) t.y_inverse(p, pre[p]);
     __syncthreads();
     // B: x lines, inverse, * V / (nx ny nz), forward
 #pragma unroll 1
-    for (int g = wid; g < G::NG; g += nw) {
-      const int y = g * LPW + l, py = pos(y);
+    for (int g = t.wid; g < G::NG; g += nw) {
+      const int y = g * LPW + t.l, py = T::pos(y);
       R vq[R2];  // V of the thread's points, used after the first two stages
       const R* vy = vz + min(y, N - 1) * N + d;
 #pragma unroll
       for (int k = 0; k < R2; ++k) vq[k] = d < R1 ? vy[R1 * k] : R(0);
-      if (onj && y < N) {
-        C v[R1];
-#pragma unroll
-        for (int r = 0; r < R1; ++r) v[r] = (in1(r) && xr[r] >= 0) ? A[xr[r] + py] : cmk<C>(0, 0);
-        dftR<R1, +1>(v, (const C*)nullptr, N);
-#pragma unroll
-        for (int k = 0; k < R1; ++k) X[k * R2P + d] = v[k];
-      }
-      line_fence();
-      if (onk && y < N) {
+      t.x_inverse1(y, py);
+      if (t.onk && y < N) {
         C u[R2];
-        C* row = X + d * R2P;
-#pragma unroll
-        for (int r = 0; r < R2; ++r) u[r] = r ? cmul(row[r], cconj(tk[r])) : row[r];
-        dftR<R2, +1>(u, (const C*)nullptr, N);
+        C* row = t.X + d * R2P;
+        t.second(row, u);
 #pragma unroll
         for (int k = 0; k < R2; ++k) u[k] = cscale(u[k], vq[k]);
         dftR<R2, -1>(u, (const C*)nullptr, N);
 #pragma unroll
-        for (int k = 0; k < R2; ++k) row[k] = k ? cmul(u[k], tk[k]) : u[k];
+        for (int k = 0; k < R2; ++k) row[k] = k ? cmul(u[k], t.tk[k]) : u[k];
       }
       line_fence();
-      if (onj && y < N) {
+      if (t.onj && y < N) {
         C v[R1];
 #pragma unroll
-        for (int j = 0; j < R1; ++j) v[j] = X[j * R2P + d];
+        for (int j = 0; j < R1; ++j) v[j] = t.X[j * R2P + d];
         dftR<R1, -1>(v, (const C*)nullptr, N);
 #pragma unroll
         for (int k = 0; k < R1; ++k)
-          if (in1(k) && xr[k] >= 0) A[xr[k] + py] = v[k];
+          if (T::in1(k) && t.xr[k] >= 0) t.A[t.xr[k] + py] = v[k];
       }
       line_fence();
     }
     __syncthreads();
     if (kPre && band + 1 < bb1) load(band + 1);
     // C: y forward of the wavefront's planes, back to the sticks
-    const auto rs = row_rsrc(band);
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
-      C* row = plane[p];
-      if (pj[p]) {
+      C* row = t.plane[p];
+      if (t.pj[p]) {
         C v[R1];
 #pragma unroll
-        for (int r = 0; r < R1; ++r) v[r] = row[pos(d + R2 * r)];
+        for (int r = 0; r < R1; ++r) v[r] = row[T::pos(d + R2 * r)];
         dftR<R1, -1>(v, (const C*)nullptr, N);
 #pragma unroll
-        for (int k = 0; k < R1; ++k) row[pos(d + R2 * k)] = v[k];
+        for (int k = 0; k < R1; ++k) row[T::pos(d + R2 * k)] = v[k];
       }
       line_fence();
-      if (pk[p]) {
+      if (t.pk[p]) {
         C u[R2];
 #pragma unroll
         for (int j = 0; j < R2; ++j) {
-          const C w = row[pos(j + R2 * d)];
-          u[j] = j ? cmul(w, tk[j]) : w;
+          const C w = row[T::pos(j + R2 * d)];
+          u[j] = j ? cmul(w, t.tk[j]) : w;
         }
         dftR<R2, -1>(u, (const C*)nullptr, N);
 #pragma unroll
         for (int k = 0; k < R2; ++k)
-          if (in2(k)) buf_st<C>(rs, sc[p][k], u[k]);
+          if (T::in2(k)) buf_st<C>(rs, sc[p][k], u[k]);
       }
       line_fence();
+    }
+  }
+}
+
+// k_slab_density with whole lines per wavefront: NW wavefronts, the FP64 sums of
+// a thread's points (NR lines of R2) in registers.  Two barriers per band.
+// Barrier kernel -> this one: 144^3 complex64 1350 -> 926 us a launch, 72^3
+// complex64 187 -> 141; 64 bands on 72^3 complex128 135 -> 95, 100 bands on
+// 108^3 complex64 434 -> 316.
+template <typename R, int N, bool Q, int NW>
+__global__ __launch_bounds__((64 * NW), (Lines<R, N>::MIND)) void k_slab_lines_density(
+    PwBatch B, const cx_t<R>* __restrict__ S, int nz, int bpg, const cx_t<R>* __restrict__ tw,
+    const double* __restrict__ occ, int occ_ks, double* __restrict__ part) {
+  using C = cx_t<R>;
+  using T = LineThread<R, N, Q>;
+  using G = Lines<R, N>;
+  constexpr int R1 = T::R1, R2 = T::R2, R2P = T::R2P, LPW = T::LPW, NP = T::NP, NR = (G::NG + NW - 1) / NW;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const PwMaps m = B.mt[B.k0 + blockIdx.z];
+  const int z = blockIdx.x;
+  T t;
+  t.init(B, m, tw, smem);
+  const int d = t.d;
+  double acc[NR][R2];
+#pragma unroll
+  for (int q = 0; q < NR; ++q)
+#pragma unroll
+    for (int k = 0; k < R2; ++k) acc[q][k] = 0.0;
+  const int bb0 = blockIdx.y * bpg, bb1 = min(B.nbb, bb0 + bpg);
+  const uint32_t row_bytes = (uint32_t)B.nst_cap * (uint32_t)sizeof(C);
+  for (int band = bb0; band < bb1; ++band) {
+    const double w = occ[(int64_t)blockIdx.z * occ_ks + band];
+    if (w == 0.0) continue;  // uniform over the workgroup
+    const auto rs = buf_rsrc(S + (((int64_t)blockIdx.z * B.nbb + band) * nz + z) * B.nst_cap, row_bytes);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+      C v[R1];
+      t.load(rs, p, v);
+      t.y_inverse(p, v);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      const int y = (t.wid + NW * q) * LPW + t.l;
+      t.x_inverse1(y, T::pos(y));
+      if (t.onk && y < N) {
+        C u[R2];
+        t.second(t.X + d * R2P, u);
+#pragma unroll
+        for (int k = 0; k < R2; ++k) {
+          const double re = (double)u[k].x, im = (double)u[k].y;
+          acc[q][k] += w * (re * re + im * im);
+        }
+      }
+      line_fence();
+    }
+    __syncthreads();
+  }
+  double* pz = part + ((int64_t)(blockIdx.z * gridDim.y + blockIdx.y) * nz + z) * N * N;
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    const int y = (t.wid + NW * q) * LPW + t.l;
+    if (t.onk && y < N) {
+#pragma unroll
+      for (int k = 0; k < R2; ++k) pz[(int64_t)y * N + d + R1 * k] = acc[q][k];
     }
   }
 }
@@ -1482,6 +1577,32 @@ void slab_vmul(const PwBatch& B, cx_t<R>* S, const Axis<R>* ax, int nz, const R*
   DEREK_HIP(hipGetLastError());
 }
 
+// The density kernel of a batch: whole lines per wavefront where its planes and
+// lines fit, the barrier kernel for more planes, at 32 (one round of lines) and
+// for complex128 at 108 (its sums leave room for seven wavefronts only: 323 us
+// against 319 for 160 bands).
+template <typename R> struct DensityKernel {
+  void (*kern)(PwBatch, const cx_t<R>*, int, int, const cx_t<R>*, const double*, int, double*);
+  int nt;
+  size_t lds;
+};
+template <typename R, int N> static DensityKernel<R> density_kernel(const PwBatch& B) {
+  DensityKernel<R> k{nullptr, 0, 0};
+  if constexpr (N > 32 && !(N == 108 && sizeof(R) == 8)) {
+    using G = Lines<R, N>;
+    constexpr int NW = N == 72 ? 4 : (N == 108 ? 8 : 12);
+    k = {B.quarter ? k_slab_lines_density<R, N, true, NW> : k_slab_lines_density<R, N, false, NW>, 64 * NW,
+         G::lds(B.nax_cap, NW)};
+    if (B.nax_cap > NW * G::LPW * G::NP || k.lds > 160 * 1024) k.kern = nullptr;
+  }
+  if (!k.kern)
+    k = {B.quarter ? k_slab_density<R, N, true> : k_slab_density<R, N, false>, Slab<R, N>::NT,
+         Slab<R, N>::lds(B.nax_cap)};
+  check_lds_pw(k.lds, N);
+  allow_lds_pw(k.kern, k.lds);
+  return k;
+}
+
 template <typename R, int N> static int slab_density_groups_n(const PwBatch& B, int nz) {
   static const int cus = [] {
     int dev = 0;
@@ -1490,11 +1611,9 @@ template <typename R, int N> static int slab_density_groups_n(const PwBatch& B, 
     DEREK_HIP(hipGetDeviceProperties(&p, dev));
     return std::max(1, p.multiProcessorCount);
   }();
-  const size_t lds = Slab<R, N>::lds(B.nax_cap);
-  auto kern = B.quarter ? k_slab_density<R, N, true> : k_slab_density<R, N, false>;
-  allow_lds_pw(kern, lds);
+  const auto k = density_kernel<R, N>(B);
   int per = 0;
-  DEREK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(kern), Slab<R, N>::NT, lds));
+  DEREK_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(k.kern), k.nt, k.lds));
   // about four rounds of resident workgroups
   const int64_t want = 4LL * std::max(1, per) * cus;
   const int64_t g = (want + (int64_t)nz * B.nkc - 1) / ((int64_t)nz * B.nkc);
@@ -1521,13 +1640,9 @@ template <typename R> int slab_density_groups(const PwBatch& B, const Axis<R>* a
 template <typename R, int N>
 static void slab_density_n(const PwBatch& B, const cx_t<R>* S, const Axis<R>* ax, int nz, const double* occ, int occ_ks,
                            double* part, int groups, hipStream_t s) {
-  using SL = Slab<R, N>;
-  const size_t lds = SL::lds(B.nax_cap);
-  check_lds_pw(lds, N);
-  auto kern = B.quarter ? k_slab_density<R, N, true> : k_slab_density<R, N, false>;
-  allow_lds_pw(kern, lds);
+  const auto k = density_kernel<R, N>(B);
   dim3 grid((unsigned)nz, (unsigned)groups, B.nkc);
-  hipLaunchKernelGGL(kern, grid, dim3(SL::NT), lds, s, B, S, nz, (int)ceil_div(B.nbb, groups), ax[0].tw, occ, occ_ks,
+  hipLaunchKernelGGL(k.kern, grid, dim3(k.nt), k.lds, s, B, S, nz, (int)ceil_div(B.nbb, groups), ax[0].tw, occ, occ_ks,
                      part);
 }
 

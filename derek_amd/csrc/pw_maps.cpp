@@ -23,14 +23,15 @@ PwMapsHost build_pw_maps(const int32_t* idx, int64_t npw, int nx, int ny, int nz
   h.pw_st.resize(npw);
   const int64_t nyz = (int64_t)ny * nz;
   int64_t prev_col = -1, prev_x = -1;
+  auto outer = [](int64_t b, int64_t n) { return 4 * b < n || 4 * b >= 3 * n; };
   for (int64_t p = 0; p < npw; ++p) {
     const int64_t f = idx[ord[p]];
     const int64_t col = f / nz;  // x*ny + y
-    const int64_t x = f / nyz;
-    h.pw_z[p] = (int32_t)(f % nz);
-    auto outer = [](int64_t b, int64_t n) { return 4 * b < n || 4 * b >= 3 * n; };
-    h.quarter = h.quarter && outer(x, nx) && outer(col % ny, ny) && outer(f % nz, nz);
+    h.pw_z[p] = (int32_t)(f - col * nz);
+    h.quarter = h.quarter && outer(h.pw_z[p], nz);
     if (col != prev_col) {
+      const int64_t x = f / nyz;
+      h.quarter = h.quarter && outer(x, nx) && outer(col - x * ny, ny);
       if (x != prev_x) {
         h.pl_st.push_back(h.nst);
         h.ax_x.push_back((int32_t)x);
@@ -38,7 +39,7 @@ PwMapsHost build_pw_maps(const int32_t* idx, int64_t npw, int nx, int ny, int nz
         prev_x = x;
       }
       h.st_pw.push_back((int32_t)p);
-      h.st_y.push_back((int32_t)(col % ny));
+      h.st_y.push_back((int32_t)(col - x * ny));
       h.nst += 1;
       prev_col = col;
     }
