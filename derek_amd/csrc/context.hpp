@@ -214,6 +214,7 @@ struct derek_ctx {
   template <typename R> void fft3d(derek::cx_t<R>* g, int howmany, int dir);
   // Grid operations on device buffers (FP64); energies land in rep[slot]
   // when rep is given (no host synchronisation).
+  void filtered(const double* in, double* out, const derek::GFilter& filter);
   void hartree(const double* rho, double* vh_out, double* rep, int slot);
   void lda(const double* rho, double* vxc_out, double* rep, int slot);
   void dot_into(const double* a, const double* b, int64_t n, double scale, bool root, double* rep, int slot);

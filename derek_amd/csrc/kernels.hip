@@ -10,10 +10,12 @@ constexpr int NT = 256;          // threads per workgroup for the FFT passes
 constexpr int TILE_LINES = 16;   // z columns per strided-axis tile
 
 // ------------------------------------------------------------------ FFT kernels
-// Contiguous lines (z axis).  Each workgroup owns `lpb` lines.
-template <typename Rl, int S, int NC>
+// Contiguous lines (z axis).  Each workgroup owns `lpb` lines.  IO 1: the input
+// is the real field rin; 2: only the real part is kept, in rout.
+template <typename Rl, int S, int NC, int IO>
 __global__ __launch_bounds__(NT) void k_fft_contig(cx_t<Rl>* __restrict__ data, int64_t nlines, int lpb,
-                                                   FftPlan plan, const cx_t<Rl>* __restrict__ tw) {
+                                                   FftPlan plan, const cx_t<Rl>* __restrict__ tw,
+                                                   const Rl* __restrict__ rin, Rl* __restrict__ rout) {
   using C = cx_t<Rl>;
   extern __shared__ __align__(16) unsigned char smem[];
   const int N = NC > 0 ? NC : plan.n;
@@ -29,21 +31,30 @@ __global__ __launch_bounds__(NT) void k_fft_contig(cx_t<Rl>* __restrict__ data, 
   const int ne = lines * N;
   for (int e = threadIdx.x; e < ne; e += NT) {
     const int line = e / N;
-    b0[line * ls + (e - line * N)] = src[e];
+    if constexpr (IO == 1)
+      b0[line * ls + (e - line * N)] = cmk<C>(rin[line0 * N + e], 0);
+    else
+      b0[line * ls + (e - line * N)] = src[e];
   }
   __syncthreads();
   C* res = fft_lds<S, false, 1, NT, NC>(b0, b1, twl, plan, lines);
   C* dst = data + line0 * N;
   for (int e = threadIdx.x; e < ne; e += NT) {
     const int line = e / N;
-    dst[e] = res[line * ls + (e - line * N)];
+    const C v = res[line * ls + (e - line * N)];
+    if constexpr (IO == 2)
+      rout[line0 * N + e] = v.x;
+    else
+      dst[e] = v;
   }
 }
 
-// Strided axis, tiles of TILE_LINES neighbouring inner indices.
-template <typename Rl, int S, int NC>
+// Strided axis, tiles of TILE_LINES neighbouring inner indices.  FILTER: the
+// last axis of a forward transform and the first of the inverse one, with the
+// field multiplied by the filter in between (S = -1).
+template <typename Rl, int S, int NC, bool FILTER>
 __global__ __launch_bounds__(NT) void k_fft_tile(cx_t<Rl>* __restrict__ data, int64_t stride, int64_t tiles,
-                                                 FftPlan plan, const cx_t<Rl>* __restrict__ tw) {
+                                                 FftPlan plan, const cx_t<Rl>* __restrict__ tw, GFilter filter) {
   using C = cx_t<Rl>;
   extern __shared__ __align__(16) unsigned char smem[];
   const int N = NC > 0 ? NC : plan.n;
@@ -63,6 +74,14 @@ __global__ __launch_bounds__(NT) void k_fft_tile(cx_t<Rl>* __restrict__ data, in
   }
   __syncthreads();
   C* res = fft_lds<S, true, TILE_LINES, NT, NC>(b0, b1, twl, plan, TILE_LINES);
+  if constexpr (FILTER) {
+    for (int e = threadIdx.x; e < ne; e += NT) {
+      const int a = e / TILE_LINES, l = e - a * TILE_LINES;
+      if (l < lines) res[e] = cscale(res[e], (Rl)filter(o * (int64_t)N * stride + (int64_t)a * stride + i0 + l));
+    }
+    __syncthreads();
+    res = fft_lds<+1, true, TILE_LINES, NT, NC>(res, res == b0 ? b1 : b0, twl, plan, TILE_LINES);
+  }
   for (int e = threadIdx.x; e < ne; e += NT) {
     const int a = e / TILE_LINES, l = e - a * TILE_LINES;
     if (l < lines) base[(int64_t)a * stride + l] = res[e];
@@ -89,29 +108,33 @@ static void check_lds(size_t bytes, int n) {
   DEREK_REQUIRE(bytes <= 160 * 1024, "FFT length " + std::to_string(n) + " exceeds the LDS budget");
 }
 
-template <typename Rl, int S, int NC>
-static void launch_contig(cx_t<Rl>* data, int64_t nlines, const Axis<Rl>& ax, hipStream_t s) {
+template <typename Rl, int S, int NC, int IO = 0>
+static void launch_contig(cx_t<Rl>* data, int64_t nlines, const Axis<Rl>& ax, hipStream_t s, const Rl* rin = nullptr,
+                          Rl* rout = nullptr) {
   const int N = ax.n;
   int lpb = 1024 / N;
   if (lpb < 1) lpb = 1;
   const size_t lds = sizeof(cx_t<Rl>) * ((size_t)N + 2 * (size_t)lpb * contig_stride(N));
   check_lds(lds, N);
-  auto kern = k_fft_contig<Rl, S, NC>;
+  auto kern = k_fft_contig<Rl, S, NC, IO>;
   allow_lds(kern, lds);
   const int64_t blocks = ceil_div(nlines, lpb);
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NT), lds, s, data, nlines, lpb, ax.plan, ax.tw);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(NT), lds, s, data, nlines, lpb, ax.plan, ax.tw, rin,
+                     rout);
   DEREK_HIP(hipGetLastError());
 }
 
-template <typename Rl, int S, int NC>
-static void launch_tile(cx_t<Rl>* data, int64_t nouter, int64_t stride, const Axis<Rl>& ax, hipStream_t s) {
+template <typename Rl, int S, int NC, bool FILTER = false>
+static void launch_tile(cx_t<Rl>* data, int64_t nouter, int64_t stride, const Axis<Rl>& ax, hipStream_t s,
+                        const GFilter& filter = {}) {
   const int N = ax.n;
   const size_t lds = sizeof(cx_t<Rl>) * ((size_t)N + 2 * (size_t)TILE_LINES * N);
   check_lds(lds, N);
-  auto kern = k_fft_tile<Rl, S, NC>;
+  auto kern = k_fft_tile<Rl, S, NC, FILTER>;
   allow_lds(kern, lds);
   const int64_t tiles = ceil_div(stride, TILE_LINES);
-  hipLaunchKernelGGL(kern, dim3((unsigned)(nouter * tiles)), dim3(NT), lds, s, data, stride, tiles, ax.plan, ax.tw);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(nouter * tiles)), dim3(NT), lds, s, data, stride, tiles, ax.plan, ax.tw,
+                     filter);
   DEREK_HIP(hipGetLastError());
 }
 
@@ -149,6 +172,24 @@ void fft_strided(cx_t<R>* data, int64_t nouter, int64_t stride, const Axis<R>& a
     DEREK_FFT_DISPATCH(ax.n, C_)
 #undef C_
   }
+}
+
+void fft_z_from_real(const double* in, double2* g, int64_t nlines, const Axis<double>& ax, hipStream_t s) {
+#define C_(NC) launch_contig<double, -1, NC, 1>(g, nlines, ax, s, in)
+  DEREK_FFT_DISPATCH(ax.n, C_)
+#undef C_
+}
+
+void fft_z_to_real(double2* g, double* out, int64_t nlines, const Axis<double>& ax, hipStream_t s) {
+#define C_(NC) launch_contig<double, +1, NC, 2>(g, nlines, ax, s, nullptr, out)
+  DEREK_FFT_DISPATCH(ax.n, C_)
+#undef C_
+}
+
+void fft_filter(double2* g, int64_t stride, const Axis<double>& ax, const GFilter& filter, hipStream_t s) {
+#define C_(NC) launch_tile<double, -1, NC, true>(g, 1, stride, ax, s, filter)
+  DEREK_FFT_DISPATCH(ax.n, C_)
+#undef C_
 }
 
 template void fft_z<double>(double2*, int64_t, const Axis<double>&, int, hipStream_t);
@@ -252,39 +293,6 @@ __global__ void k_lda_eps(const double* __restrict__ rho, double* __restrict__ e
 }
 void lda_eps(const double* rho, double* eps, int64_t n, hipStream_t s) {
   hipLaunchKernelGGL(k_lda_eps, dim3(grid1d(n)), dim3(256), 0, s, rho, eps, n);
-  DEREK_HIP(hipGetLastError());
-}
-
-__global__ void k_real_to_cx(const double* __restrict__ in, double2* __restrict__ out, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    out[i] = make_double2(in[i], 0.0);
-}
-void real_to_cx(const double* in, double2* out, int64_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_real_to_cx, dim3(grid1d(n)), dim3(256), 0, s, in, out, n);
-  DEREK_HIP(hipGetLastError());
-}
-
-__global__ void k_cx_real(const double2* __restrict__ in, double* __restrict__ out, double scale, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    out[i] = in[i].x * scale;
-}
-void cx_real(const double2* in, double* out, double scale, int64_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_cx_real, dim3(grid1d(n)), dim3(256), 0, s, in, out, scale, n);
-  DEREK_HIP(hipGetLastError());
-}
-
-__global__ void k_gspace_scale(double2* __restrict__ g, const double* __restrict__ gsq, double q0sq, double scale,
-                               int mode, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const double q = gsq[i];
-    double f;
-    if (mode == 0) f = q > 0.0 ? 4.0 * 3.141592653589793238462643383279502884197 / q * scale : 0.0;
-    else f = q > 0.0 ? q / (q + q0sq) * scale : 0.0;
-    g[i] = make_double2(g[i].x * f, g[i].y * f);
-  }
-}
-void gspace_scale(double2* g, const double* gsq, double q0sq, double scale, int mode, int64_t n, hipStream_t s) {
-  hipLaunchKernelGGL(k_gspace_scale, dim3(grid1d(n)), dim3(256), 0, s, g, gsq, q0sq, scale, mode, n);
   DEREK_HIP(hipGetLastError());
 }
 

@@ -28,17 +28,32 @@ template <typename R> void fft_z(cx_t<R>* data, int64_t nlines, const Axis<R>& a
 // Strided axis: element (o, a, i) at o*n*stride + a*stride + i, i < stride.
 template <typename R>
 void fft_strided(cx_t<R>* data, int64_t nouter, int64_t stride, const Axis<R>& ax, int sign, hipStream_t s);
+// What a G-space field is multiplied with: 4 pi / G^2 (0 at G = 0) or the Kerker
+// factor G^2 / (G^2 + q0^2).
+struct GFilter {
+  const double* gsq;
+  double q0sq, scale;
+  int kerker;
+  __device__ double operator()(int64_t i) const {
+    const double q = gsq[i];
+    if (!(q > 0.0)) return 0.0;
+    return kerker ? q / (q + q0sq) * scale : 4.0 * 3.141592653589793238462643383279502884197 / q * scale;
+  }
+};
+
+// The z pass of a forward transform from a real field, and of an inverse one
+// that keeps the real part.
+void fft_z_from_real(const double* in, double2* g, int64_t nlines, const Axis<double>& ax, hipStream_t s);
+void fft_z_to_real(double2* g, double* out, int64_t nlines, const Axis<double>& ax, hipStream_t s);
+// The outermost axis forward, times the filter, and back (element (a, i) at
+// a*stride + i, i < stride).
+void fft_filter(double2* g, int64_t stride, const Axis<double>& ax, const GFilter& filter, hipStream_t s);
 // ---- buffers
 template <typename R> void zero(cx_t<R>* p, int64_t n, hipStream_t s);
 // ---- real-space fields (FP64)
 void lda_xc(const double* rho, double* vxc, double* partial_exc, int64_t n, hipStream_t s);
 int lda_partials(int64_t n);
 void lda_eps(const double* rho, double* eps, int64_t n, hipStream_t s);
-void real_to_cx(const double* in, double2* out, int64_t n, hipStream_t s);
-void cx_real(const double2* in, double* out, double scale, int64_t n, hipStream_t s);
-// g(G) *= fac(|G|^2): mode 0 Hartree 4*pi/G^2 * scale (G=0 -> 0);
-// mode 1 Kerker G^2/(G^2+q0sq) * scale.
-void gspace_scale(double2* g, const double* gsq, double q0sq, double scale, int mode, int64_t n, hipStream_t s);
 // out = a + b + c (any may be null -> 0)
 void add3(const double* a, const double* b, const double* c, double* out, int64_t n, hipStream_t s);
 // partial dot products: partial[blk] = sum a*b over the block's slice
