@@ -877,8 +877,8 @@ void planes_x_density(const PwBatch& B, const cx_t<R>* P, const Axis<R>* ax, int
 //   B  x lines in rounds of LR: inverse transform of the active rows,
 //      * V(x, y, z) / (nx ny nz), forward transform, active rows back into A;
 //   C  y forward of each active plane, stick rows written back.
-// (k_slab_vmul at N = 32 and k_slab_density; k_slab_lines below is the pass of
-// H|psi> at the other lengths.)
+// (k_slab_vmul and k_slab_density; k_slab_lines below is the pass of H|psi> of
+// most lengths, see kSlabBarrier.)
 // Each length-N transform is two register stages, N = R1 R2: R2 threads
 // (digit j2) take R1-point DFTs over the inputs j2 + R2 r, R1 threads (digit
 // k1) finish with R2-point DFTs; the result with index k1 + R1 k2 sits in
@@ -1129,9 +1129,10 @@ __global__ __launch_bounds__((Slab<R, N>::NT)) void k_slab_vmul(PwBatch B, cx_t<
 // in every phase.  The sticks of a thread's planes (at most two) stay in registers.
 // 256 items, barrier kernel -> this one: 144^3 complex64 2114 -> 1570 us, 72^3
 // complex64 299 -> 211, 72^3 complex128 (64 items) 148 -> 121, 108^3 complex128
-// (100 items) 719 -> 661, complex64 374 -> 357.  At 32 the lines of a plane are
-// one round of the barrier kernel, which stays for it (64 items: 15.1 us in
-// complex128 and 11.4 in complex64 against 17.2 and 11.8).
+// (100 items) 719 -> 661.  The barrier kernel stays at 32, where the lines of a
+// plane are one round of it (64 items: 15.1 us in complex128 and 11.4 in
+// complex64 against 17.2 and 11.8), and for complex64 at 108, where two of its
+// workgroups fit a CU (100 items: 374 us against 415 with twelve wavefronts).
 // Pitch of A and X at 144: 156, the fewest LDS passes over all accesses of the
 // kernel (593 against 744 for 156 / 157, counted over 32 eight-byte banks).
 template <typename R, int N> struct Lines {
@@ -1140,10 +1141,9 @@ template <typename R, int N> struct Lines {
   // wavefronts of a workgroup: four where several workgroups fit a CU (their
   // wavefronts then spread evenly over the four SIMDs), else as many as fit.
   // 64 bands at 72: complex64 66 us with four, 90 with six, 97 with five;
-  // complex128 121, 166, 175.  100 bands at 108: complex64 357 with four, 432
-  // with eight; complex128 661 with seven, 693 with six, 735 with four.
-  static constexpr bool kMany = N == 72 || (N == 108 && sizeof(R) == 4);
-  static constexpr int W = kMany ? 4 : (sizeof(R) == 8 ? 8 : 12);
+  // complex128 121, 166, 175.  100 bands of complex128 at 108: 661 with seven,
+  // 693 with six.
+  static constexpr int W = N == 72 ? 4 : (sizeof(R) == 8 ? 8 : 12);
   static constexpr int MAXW = N == 72 ? 6 : (sizeof(R) == 8 ? 8 : 12);
   static constexpr int MINW = sizeof(R) == 4 ? (N == 72 ? 4 : 3) : 2;  // wavefronts per SIMD
   static constexpr int MIND = sizeof(R) == 4 && N == 72 ? 4 : 2;       // the same, density
@@ -1159,6 +1159,9 @@ template <typename R, int N> struct Lines {
     return 0;
   }
 };
+
+// lengths whose H|psi> pass is the barrier kernel (both measured above)
+template <typename R, int N> constexpr bool kSlabBarrier = N == 32 || (N == 108 && sizeof(R) == 4);
 
 // LDS accesses of one wavefront on lines of its own stay in program order
 __device__ __forceinline__ void line_fence() {
@@ -1525,7 +1528,7 @@ __global__ __launch_bounds__(256) void k_slab_rho_sum(const double* __restrict__
 
 // both fused kernels (H|psi> and density) fit the LDS for nax_cap planes
 template <typename R, int N> static bool slab_fits(int nax_cap) {
-  return Slab<R, N>::lds(nax_cap) <= 160 * 1024 && (N == 32 || Lines<R, N>::waves(nax_cap) > 0);
+  return Slab<R, N>::lds(nax_cap) <= 160 * 1024 && (kSlabBarrier<R, N> || Lines<R, N>::waves(nax_cap) > 0);
 }
 
 template <typename R> bool slab_supported(int nx, int ny, int nz, int nax_cap, int nst_cap) {
@@ -1543,7 +1546,7 @@ template <typename R> bool slab_supported(int nx, int ny, int nz, int nax_cap, i
 template <typename R, int N>
 static void slab_vmul_n(const PwBatch& B, cx_t<R>* S, const Axis<R>* ax, int nz, const R* vt, int bpw, hipStream_t s) {
   const dim3 grid((unsigned)nz, (unsigned)ceil_div(B.nbb, bpw), B.nkc);
-  if constexpr (N == 32) {
+  if constexpr (kSlabBarrier<R, N>) {
     using SL = Slab<R, N>;
     const size_t lds = SL::lds(B.nax_cap);
     check_lds_pw(lds, N);
