@@ -889,7 +889,9 @@ void planes_x_density(const PwBatch& B, const cx_t<R>* P, const Axis<R>* ax, int
 // x rows in registers for the whole launch.  Compared with the separate y and
 // x passes the active planes stay on chip: HBM sees the stick rows once each
 // way and V once per band group.
-template <typename R, int N> struct Slab {
+// VM: parameters of k_slab_vmul (false: k_slab_density, whose FP64
+// accumulators need more registers per thread)
+template <typename R, int N, bool VM = false> struct Slab {
   static constexpr int R1 = Split<N>::R1, R2 = Split<N>::R2;
   static constexpr int R2P = R2 % 2 ? R2 : R2 + 1;
   static constexpr int L = R1 * R2P;              // slots of a line
@@ -909,11 +911,14 @@ template <typename R, int N> struct Slab {
   // 360 threads at N = 72 (not 288): the R1- and R2-thread stages then take
   // 40 and 45 planes per pass, so the 33 active planes of a 16 bohr cell at
   // Ecut 20 Ha need one pass per y stage instead of two
-  static constexpr int NT = N == 32 ? 256 : (N == 72 ? 360 : 504);
+  // FP64 H|psi> at 72 runs 720 threads with all 72 x lines in one round
+  // (7 barrier phases per band instead of 13; one 136 KB workgroup per CU)
+  static constexpr bool kWide72 = VM && N == 72 && sizeof(R) == 8;
+  static constexpr int NT = N == 32 ? 256 : (N == 72 ? (kWide72 ? 720 : 360) : 504);
   // x lines per round: the complex64 108 case is sized for two workgroups per
   // CU; complex64 at 72 takes the 72 lines in two rounds
   static constexpr int LR =
-      N == 32 ? 32 : (N == 72 ? (sizeof(R) == 4 ? 36 : 24) : (N == 108 && sizeof(R) == 4 ? 27 : 36));
+      N == 32 ? 32 : (N == 72 ? (kWide72 ? 72 : (sizeof(R) == 4 ? 36 : 24)) : (N == 108 && sizeof(R) == 4 ? 27 : 36));
   static constexpr int NR = (N + LR - 1) / LR;
   static constexpr int LJ = NT / R2, LK = NT / R1;  // lines per pass of the R2- / R1-thread stages
   static_assert(NT % R1 == 0 && NT % R2 == 0, "workgroup size must keep each thread's digits");
@@ -930,9 +935,9 @@ template <typename R, int N> struct Slab {
 // (j2 in the R2-thread stages, k1 in the R1-thread stages, and its line in
 // each), its twiddles exp(-2 pi i k1 r / N) and the LDS rows of the active
 // planes at x = j2 + R2 r (-1 if none).
-template <typename R, int N, bool Q> struct SlabThread {
+template <typename R, int N, bool VM, bool Q> struct SlabThread {
   using C = cx_t<R>;
-  using SL = Slab<R, N>;
+  using SL = Slab<R, N, VM>;
   static constexpr int R1 = SL::R1, R2 = SL::R2, R2P = SL::R2P, NT = SL::NT, LR = SL::LR;
   static constexpr int LPA = SL::LPA, LPX = SL::LPX;
   static constexpr int LJ = SL::LJ, LK = SL::LK;
@@ -1027,12 +1032,12 @@ template <typename R, int N, bool Q> struct SlabThread {
 };
 
 template <typename R, int N, bool Q>
-__global__ __launch_bounds__((Slab<R, N>::NT)) void k_slab_vmul(PwBatch B, cx_t<R>* __restrict__ S, int nz, int bpw,
+__global__ __launch_bounds__((Slab<R, N, true>::NT)) void k_slab_vmul(PwBatch B, cx_t<R>* __restrict__ S, int nz, int bpw,
                                                               const cx_t<R>* __restrict__ tw,
                                                               const R* __restrict__ vt) {
   using C = cx_t<R>;
-  using ST = SlabThread<R, N, Q>;
-  constexpr int R1 = ST::R1, R2 = ST::R2, LR = ST::LR, NR = Slab<R, N>::NR, LJ = ST::LJ, LK = ST::LK;
+  using ST = SlabThread<R, N, true, Q>;
+  constexpr int R1 = ST::R1, R2 = ST::R2, LR = ST::LR, NR = Slab<R, N, true>::NR, LJ = ST::LJ, LK = ST::LK;
   constexpr int LPA = ST::LPA, LPX = ST::LPX;
   extern __shared__ __align__(16) unsigned char smem[];
   const PwMaps m = B.mt[B.k0 + blockIdx.z];
@@ -1160,8 +1165,17 @@ template <typename R, int N> struct Lines {
   }
 };
 
-// lengths whose H|psi> pass is the barrier kernel (both measured above)
+// Lengths whose H|psi> pass is always the barrier kernel (both measured above).
+// At 72 it also takes bases that reach beyond the outer quarters, whose planes
+// need two groups or a fifth wavefront (128 bands of complex64 with 49 planes
+// 226 us against 224, 64 with 61 planes 130 against 186; 64 of complex128 with
+// 45 planes 178 against 213).
 template <typename R, int N> constexpr bool kSlabBarrier = N == 32 || (N == 108 && sizeof(R) == 4);
+template <typename R, int N> static bool slab_barrier(int nax_cap, bool quarter) {
+  if (kSlabBarrier<R, N>) return true;
+  if (Lines<R, N>::waves(nax_cap) == 0) return true;
+  return N == 72 && !quarter && Slab<R, N, true>::lds(nax_cap) <= 160 * 1024;
+}
 
 // LDS accesses of one wavefront on lines of its own stay in program order
 __device__ __forceinline__ void line_fence() {
@@ -1451,7 +1465,7 @@ __global__ __launch_bounds__((Slab<R, N>::NT)) void k_slab_density(PwBatch B, co
                                                                  const double* __restrict__ occ, int occ_ks,
                                                                  double* __restrict__ part) {
   using C = cx_t<R>;
-  using ST = SlabThread<R, N, Q>;
+  using ST = SlabThread<R, N, false, Q>;
   constexpr int R1 = ST::R1, R2 = ST::R2, LR = ST::LR, NR = Slab<R, N>::NR;
   extern __shared__ __align__(16) unsigned char smem[];
   const PwMaps m = B.mt[B.k0 + blockIdx.z];
@@ -1546,19 +1560,22 @@ template <typename R> bool slab_supported(int nx, int ny, int nz, int nax_cap, i
 template <typename R, int N>
 static void slab_vmul_n(const PwBatch& B, cx_t<R>* S, const Axis<R>* ax, int nz, const R* vt, int bpw, hipStream_t s) {
   const dim3 grid((unsigned)nz, (unsigned)ceil_div(B.nbb, bpw), B.nkc);
-  if constexpr (kSlabBarrier<R, N>) {
-    using SL = Slab<R, N>;
-    const size_t lds = SL::lds(B.nax_cap);
-    check_lds_pw(lds, N);
-    auto kern = B.quarter ? k_slab_vmul<R, N, true> : k_slab_vmul<R, N, false>;
-    allow_lds_pw(kern, lds);
-    hipLaunchKernelGGL(kern, grid, dim3(SL::NT), lds, s, B, S, nz, bpw, ax[0].tw, vt);
-  } else {
-    using G = Lines<R, N>;
+  if (slab_barrier<R, N>(B.nax_cap, B.quarter)) {
+    if constexpr (kSlabBarrier<R, N> || N == 72) {  // (at 72 never with the quarters)
+      using SL = Slab<R, N, true>;
+      const size_t lds = SL::lds(B.nax_cap);
+      check_lds_pw(lds, N);
+      auto kern = B.quarter ? k_slab_vmul<R, N, N != 72> : k_slab_vmul<R, N, false>;
+      allow_lds_pw(kern, lds);
+      hipLaunchKernelGGL(kern, grid, dim3(SL::NT), lds, s, B, S, nz, bpw, ax[0].tw, vt);
+    } else {
+      throw ArgError("active planes do not fit the LDS");
+    }
+  } else if constexpr (!kSlabBarrier<R, N>) {
+    using G = Lines<R, N>;  // (complex64 at 72 only with the quarters)
     const int nw = G::waves(B.nax_cap);
-    DEREK_REQUIRE(nw > 0, "active planes do not fit the LDS");
     const size_t lds = G::lds(B.nax_cap, nw);
-    auto kern = B.quarter ? k_slab_lines<R, N, true> : k_slab_lines<R, N, false>;
+    auto kern = B.quarter ? k_slab_lines<R, N, true> : k_slab_lines<R, N, (N == 72 && sizeof(R) == 4)>;
     allow_lds_pw(kern, lds);
     hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, B, S, nz, bpw, ax[0].tw, vt);
   }
@@ -1583,7 +1600,8 @@ void slab_vmul(const PwBatch& B, cx_t<R>* S, const Axis<R>* ax, int nz, const R*
 // The density kernel of a batch: whole lines per wavefront where its planes and
 // lines fit, the barrier kernel for more planes, at 32 (one round of lines) and
 // for complex128 at 108 (its sums leave room for seven wavefronts only: 323 us
-// against 319 for 160 bands).
+// against 319 for 160 bands), and at 72 for bases beyond the outer quarters (128
+// bands of complex64 171 us against 178, 64 of complex128 145 against 148).
 template <typename R> struct DensityKernel {
   void (*kern)(PwBatch, const cx_t<R>*, int, int, const cx_t<R>*, const double*, int, double*);
   int nt;
@@ -1594,9 +1612,9 @@ template <typename R, int N> static DensityKernel<R> density_kernel(const PwBatc
   if constexpr (N > 32 && !(N == 108 && sizeof(R) == 8)) {
     using G = Lines<R, N>;
     constexpr int NW = N == 72 ? 4 : (N == 108 ? 8 : 12);
-    k = {B.quarter ? k_slab_lines_density<R, N, true, NW> : k_slab_lines_density<R, N, false, NW>, 64 * NW,
+    k = {B.quarter ? k_slab_lines_density<R, N, true, NW> : k_slab_lines_density<R, N, N == 72, NW>, 64 * NW,
          G::lds(B.nax_cap, NW)};
-    if (B.nax_cap > NW * G::LPW * G::NP || k.lds > 160 * 1024) k.kern = nullptr;
+    if (B.nax_cap > NW * G::LPW * G::NP || k.lds > 160 * 1024 || (N == 72 && !B.quarter)) k.kern = nullptr;
   }
   if (!k.kern)
     k = {B.quarter ? k_slab_density<R, N, true> : k_slab_density<R, N, false>, Slab<R, N>::NT,

@@ -97,3 +97,29 @@ def test_outer_quarters(dims, precision, quarter):
         assert_close(ctx.apply_h(0, psi), ref, tol, "H psi")
         assert_close(ctx.density(0, psi, occ), rref, tol, "density")
     ctx.close()
+
+
+@pytest.mark.parametrize("n", [72, 108, 144])
+@pytest.mark.parametrize("planes", [27, 28, 29, 45, 56, 57, 70, 76, 108])
+@pytest.mark.parametrize("precision", [lib.DEREK_FP64, lib.DEREK_MIXED])
+def test_fused_pass_plane_counts(n, planes, precision):
+    """Active x planes at the edges of the fused pass: groups of planes per
+    wavefront, wavefronts that the LDS holds, and the switches to the barrier
+    kernel and to the separate passes."""
+    planes, nz = min(planes, n), 6
+    rng = np.random.default_rng(n + planes)
+    xs = rng.permutation(n)[:planes]
+    idx = np.concatenate([(x * n + y) * nz + np.arange(0, nz, 1 + y % 3) for x in xs for y in rng.permutation(n)[:3]])
+    idx = rng.permutation(np.unique(idx)).astype(np.int32)
+    kin = rng.uniform(0.0, 3.0, len(idx))
+    v = rng.normal(size=n * n * nz)
+    tol = 1e-12 if precision == lib.DEREK_FP64 else 5e-5
+    print("planes", n, planes, precision, flush=True)
+    ctx = lib.Context([n, n, nz], 1, 2, 13.0, len(idx), precision)
+    ctx.set_basis(0, idx, kin, 1.1)
+    ctx.set_vloc(v)
+    psi = rng.normal(size=(2, len(idx))) + 1j * rng.normal(size=(2, len(idx)))
+    occ = np.array([2.0, 0.7])
+    assert_close(ctx.apply_h(0, psi), oks.apply_h(psi, idx, kin, v, (n, n, nz)), tol, "H psi")
+    assert_close(ctx.density(0, psi, occ), oks.density([psi], [occ], [1.1], [idx], (n, n, nz), 13.0), tol, "density")
+    ctx.close()
