@@ -609,7 +609,7 @@ int32_t derek_hip_init(derek_ctx** out, const derek_dims* d) {
     c->max_npw = d->max_npw;
     DEREK_HIP(hipGetDevice(&c->device));
     DEREK_HIP(hipStreamCreateWithFlags(&c->s, hipStreamNonBlocking));
-    noalloc_setup(c->device);
+    if (c->prec == DEREK_FP64) c->noalloc.init();
     for (int a = 0; a < 3; ++a) {
       c->tw64[a] = reinterpret_cast<double2*>(make_twiddles<double>(c->dims[a]));
       c->tw32[a] = reinterpret_cast<float2*>(make_twiddles<float>(c->dims[a]));
@@ -860,12 +860,17 @@ int32_t derek_hip_overlap(derek_ctx* c, int64_t npw, int32_t m, int32_t n, const
 
 int32_t derek_hip_overlap_noalloc(derek_ctx* c, int64_t npw, int32_t m, int32_t n, const double* X, const double* Y,
                                   double* S) {
+  return derek_hip_overlap_noalloc_on(c, nullptr, npw, m, n, X, Y, S);
+}
+
+int32_t derek_hip_overlap_noalloc_on(derek_ctx* c, void* stream, int64_t npw, int32_t m, int32_t n, const double* X,
+                                     const double* Y, double* S) {
   return guard([&] {
     DEREK_REQUIRE(c && X && Y && S, "null argument");
     DEREK_REQUIRE(npw >= 1 && m >= 1 && n >= 1, "empty overlap");
     DEREK_REQUIRE(c->prec == DEREK_FP64, "overlap_noalloc multiplies complex128 operands: it needs a DEREK_FP64 context");
-    overlap_noalloc(c, npw, m, n, reinterpret_cast<const double2*>(X), reinterpret_cast<const double2*>(Y),
-                    reinterpret_cast<double2*>(S));
+    overlap_noalloc(c, static_cast<hipStream_t>(stream), npw, m, n, reinterpret_cast<const double2*>(X),
+                    reinterpret_cast<const double2*>(Y), reinterpret_cast<double2*>(S));
   });
 }
 
@@ -1178,12 +1183,14 @@ int32_t derek_hip_sync(derek_ctx* c) {
   return guard([&] {
     DEREK_REQUIRE(c, "null context");
     c->sync();
+    c->noalloc.sync();
   });
 }
 
 int32_t derek_hip_stream(derek_ctx* c, void** stream) {
   return guard([&] {
     DEREK_REQUIRE(c && stream, "null argument");
+    c->noalloc.share(c->s);
     *stream = (void*)c->s;
   });
 }

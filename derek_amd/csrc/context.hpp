@@ -58,9 +58,22 @@ inline void dfree(void* p) {
 
 inline int64_t round_up(int64_t a, int64_t b) { return ceil_div(a, b) * b; }
 
-// Allocation-free overlap (noalloc.hip): a file-scope device array of this
-// many double2 (32 MiB per GPU) holds its split-K partial sums.
+// What the allocation-free overlap (noalloc.hip) keeps: kNoAllocScratchElems
+// double2 (32 MiB) for its split-K partial sums and the events that order
+// streams.  Made at init by DEREK_FP64 contexts only.
 constexpr int64_t kNoAllocScratchElems = (int64_t)1 << 21;
+struct NoAlloc {
+  double2* work = nullptr;
+  hipEvent_t ready = nullptr, done = nullptr;
+  hipStream_t last = nullptr;  // the stream of the latest overlap; `done` follows it there, unless null
+  bool pending = false;        // that overlap may still run
+  bool shared = false;         // the caller has the context's stream
+  void init();
+  void order(hipStream_t to);
+  void share(hipStream_t s);  // the context's stream s is handed out
+  void sync();
+  ~NoAlloc();
+};
 
 // Per-kernel-class timers: HIP events recorded on the context's stream around
 // each launch while enabled, resolved lazily; algorithmic bytes and flops of
@@ -175,6 +188,7 @@ struct derek_ctx {
   template <typename R> derek::cx_t<R>* planes(int items);
   double2* cgrid = nullptr;
   derek::DevBuf tA, tB, tC, tD, ovwork, partial;
+  derek::NoAlloc noalloc;
   derek::Profiler prof;
   std::unique_ptr<derek::ScfEngine, derek::EngineDeleter> scf;
   template <typename F> void timed(int cls, double bytes, double flops, F&& launch) {
@@ -222,10 +236,9 @@ struct derek_ctx {
 };
 
 namespace derek {
-// resolves the allocation-free overlap's scratch address on device `dev`
-// (current); once per device
-void noalloc_setup(int dev);
-// S = X^H Y (device pointers, complex128) on the context's stream, partial
-// sums in the scratch array; no allocation, no synchronisation
-void overlap_noalloc(derek_ctx* c, int64_t npw, int m, int n, const double2* X, const double2* Y, double2* S);
+// S = X^H Y (device pointers, complex128) in the order of the stream `caller`,
+// partial sums in the context's scratch; no allocation, no synchronisation of
+// the host
+void overlap_noalloc(derek_ctx* c, hipStream_t caller, int64_t npw, int m, int n, const double2* X, const double2* Y,
+                     double2* S);
 }  // namespace derek

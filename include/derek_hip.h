@@ -237,15 +237,25 @@ int32_t derek_hip_overlap(derek_ctx* ctx, int64_t npw, int32_t m, int32_t n, con
  * (complex128; X == Y with m == n takes the Hermitian path), for callers
  * that cannot allocate: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  No counterpart in the reference.  It
- * allocates nothing: the split-K partial sums go to a file-scope device
- * array of 2^21 complex128 values (32 MiB per GPU, held until the process
- * ends), whose address derek_hip_init resolves once per device; m * n above
- * 2^21 is refused with DEREK_ERR_ARG, and the row chunks are capped so their
- * partials fit.  Needs a DEREK_FP64 context.  Asynchronous on the context's
- * stream (derek_hip_stream; derek_hip_sync waits).  Every call on one GPU
- * shares the array: calls that overlap in time on one GPU race. */
+ * allocates nothing: the split-K partial sums go to a buffer of 2^21
+ * complex128 values (32 MiB) that the context holds from derek_hip_init on;
+ * m * n above 2^21 is refused with DEREK_ERR_ARG, and the row chunks are
+ * capped so their partials fit.  Needs a DEREK_FP64 context.
+ *
+ * Asynchronous (derek_hip_sync waits), in the order of the device's default
+ * (null) stream: what that holds at the call (writes of X and Y) comes before,
+ * what it is given later (reads of S, reuse of the memory) after.  Once the
+ * caller has asked for the context's stream (derek_hip_stream), the overlap is
+ * in order on that one as well; while that one is being captured, on it
+ * alone. */
 int32_t derek_hip_overlap_noalloc(derek_ctx* ctx, int64_t npw, int32_t m, int32_t n, const double* X,
                                   const double* Y, double* S);
+/* The same in the order of another stream (hipStream_t; null: the default
+ * stream, as above).  A stream that is being captured takes the overlap into
+ * its graph.  The replays of a captured overlap use the context's buffer: order
+ * them with the context's other overlaps. */
+int32_t derek_hip_overlap_noalloc_on(derek_ctx* ctx, void* stream, int64_t npw, int32_t m, int32_t n, const double* X,
+                                     const double* Y, double* S);
 /* Z = X U; X: npw x m, U: m x n, Z: npw x n (complex). */
 int32_t derek_hip_rotate(derek_ctx* ctx, int64_t npw, int32_t m, int32_t n, const double* X, const double* U,
                          double* Z);
@@ -364,7 +374,8 @@ int32_t derek_hip_set_launch(derek_ctx* ctx, int32_t bands_per_wg, int32_t items
  * 24).  FP64 data is unaffected.
  * No counterpart in the reference (precision control of the GPU GEMMs). */
 int32_t derek_hip_set_gemm(derek_ctx* ctx, int32_t bf16_terms);
-/* Block until all work on the context's stream is done. */
+/* Block until all work on the context's stream, and the allocation-free
+ * overlaps, are done. */
 int32_t derek_hip_sync(derek_ctx* ctx);
 /* Host-visible stream handle (hipStream_t) for event timing. */
 int32_t derek_hip_stream(derek_ctx* ctx, void** stream);
