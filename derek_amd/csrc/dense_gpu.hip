@@ -326,16 +326,17 @@ __device__ __forceinline__ double read_lane(double x, int l) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Householder scalars of column k from xn2 = sum_{i>k} |A(i,k)|^2 and
+// Householder scalars of column k from tail2 = sum_{i>k+1} |A(i,k)|^2 and
 // x0 = A(k+1,k) (both wave-uniform): alpha = -(x0/|x0|) ||x|| (the new
 // sub-diagonal), v0 = x0 - alpha and iv = 1/||v|| with
-// ||v||^2 = 2 ||x|| (||x|| + |x0|); skip when x is already reduced.  When rec
-// is set the caller's lane records alpha and the skip flag.
-__device__ __forceinline__ void tri_scalars(bool rec, int k, double xn2, double2 x0, HeevWork& W, int& skip,
+// ||v||^2 = 2 ||x|| (||x|| + |x0|); skip when x is already reduced, which the
+// tail alone decides: in ||x||^2 - |x0|^2 entries below 1e-8 |x0| are lost.
+// When rec is set the caller's lane records alpha and the skip flag.
+__device__ __forceinline__ void tri_scalars(bool rec, int k, double tail2, double2 x0, HeevWork& W, int& skip,
                                             double& iv, double2& v0) {
   // without branches: the two square roots overlap
-  const double a2 = x0.x * x0.x + x0.y * x0.y;
-  skip = (xn2 == 0.0 || xn2 - a2 <= 1e-300) ? 1 : 0;
+  const double a2 = x0.x * x0.x + x0.y * x0.y, xn2 = a2 + tail2;
+  skip = tail2 <= 1e-300 ? 1 : 0;
   const double rx = rsqrt_nr(xn2), ra = rsqrt_nr(a2), xn = xn2 * rx;
   const bool nz = a2 > 0.0;
   const double ax0 = nz ? a2 * ra : 0.0;
@@ -350,12 +351,12 @@ __device__ __forceinline__ void tri_scalars(bool rec, int k, double xn2, double2
   }
 }
 
-// Reflector of column k from sum |A(i,k)|^2 (i > k) and x0 = A(k+1,k), both
+// Reflector of column k from sum |A(i,k)|^2 (i > k+1) and x0 = A(k+1,k), both
 // wave-uniform, for the multi-workgroup steps: every lane derives the
 // scalars, lane 0 records them (with the scalars for the next launch).
-__device__ __forceinline__ void wide_reflector_scalars(int lane, int k, double xn2, double2 x0, HeevWork& W,
+__device__ __forceinline__ void wide_reflector_scalars(int lane, int k, double tail2, double2 x0, HeevWork& W,
                                                        int& skip, double& iv, double2& v0) {
-  tri_scalars(lane == 0, k, xn2, x0, W, skip, iv, v0);
+  tri_scalars(lane == 0, k, tail2, x0, W, skip, iv, v0);
   if (lane == 0) {
     double* sc = W.scal + 4 * (k & 1);
     sc[0] = skip;
@@ -448,9 +449,11 @@ __global__ __launch_bounds__(TDT) void k_tridiag(double2* __restrict__ Aall, int
   // reflector of column c from its values x (rows lane and lane + 64, zero
   // outside c+1..nb-1): into s_vu and, for the back-transformation, column c
   auto reflector = [&](int c, const double2* x) {
-    const double part = wave_sum(x[0].x * x[0].x + x[0].y * x[0].y + x[1].x * x[1].x + x[1].y * x[1].y);
     const int l = (c + 1) & 63;
-    const double2 y = (c + 1) >> 6 ? x[1] : x[0];
+    const bool hi = (c + 1) >> 6;  // row c + 1 is x[hi] of lane l
+    const double q0 = x[0].x * x[0].x + x[0].y * x[0].y, q1 = x[1].x * x[1].x + x[1].y * x[1].y;
+    const double part = wave_sum(lane == l ? (hi ? q0 : q1) : q0 + q1);
+    const double2 y = hi ? x[1] : x[0];
     const double2 x0 = make_double2(read_lane(y.x, l), read_lane(y.y, l));
     int skip;
     double iv;
@@ -619,7 +622,7 @@ __device__ __forceinline__ void wide_reflector(const double2* __restrict__ A, in
                                                int lane) {
   const double2* col = A + (int64_t)k * lda;
   double part = 0.0;
-  for (int i = k + 1 + lane; i < n; i += 64) part += col[i].x * col[i].x + col[i].y * col[i].y;
+  for (int i = k + 2 + lane; i < n; i += 64) part += col[i].x * col[i].x + col[i].y * col[i].y;
   part = wave_sum(part);
   const double2 x0 = col[k + 1];
   int skip;
@@ -738,7 +741,7 @@ __global__ __launch_bounds__(WT) void k_wide_step(double2* __restrict__ Aall, in
       const double2 ci = i == i1 ? c1pre : c1[i];
       const double2 c = skip ? ci : upd(ci, v[i], wof(i), v1, w1);
       vn[i] = c;
-      part += c.x * c.x + c.y * c.y;
+      if (i > k + 2) part += c.x * c.x + c.y * c.y;
     }
     part = wave_sum(part);
     if (lane == 0) red[wid] = part;
@@ -865,7 +868,7 @@ __global__ __launch_bounds__(WT) void k_wide_regs(double2* __restrict__ Aall, in
         if (own && !skip) col[k1] = c[0];  // the diagonal entry
         c[0] = zero;
       }
-      part += c[q].x * c[q].x + c[q].y * c[q].y;
+      if (q > 0 || lane > 1) part += c[q].x * c[q].x + c[q].y * c[q].y;
     }
     part = wave_sum(part);
     const double2 x0 = make_double2(read_lane(c[0].x, 1), read_lane(c[0].y, 1));
