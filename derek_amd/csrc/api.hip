@@ -1137,9 +1137,7 @@ int32_t derek_hip_get_tuning(derek_ctx* c, int32_t out[8]) {
     out[4] = c->fused;
     out[5] = c->zsl ? c->zsl : (c->prec == DEREK_FP64 ? 16 : 32);
     out[6] = c->ov_rounds;
-    // the C tile edge in use; left to the size, the one of the engine's 2nb x 2nb overlaps
     out[7] = c->ov_tile ? c->ov_tile : 64;
-    if (!c->ov_tile && c->gemm_bf16 == 2 && c->scf && overlap_wide(2 * c->nb, 2 * c->nb, c->max_npw, out[2])) out[7] = 128;
   });
 }
 
@@ -1162,10 +1160,11 @@ int32_t derek_hip_set_tiles(derek_ctx* c, int32_t z_sticks, int32_t gemm_rounds,
     DEREK_REQUIRE(c, "null context");
     DEREK_REQUIRE(z_sticks == 0 || z_sticks == 16 || z_sticks == 32, "sticks per z-pass workgroup must be 0, 16 or 32");
     DEREK_REQUIRE(gemm_rounds == 1 || gemm_rounds == 2 || gemm_rounds == 4, "GEMM rounds must be 1, 2 or 4");
-    DEREK_REQUIRE(gemm_tile == 64 || gemm_tile == 128, "GEMM tile must be 64 or 128");
+    DEREK_REQUIRE(gemm_tile == 0 || gemm_tile == 64 || gemm_tile == 128, "GEMM tile must be 0, 64 or 128");
     c->zsl = z_sticks;
     c->ov_rounds = gemm_rounds;
-    c->ov_tile = gemm_tile;
+    c->ov_tile = gemm_tile == 128 ? 128 : 0;
+    c->ov_tuned = 0;
     ++c->graph_epoch;
   });
 }
@@ -1175,6 +1174,8 @@ int32_t derek_hip_set_gemm(derek_ctx* c, int32_t bf16_terms) {
     DEREK_REQUIRE(c, "null context");
     DEREK_REQUIRE(bf16_terms >= 0 && bf16_terms <= 3, "bf16 terms must be 0 (FP32 matrix cores) or 1..3");
     c->gemm_bf16 = bf16_terms;
+    // an edge timed with other terms says nothing about these
+    if (c->ov_tuned && c->ov_tuned != bf16_terms) c->ov_tile = c->ov_tuned = 0;
     ++c->graph_epoch;
   });
 }

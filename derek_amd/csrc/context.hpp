@@ -175,8 +175,11 @@ struct derek_ctx {
   // row chunks fill (1, 2 or 4); both autotuned by the SCF engine when asked
   int zsl = 0;
   int ov_rounds = 2;
-  // C tile edge of the BF16 overlaps (64 or 128; 0: by size), autotuned as well
+  // C tile edge of the BF16 overlaps: 128, or 0 for 64 and the kernel on
+  // interleaved values where the size asks for it (overlap_wide).  Autotuned as
+  // well, for ov_tuned terms; 0: not by the autotuner
   int ov_tile = 0;
+  int ov_tuned = 0;
   // Moves whenever a work buffer below is freed or reallocated, or a launch
   // setting changes (set_launch, set_gemm): a graph captured at another
   // epoch may hold freed addresses or stale shapes and is not replayed.

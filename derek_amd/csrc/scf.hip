@@ -512,15 +512,19 @@ template <typename R> void autotune(derek_ctx* c) {
       return tb;
     };
     float bestg = time_ov();
-    // tile edge first (BF16 overlaps only), then the rounds at that edge; an
-    // edge left to the size stays so for two terms, whose large overlaps have
-    // a kernel of their own
-    if (bf16_terms<R>(c) > 0 && (c->ov_tile || bf16_terms<R>(c) != 2)) {
+    // tile edge first (BF16 overlaps only), then the rounds at that edge; the
+    // large two-term overlaps keep the kernel of their own
+    const int terms = bf16_terms<R>(c);
+    if (terms > 0 && (c->ov_tile || terms != 2 || !overlap_wide(E.m2, E.m2, c->max_npw, nkg))) {
       const int t0 = c->ov_tile;
-      c->ov_tile = t0 == 128 ? 64 : 128;
+      c->ov_tile = t0 ? 0 : 128;
       const float t = time_ov();
-      if (t < kGain * bestg) bestg = t;
-      else c->ov_tile = t0;
+      if (t < kGain * bestg) {
+        bestg = t;
+        c->ov_tuned = terms;
+      } else {
+        c->ov_tile = t0;
+      }
     }
     const int r0 = c->ov_rounds;
     for (int q : kOvRounds) {

@@ -509,17 +509,18 @@ class Context:
         check(self.lib.derek_hip_scf_init(self.h, C.byref(p)))
 
     def tuning(self):
-        """{bands_per_wg, items_per_launch, kbatch, graph, fused, fused_density, z_sticks, gemm_rounds}"""
+        """{bands_per_wg, items_per_launch, kbatch, graph, fused, fused_density, z_sticks, gemm_rounds, gemm_tile}"""
         out = (C.c_int32 * 8)()
         check(self.lib.derek_hip_get_tuning(self.h, out))
         return {"bands_per_wg": out[0], "items_per_launch": out[1], "kbatch": out[2], "graph": bool(out[3]),
                 "fused": bool(out[4] & 1), "fused_density": bool(out[4] & 2), "z_sticks": out[5],
                 "gemm_rounds": out[6], "gemm_tile": out[7]}
 
-    def set_tiles(self, z_sticks=0, gemm_rounds=2, gemm_tile=64):
+    def set_tiles(self, z_sticks=0, gemm_rounds=2, gemm_tile=0):
         """Sticks per z-pass workgroup (16, 32; 0: the precision's default),
         the rounds of resident workgroups the overlaps' row chunks fill (1, 2,
-        4) and the C tile edge of the BF16 overlaps (64, 128)."""
+        4) and the C tile edge of the BF16 overlaps (128; 0 or 64: 64, and the
+        kernel on interleaved values for the large two-term ones)."""
         check(self.lib.derek_hip_set_tiles(self.h, int(z_sticks), int(gemm_rounds), int(gemm_tile)))
 
     def set_launch(self, bands_per_wg=2, items_per_launch=256, fused=True, fused_density=None):
