@@ -1016,7 +1016,7 @@ void overlap(const cx_t<R>* X, int64_t ldx, int64_t sx, const cx_t<R>* Y, int64_
                                         : ov_slots<R>();
   DEREK_REQUIRE(rounds == 1 || rounds == 2 || rounds == 4, "overlap: rounds must be 1, 2 or 4");
   OvGeom g = ov_geom(m, n, npw, hermitian, batch, slots, bf16_terms ? BF_KS : OV_KS, rounds, tt);
-  ov_limit_chunks(g, max_chunks, bf16_terms ? BF_KS : OV_KS);
+  ov_limit_chunks(g, max_chunks, bf16_terms ? BF_KS : OV_KS, batch, slots);
   DEREK_REQUIRE((int64_t)batch * g.nchunk * m * n <= work_cap, "overlap: partial-sum buffer too small");
   const int64_t items = (int64_t)g.ntiles * g.nchunk * batch;
   DEREK_REQUIRE(items < (int64_t)1 << 31, "overlap: too many workgroups");

@@ -62,14 +62,25 @@ inline OvGeom ov_geom(int m, int n, int64_t npw, bool herm, int batch, int slots
   return g;
 }
 
-// At most max_chunks row chunks (a fixed partial-sum buffer): each chunk
-// takes more rows, still a whole number of `ks`-row slabs.
-inline void ov_limit_chunks(OvGeom& g, int64_t max_chunks, int ks) {
+// At most max_chunks row chunks (a fixed partial-sum buffer): each chunk takes
+// more rows, still a whole number of `ks`-row slabs.  Of the counts allowed, the
+// one with the fewest rows in turn over its rounds of resident workgroups: with
+// so few rounds a nearly empty last one counts as a whole (161214 x 600 x 300 in
+// complex128: 11 chunks, 550 workgroups in 512 slots, 6.9 ms; 10 chunks 3.7 ms).
+inline void ov_limit_chunks(OvGeom& g, int64_t max_chunks, int ks, int64_t batch, int slots) {
   if (max_chunks < 1 || g.nchunk <= max_chunks) return;
-  int64_t kch = ov_ceil_div(std::max<int64_t>(g.npw, 1), max_chunks);
-  kch = std::max<int64_t>(ks, ov_ceil_div(kch, ks) * ks);
-  g.kch = kch;
-  g.nchunk = (int)std::max<int64_t>(1, ov_ceil_div(g.npw, kch));
+  int64_t least = INT64_MAX;
+  // (half the chunks take at least as long in any number of rounds)
+  for (int64_t c = max_chunks; 2 * c > max_chunks; --c) {
+    int64_t kch = ov_ceil_div(std::max<int64_t>(g.npw, 1), c);
+    kch = std::max<int64_t>(ks, ov_ceil_div(kch, ks) * ks);
+    const int64_t nchunk = std::max<int64_t>(1, ov_ceil_div(g.npw, kch));
+    const int64_t rows = ov_ceil_div(g.ntiles * batch * nchunk, slots) * kch;
+    if (rows >= least) continue;
+    least = rows;
+    g.kch = kch;
+    g.nchunk = (int)nchunk;
+  }
 }
 
 // double2 elements of the partial sums of an m x n overlap of `batch`
