@@ -24,15 +24,20 @@ inline int64_t ov_ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // Row chunks per tile: at least `rounds` full rounds of workgroups over the
 // chip's resident slots (`slots` = resident workgroups per CU x CUs), then,
 // among the next few counts, the one that leaves the smallest idle tail in
-// the last round; every chunk keeps a whole number of `ks`-row slabs and at
-// least 4 m n / (m + n) rows (64 to 256), so that writing and reading the m x n
-// partial costs at most half of what the chunk's rows of X and Y do.  (With
-// 256 rows for every size the 32^3 system's 20-column overlaps of 1503 rows
-// ran in five workgroups of 19 serial slabs, 42 us each.)  The SCF autotuner picks `rounds` among kOvRounds.
+// the last round; every chunk keeps a whole number of `ks`-row slabs and 256
+// rows.  Shorter chunks, of at least 4 m n / (m + n) rows (64 to 256) so that
+// writing and reading the m x n partial costs at most half of what the chunk's
+// rows of X and Y do, only up to 128 of them and a workgroup per CU: beyond that
+// the reduction, a serial chain over the chunks, costs more than the products
+// gain.  (256 rows for every size: the 32^3 system's 20-column overlaps of 1503
+// rows ran in five workgroups of 19 serial slabs, 42 us each.  64 rows for every
+// size: 140000 rows of 16 columns in complex64 89 us, 55 with 256.)  The SCF
+// autotuner picks `rounds` among kOvRounds.
 constexpr int kOvRounds[3] = {1, 2, 4};
+constexpr int kOvCus = 256;  // MI355X
 inline OvGeom ov_geom(int m, int n, int64_t npw, bool herm, int batch, int slots, int ks = OV_KS, int rounds = 2,
                       int tile = OV_T) {
-  OvGeom g{};
+  OvGeom g;
   g.m = m;
   g.n = n;
   g.npw = npw;
@@ -43,7 +48,8 @@ inline OvGeom ov_geom(int m, int n, int64_t npw, bool herm, int batch, int slots
   g.ntiles = herm ? g.tm * (g.tm + 1) / 2 : g.tm * g.tn;
   const int64_t units = (int64_t)g.ntiles * std::max(1, batch);
   const int64_t rows = std::min<int64_t>(256, std::max<int64_t>(64, 4 * (int64_t)m * n / (m + n)));
-  const int64_t cmax = std::max<int64_t>(1, npw / rows);
+  const int64_t few = std::min<int64_t>({npw / rows, 128, kOvCus / units});
+  const int64_t cmax = std::max<int64_t>({1, npw / 256, few});
   const int64_t c0 = std::min(cmax, std::max<int64_t>(1, ov_ceil_div((int64_t)rounds * slots, units)));
   int64_t best = c0;
   double best_eff = -1.0;

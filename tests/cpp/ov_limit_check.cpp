@@ -20,6 +20,7 @@ int main() {
               for (int ks : {OV_KS, BF_KS})
                 for (int64_t cap : {0, 1, 2, 3, 5, 11, 23, 81, 1000, 1 << 21}) {
                   if (herm && m != n) continue;
+                  const int64_t most = std::max<int64_t>({1, npw / 256, std::min<int64_t>(npw / 64, 128)});
                   OvGeom g = ov_geom(m, n, npw, herm, batch, slots, ks);
                   const OvGeom free = g;
                   ov_limit_chunks(g, cap, ks, batch, slots);
@@ -29,7 +30,8 @@ int main() {
                   auto rows = [&](int64_t chunks, int64_t kch) {
                     return ov_ceil_div(g.ntiles * batch * chunks, slots) * kch;
                   };
-                  const bool ok = g.kch % ks == 0 && g.nchunk <= c && (int64_t)g.nchunk * g.kch >= npw &&
+                  const bool ok = free.nchunk <= most && (int64_t)free.nchunk * free.kch >= npw &&
+                                  (int64_t)(free.nchunk - 1) * free.kch < npw && g.kch % ks == 0 && g.nchunk <= c && (int64_t)g.nchunk * g.kch >= npw &&
                                   (int64_t)(g.nchunk - 1) * g.kch < npw &&
                                   (c == free.nchunk ? g.kch == free.kch && g.nchunk == free.nchunk
                                                     : rows(g.nchunk, g.kch) <= rows(ov_ceil_div(npw, k), k));
