@@ -184,20 +184,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 __host__ __device__ constexpr int ov_row_groups(int nblk) { return nblk <= 4 ? 4 : (nblk <= 2 * kOvBlocks ? 2 : 1); }
 
 // Whether the tiles of an m x n overlap take the quarter layout: matrix-core
-// steps per slab of the busiest wavefront, summed over the tiles, against the
-// dealt layout's, whose single-use operands cost 9 % per step on full tiles
-// (161214 x 600 x 300: 4.00 against 3.68 ms).
-inline bool ov_quarter(int m, int n, bool herm) {
+// steps per slab of the busiest wavefront against the dealt layout's, whose
+// operands are single-use and cost more LDS reads per step.  They are compared
+// summed over the tiles, or, while every workgroup has a CU to itself, by the
+// tile that takes longest.  The dealt layout wins from a quarter fewer steps on,
+// a third fewer where none of it comes from a diagonal.  Its time over the quarter
+// layout's, FP64 / FP32, by the ratio of steps: 1: 1.13 / 1.20 (1503 x 160
+// Hermitian, by the longest tile); 1.23: 1.09 / 1.05 (62669 x 200 x 100); 1.33:
+// 1.06 / 0.92 (62669 x 128 Hermitian); 1.36: 0.91 / 0.96 (62669 x 200 Hermitian);
+// 1.44: 1.09 / 1.04 (40000 x 160 x 80); 1.6: 0.94 / 1.04 (40000 x 80 x 40); 1.75:
+// 0.84 / 0.93 (62669 x 160 Hermitian); 5.3: 0.68 / 0.78 (62669 x 20 Hermitian).
+inline bool ov_quarter(int m, int n, bool herm, int64_t workgroups) {
   const int tm = (int)ceil_div(m, OV_T), tn = (int)ceil_div(n, OV_T);
+  const bool alone = workgroups <= kOvCus;
   int64_t quarter = 0, dealt = 0;
+  auto add = [alone](int64_t& t, int64_t x) { t = alone ? std::max(t, x) : t + x; };
   for (int ti = 0; ti < tm; ++ti)
     for (int tj = herm ? ti : 0; tj < tn; ++tj) {
       const int na = std::min(4, (int)ceil_div(m - ti * OV_T, 16)), nb = std::min(4, (int)ceil_div(n - tj * OV_T, 16));
       const int nblk = herm && ti == tj ? na * (na + 1) / 2 : na * nb, ks = ov_row_groups(nblk);
-      quarter += std::min(2, na) * std::min(2, nb) * 4;
-      dealt += ceil_div(nblk, 4 / ks) * (4 / ks);
+      add(quarter, std::min(2, na) * std::min(2, nb) * 4);
+      add(dealt, ceil_div(nblk, 4 / ks) * (4 / ks));
     }
-  return 8 * quarter <= 9 * dealt;
+  return herm ? 3 * quarter <= 4 * dealt : 2 * quarter <= 3 * dealt;
 }
 
 // The same overlap with the 16 x 16 blocks that C needs (inside C; on a
@@ -1036,7 +1045,7 @@ void overlap(const cx_t<R>* X, int64_t ldx, int64_t sx, const cx_t<R>* Y, int64_
     else if (bf16_terms == 2)
       hipLaunchKernelGGL((k_overlap_bf16<2, 128>), grid, b128, 0, s, X, ldx, sx, Y, ldy, sy, npwk, g, work);
   }
-  if (bf16_terms == 0 && ov_quarter(m, n, hermitian))
+  if (bf16_terms == 0 && ov_quarter(m, n, hermitian, items))
     hipLaunchKernelGGL(k_overlap<R>, grid, dim3(256), 0, s, X, ldx, sx, Y, ldy, sy, npwk, g, work);
   else if (bf16_terms == 0)
     hipLaunchKernelGGL(k_overlap_dealt<R>, grid, dim3(256), 0, s, X, ldx, sx, Y, ldy, sy, npwk, g, work);
