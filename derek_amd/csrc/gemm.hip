@@ -1290,10 +1290,13 @@ void rotate2(const cx_t<R>* X, const cx_t<R>* X2, int64_t ldx, int64_t sx, const
   if constexpr (std::is_same<R, float>::value) {
     // two terms: the 128-row workgroups once there is one per CU (600 -> 300
     // columns of 8 x 161214 rows 10.2 -> 5.3 ms, 48 -> 24 of 64 x 17529 0.248
-    // -> 0.183 ms; with 125 workgroups, 80 -> 40 of 4 x 4000 rows, 13 against
-    // 18 us), a buffer for the split U and 32-bit offsets
+    // -> 0.183 ms, 48 -> 24 of 40000 18.2 -> 17.6 us; with 125 workgroups, 80 ->
+    // 40 of 4 x 4000 rows, 13 against 18 us), or four where the few columns of X
+    // hardly pay the split's launch (32 -> 16 of 40000 rows 12.9 against 14.4 us,
+    // of 62669 14.6 and 16.2, of 140000 25.8 and 25.9; 16 -> 8 of 140000 21.9 ->
+    // 18.2), a buffer for the split U and 32-bit offsets
     const int64_t wide = ceil_div(npw, RC_ROWS) * ceil_div(n, RC_COLS) * batch;
-    if (bf16_terms == 2 && wide * two >= 256 && work && rotate_work_slots(m, n, batch) <= work_slots &&
+    if (bf16_terms == 2 && wide * two >= (m > 32 ? 256 : 1024) && work && rotate_work_slots(m, n, batch) <= work_slots &&
         (int64_t)m * ldx * 8 < (int64_t)kOob) {
       u4* img = reinterpret_cast<u4*>(work);
       hipLaunchKernelGGL(k_rotate_split, dim3((unsigned)ceil_div(m, CX_KS), (unsigned)ceil_div(n, RC_COLS), batch),
