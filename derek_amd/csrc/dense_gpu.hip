@@ -1,7 +1,6 @@
-// FP64 dense subspace solvers on the GPU, one 1024-thread workgroup per
-// matrix (blockIdx.x selects the matrix of a batch).
+// FP64 dense subspace solvers on the GPU for batches of matrices.
 //
-// k_heev: lowest nev eigenpairs of a Hermitian n x n matrix.
+// heev_gpu: lowest nev eigenpairs of a Hermitian n x n matrix.
 //   1. Householder reduction to real tridiagonal form: while the trailing
 //      matrix exceeds 128 columns, one multi-workgroup launch per column on the
 //      matrix in global memory (L2 resident); then the last 128 columns in the
@@ -17,9 +16,9 @@
 //      whose vectors are computed by one thread in order and re-orthogonalised
 //      (modified Gram-Schmidt) against the earlier members.
 //   5. Back-transformation by the reflectors, one wavefront per vector.
-// k_chol_panel: inverse Cholesky factor of a unit-diagonal Hermitian overlap,
-//   skipping every column whose remaining pivot is below tol (dependent on
-//   earlier columns); many workgroups, one launch per panel of columns.
+// chol_inverse_gpu: inverse Cholesky factor of a unit-diagonal Hermitian
+//   overlap, skipping every column whose remaining pivot is below tol (dependent
+//   on earlier columns); many workgroups, one launch per panel of columns.
 #include <cfloat>
 #include <type_traits>
 
@@ -64,29 +63,7 @@ __device__ __forceinline__ double wave_sum(double x) {
   return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Sum over the workgroup; every thread gets the result.
-__device__ double block_sum_all(double x, double* red) {
-  x = wave_sum(x);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) red[wid] = x;
-  __syncthreads();
-  double t = 0.0;
-  for (int w = 0; w < DW; ++w) t += red[w];
-  return t;
-}
-
-__device__ double block_min_all(double x, double* red) {
-  for (int o = 32; o > 0; o >>= 1) x = fmin(x, __shfl_down(x, o, 64));
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) red[wid] = x;
-  __syncthreads();
-  double t = red[0];
-  for (int w = 1; w < DW; ++w) t = fmin(t, red[w]);
-  return t;
-}
-
+// Maximum over the workgroup; every thread gets the result.
 __device__ double block_max_all(double x, double* red) {
   for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_down(x, o, 64));
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;

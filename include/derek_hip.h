@@ -6,7 +6,8 @@
  * failure of the calling thread.  Arguments are plain pointers and sizes.
  * Host arrays are Fortran-compatible: column-major, contiguous, complex
  * values interleaved (re, im) as complex(C_DOUBLE_COMPLEX).  No device
- * pointer crosses the boundary: the context owns all GPU memory.
+ * pointer crosses the boundary (but for the allocation-free overlap): the
+ * context owns all GPU memory.
  *
  * Grids are flat with z fastest and x slowest, exactly the layout the
  * reference's fft_3d reshapes around FFTW (Source/fft.f90:258-273).
